@@ -131,23 +131,48 @@ __device__ __forceinline__ double exp_nonpos(double x) {
   return __builtin_ldexp(__builtin_fma(r8, s1, s0), (int)k);
 }
 
-// fround(Math.exp(x)) for x <= 0 (or NaN): V8's exp rounded to f32, the exps of the reference's
-// f32 softmax (src/reference/cpu.ts:253). exp_nonpos gives e^x within a few f64 ulps, and
-// V8's fdlibm exp is within one; both round to the same f32 unless e^x lies within their
-// combined error of a rounding boundary of f32 (the midpoint between two neighbours). So the
-// fast value is kept when its distance to that boundary exceeds 2^-44 of it -- thousands of
-// times either error bound -- and otherwise (about one argument in 2^20) fdlibm_exp decides.
+// The fast half of fround(Math.exp(x)) for x <= 0 (or NaN), the exps of the reference's f32
+// softmax (src/reference/cpu.ts:253): V8's exp rounded to f32. e^r by its Taylor series to
+// degree 11 (|r| <= ln2/2: truncation below 2^-46 of e^r; the roundings of the form add a few
+// 2^-53), scaled by 2^k. That value and V8's round to the same f32 unless e^x lies within their
+// combined error of a midpoint between two neighbouring f32 values, which the 29 bits below the
+// f32 significand show directly (their value at a midpoint is 2^28): `slow` is set when they lie
+// within 2^9 of it -- 2^-44 of the value at least, four times the error bound; one argument
+// in 2^19 -- and for arguments whose f32 result is subnormal (x < -87, but zero for certain
+// below -104, as e^-104 < 2^-150) and NaN. Where `slow` is set the returned value means nothing.
+__device__ __forceinline__ float exp_to_f32_fast(float x, bool &slow) {
+  const double xd = fmax((double)x, -128.0);  // NaN too: marked slow below
+  const double k = __builtin_rint(xd * 1.44269504088896338700e+00);
+  double r = __builtin_fma(-k, 6.93147180369123816490e-01, xd);
+  r = __builtin_fma(-k, 1.90821492927058770002e-10, r);
+  const double r2 = r * r, r4 = r2 * r2;
+  const double p01 = 1.0 + r;
+  const double p23 = __builtin_fma(r, 1.66666666666666666667e-01, 5.0e-01);
+  const double p45 = __builtin_fma(r, 8.33333333333333333333e-03, 4.16666666666666666667e-02);
+  const double p67 = __builtin_fma(r, 1.98412698412698412698e-04, 1.38888888888888888889e-03);
+  const double p89 = __builtin_fma(r, 2.75573192239858906526e-06, 2.48015873015873015873e-05);
+  const double pab = __builtin_fma(r, 2.50521083854417187751e-08, 2.75573192239858906526e-07);
+  const double q0 = __builtin_fma(r2, p23, p01);
+  const double q1 = __builtin_fma(r2, p67, p45);
+  const double q2 = __builtin_fma(r2, pab, p89);
+  const double e = __builtin_ldexp(__builtin_fma(r4, __builtin_fma(r4, q2, q1), q0), (int)k);
+  const uint32_t below = (uint32_t)__double_as_longlong(e) & 0x1fffffffu;
+  const bool near = below - (0x10000000u - 0x200u) <= 0x400u;
+  const bool zero = x < -104.0f;
+  slow = !zero && (near || !(x >= -87.0f));
+  return zero ? 0.0f : (float)e;
+}
+
+// What exp_to_f32_fast leaves to V8's method: an argument it marked slow.
+__device__ __forceinline__ float exp_to_f32_slow(float x) {
+  return x != x ? x : (float)fdlibm_exp_inline((double)x);
+}
+
+// fround(Math.exp(x)) for x <= 0 (or NaN).
 __device__ __forceinline__ float exp_to_f32(float x) {
-  if (x != x) return x;
-  const double r = exp_nonpos((double)x);
-  const float y = (float)r;
-  const double res = r - (double)y;  // exact: r and y are within half an f32 ulp
-  const uint32_t yb = __float_as_uint(y);
-  const int e = (int)(yb >> 23);
-  double half = __builtin_ldexp(1.0, (e > 1 ? e : 1) - 151);  // half the f32 ulp above y
-  if (res < 0.0 && (yb & 0x7fffffu) == 0u && e > 1) half *= 0.5;  // below a power of two
-  if (__builtin_fabs(res) < half - r * 0x1p-44) return y;
-  return (float)fdlibm_exp_inline((double)x);
+  bool slow;
+  const float y = exp_to_f32_fast(x, slow);
+  return slow ? exp_to_f32_slow(x) : y;
 }
 
 // Out-of-line form for call sites where code size matters more than the call.

@@ -210,6 +210,35 @@ def test_softmax_attention_shapes(oracle):
         _check_softmax(oracle, y, 14, total, 1, total - 1)
 
 
+@pytest.mark.parametrize("n_rows,row_len", [(5, 2), (5, 255), (5, 256), (5, 257), (5, 511), (5, 513), (5, 1023),
+                                            (5, 1025), (5, 2047), (5, 2048), (5, 2049), (5, 4095), (5, 8190),
+                                            (5, 8193), (5, 16383), (5, 16384), (5, 16385), (300, 514),
+                                            (1030, 513), (1029, 700), (1027, 1023), (1026, 1024)])
+def test_softmax_chunk_edges(oracle, n_rows, row_len):
+    # Every width of the chunked sum (a thread's entries, a wave, the last partial group of
+    # four) and the lane-per-row sum of long rows, on the inputs where their bookkeeping can go
+    # wrong: sums that cross a binade at every entry (a geometric rise), that never leave one
+    # after the first entry, that tie on most additions, leading exps of zero or subnormal size,
+    # and NaN. Bit for bit.
+    rng = np.random.default_rng(row_len * 7 + n_rows)
+    x = rng.normal(0, 3, (n_rows, row_len)).astype(np.float32)
+    x[0] = np.linspace(-60.0, 0.0, row_len, dtype=np.float32)     # rising
+    x[1] = np.round(x[1] * 2) * 0.5                               # ties
+    x[2] = -30.0
+    x[2, 0] = 0.0                                                 # terms below half an ulp or near it
+    x[3, : row_len // 2] = -101.0 - rng.random(row_len // 2) * 5  # subnormal and zero exps first
+    x[4, row_len - 1] = 25.0                                      # the sum doubles many times at its last entry
+    if n_rows > 5:
+        x[5] = 0.0
+        x[6, row_len // 3] = np.nan
+        x[7] = -np.inf
+    x = x.reshape(-1)
+    _check_softmax(oracle, x, n_rows, row_len)
+    period = min(n_rows, row_len)
+    _check_softmax(oracle, x, n_rows, row_len, period, row_len - period, in_place=True)
+    _check_softmax(oracle, x, n_rows, row_len, period, 0)         # short causal prefixes
+
+
 def test_softmax_special_rows(oracle):
     row_len = 300
     x = np.random.default_rng(9).normal(0, 1, (6, row_len)).astype(np.float32)
