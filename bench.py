@@ -337,9 +337,9 @@ CALL_KERNELS = {
     2: "row_kernel on parts of the row, then wave_merge_kernel merging their lists and sampling",
     3: "row_kernel, one workgroup per row (streaming: max, sum-exp, candidates; then in LDS "
        "the exact top-k, top-p and draw)",
-    4: "row_kernel on parts of each row, wave_merge_kernel (statistics, head key, top list), "
-       "then the head kernels (head_kernel re-reads the row for its head, head_fast_kernel "
-       "finishes it; head_sort_kernel and head_finish_kernel for rows it cannot)",
+    4: "row_kernel on parts of each row, wave_merge_kernel (finishes rows that their top list "
+       "decides), then the head kernels for the rest (head_kernel re-reads the row, "
+       "head_pick_kernel finishes it by selection; head_sort_kernel for rows it cannot)",
     5: "pool_row_kernel, one workgroup per row (streaming with candidate appends; then in LDS "
        "the exact top-1024 selection, its sort, top-p and the draw)",
 }

@@ -27,8 +27,8 @@
 //     (sequential sums; V8's exp by the fdlibm method).
 // The kernel boundary orders the first kernel's writes before the second's reads; no
 // workgroup waits on another. Rows whose pool is the whole vocabulary (top_k = 0 beyond the
-// pool capacity) are finished by two more kernels that collect and sort the row's head
-// (see head_kernel).
+// pool capacity) end in the merge when their largest entries decide them, else in two more
+// kernels that weigh the row's head and select in it (see head_kernel, head_pick_kernel).
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -104,9 +104,9 @@ constexpr int kMaxSplits = kBlock;  // one merge lane per slice
 // reference ml = fl(lane_max * L). Rebased on a max m it is sum * 2^(ml - m*L), with m*L
 // formed exactly in f64 (two 24-bit significands): the exponent difference has no error
 // proportional to |m|, so the sum's accuracy does not depend on where the logits sit.
-__device__ __forceinline__ double rebase_sum(double sum, float lane_max, float ml, float m) {
+__device__ __forceinline__ double rebase_sum(double sum, float lane_max, float ml, float m, float scale = kLog2e) {
   if (lane_max == -INFINITY) return 0.0;
-  const double d = (double)ml - (double)m * (double)kLog2e;
+  const double d = (double)ml - (double)m * (double)scale;
   return sum * (double)__builtin_amdgcn_exp2f((float)d);
 }
 constexpr int kKcapSmall = 256;
@@ -125,15 +125,16 @@ constexpr uint32_t kPoolRowDone = 0xffffffffu;
 struct RowState {
   float max;
   uint32_t head_key;  // elements with key >= head_key form the row's head
+  uint32_t store_key; // >= head_key: those with key >= store_key hold the cut and the draw, and lie
+                      // within 37.5 T of the max
   double sum_exp;
   int32_t status;
   uint32_t handoff;   // bits 16..: length N of the row's sorted top list in head_sorted (0: none);
-                      // bit 0: head_fast_kernel finished the row
-  double list_sum;    // T > 0: the sequential sum of the list's terms exp((l_i - M)/T)
+                      // bit 0: the row is finished (by the merge or head_pick_kernel)
 };
 
 // Whole-vocabulary rows hand at least this many of their largest composites, sorted, from the
-// merge to head_fast_kernel.
+// merge to head_pick_kernel.
 constexpr int kHeadList = 32;
 
 struct Workspace {
@@ -141,15 +142,20 @@ struct Workspace {
   SliceStat *stats;         // [rows_cap * kMaxSplits]
   uint64_t *cands;          // [rows_cap * row_cand_stride]
   RowState *row_state;      // [rows_cap]
-  uint64_t *head;           // [head_rows * head_stride] whole-vocabulary rows: the head, slice s
-                            // of head_kernel at [s * h_slice_len, + head_slice_count)
+  uint64_t *head;           // [head_rows * head_stride] whole-vocabulary rows: slice s of head_kernel
+                            // stores from s * h_slice_len; a head to be sorted, from 0
   uint64_t *head_sorted;    // [head_rows * head_stride] the head, sorted
   double *head_s;           // [head_rows * head_stride] exp((l - max)/T) in sorted order
   double *head_c;           // [head_rows * head_stride] running sums of the weights
   uint32_t *head_plan;      // [head_rows * plan_stride] segment offsets of the sorted head
   double *head_part;        // [head_rows * 2 * (plan_stride - 2)] per-segment exp sums
-  double *head_acc;         // [head_rows * 3 * acc_stride] head_kernel's per-slice ulp counts
-  uint32_t *head_slice_count;  // [head_rows * acc_stride] head entries each slice stored
+  double *scaled;           // [head_rows * kMaxSplits] each slice's (or part's) sum over its elements of
+                            // exp((x - max) / T), max the slice's (whole-vocabulary rows)
+  double *head_bin_sum;     // [head_rows * acc_stride * kTableBins] a head slice's weight by bin, and ...
+  uint16_t *head_bin_start; // [same] ... its entries in the bins before (slices storing over kTableMin)
+  uint32_t *head_arrived;   // [head_rows] head_sort_kernel's workgroups that have sorted their share
+  uint32_t *head_slice_count;  // [head_rows * acc_stride * 2] entries each slice stored, and its head's size
+  double *head_slice_sum;   // [head_rows * acc_stride] each slice's weight over its head
   int32_t plan_stride;
   int32_t acc_stride;       // >= the head kernel's slices per row
   int64_t row_cand_stride;  // composites per row in cands
@@ -223,7 +229,7 @@ __device__ __forceinline__ bool greedy_temp(double T) { return T <= 0.0; }
 // whose pool fits the kernels (keff <= kcap); for a whole-vocabulary row, the top-k list the
 // caller asked for (topk_cap <= k_max <= kcap) and at least kHeadList, which the merge uses
 // to lower the row's head threshold far enough that the head holds that list, and hands on
-// sorted to head_fast_kernel.
+// sorted to head_pick_kernel.
 __device__ __forceinline__ int slice_keep(bool valid, int keff, int n, int kcap, int head_pass,
                                           int topk_cap) {
   if (!valid) return 0;
@@ -1190,6 +1196,13 @@ __device__ __forceinline__ SelBins sel_bins(uint32_t top, uint32_t bound) {
   return SelBins{top, bits > 8 ? bits - 8 : 0};
 }
 
+__device__ __forceinline__ bool is_head_row(const tabby_row_params &P, const Launch &L) {
+  return params_valid(P, L.k_max) && effective_k(P, L.vocab) > L.kcap;
+}
+
+// log2(e) / T in f32: the exponent's scale of a whole-vocabulary row's weights.
+__device__ __forceinline__ float scaled_log2e(double T) { return (float)((double)kLog2e / T); }
+
 // One wave's share of row `row`: slice `slice` of L.slice_len elements or, when `claim` is
 // given (CLAIM), chunk `slice` of the whole row and then every chunk the wave claims from the
 // LDS counter *claim (shared by the row's waves, starting past their first chunks), so that
@@ -1199,12 +1212,15 @@ __device__ __forceinline__ SelBins sel_bins(uint32_t top, uint32_t bound) {
 // workgroup, *claim starting at `waves`) also agree on a first bound through bound_keys (LDS
 // room for 8 x 64 keys) and one barrier. The wave's top min(count, kk), sorted descending,
 // go to out[0..keep) as composites (out may be sm.list itself: the list is read into
-// registers before anything is written), its statistics to *stat.
-template <typename In, int VEC, bool CLAIM>
+// registers before anything is written), its statistics to *stat. HEAD (launches that may hold
+// whole-vocabulary rows): such a row's sum of exp((x - max) / T) too, in the same f32 terms, to
+// *scaled, from which the merge finishes the rows whose top list decides them.
+template <typename In, int VEC, bool CLAIM, bool HEAD>
 __device__ __forceinline__ void wave_slice(WaveSmem &sm, const Launch &L, const tabby_row_params &P, int row,
                                            int slice, int part, uint64_t *out, SliceStat *stat, int *claim,
                                            uint32_t *bound_keys, int waves, bool sort_end = true,
-                                           uint32_t *bound_out = nullptr, uint32_t *sel_hist = nullptr) {
+                                           uint32_t *bound_out = nullptr, uint32_t *sel_hist = nullptr,
+                                           double *scaled = nullptr) {
   const int V = L.vocab;
   // CLAIM: the row, or part `part` of it (L.slice_len elements) when the row has several
   // workgroups.
@@ -1222,6 +1238,11 @@ __device__ __forceinline__ void wave_slice(WaveSmem &sm, const Launch &L, const 
   float lane_max = -INFINITY;
   float lane_ml = 0.0f;   // fl(lane_max * L): the reference of lane_sum's terms
   double lane_sum = 0.0;  // sum of 2^(x*L - lane_ml) over this lane's elements so far
+  // HEAD: the same at the row's temperature (at T = 1 the two are one).
+  const bool weigh = HEAD && is_head_row(P, L) && !greedy_temp(P.temperature) && P.temperature != 1.0;
+  const float lt = HEAD && weigh ? scaled_log2e(P.temperature) : 0.0f;
+  float lane_mlt = 0.0f;
+  double lane_sum_t = 0.0;
   int count = 0;          // entries in the list; wave-uniform (readfirstlane keeps it scalar)
   uint32_t theta_key = kNegInfKey;
   float theta = -INFINITY;  // == value_of(theta_key)
@@ -1262,6 +1283,21 @@ __device__ __forceinline__ void wave_slice(WaveSmem &sm, const Launch &L, const 
       const float part = t[0];
       const double rescale = lane_max == -INFINITY ? 0.0 : (double)__builtin_amdgcn_exp2f(lane_ml - ml);
       lane_sum = lane_sum * rescale + (double)part;
+      if constexpr (HEAD) {
+        if (weigh) {
+          const float mlt = nm * lt;
+#pragma unroll
+          for (int e = 0; e < kWChunkPerLane; ++e) t[e] = __builtin_amdgcn_exp2f(fmaf(cur[e], lt, -mlt));
+#pragma unroll
+          for (int h = kWChunkPerLane / 2; h > 0; h >>= 1) {
+#pragma unroll
+            for (int e = 0; e < h; ++e) t[e] += t[e + h];
+          }
+          const double down = lane_max == -INFINITY ? 0.0 : (double)__builtin_amdgcn_exp2f(lane_mlt - mlt);
+          lane_sum_t = lane_sum_t * down + (double)t[0];
+          lane_mlt = mlt;
+        }
+      }
       lane_max = nm;
       lane_ml = ml;
     }
@@ -1404,6 +1440,10 @@ __device__ __forceinline__ void wave_slice(WaveSmem &sm, const Launch &L, const 
 
   const float ms = wave_max(lane_max);
   const double ss = wave_sum(rebase_sum(lane_sum, lane_max, lane_ml, ms));
+  if constexpr (HEAD) {
+    const double st = weigh ? wave_sum(rebase_sum(lane_sum_t, lane_max, lane_mlt, ms, lt)) : ss;
+    if (wave_lane() == 0) *scaled = st;
+  }
   // The slice's top min(count, kk), sorted descending: the merge only has to merge sorted
   // lists.
   int keep = 0;
@@ -1439,15 +1479,16 @@ __device__ __forceinline__ void wave_slice(WaveSmem &sm, const Launch &L, const 
   }
 }
 
-template <typename In, int VEC>
+template <typename In, int VEC, bool HEAD>
 __global__ __launch_bounds__(kWaveSize) void wave_kernel(Launch L, Workspace W) {
   __shared__ WaveSmem sm;
   int row, slice;
   row_slice_of((int)blockIdx.x, L.rows, L.splits, row, slice);
   const tabby_row_params P = L.params[row];
-  wave_slice<In, VEC, false>(sm, L, P, row, slice, 0,
-                             W.cands + (size_t)row * W.row_cand_stride + (size_t)slice * L.list_stride,
-                             W.stats + (size_t)row * kMaxSplits + slice, nullptr, nullptr, 0);
+  wave_slice<In, VEC, false, HEAD>(sm, L, P, row, slice, 0,
+                                   W.cands + (size_t)row * W.row_cand_stride + (size_t)slice * L.list_stride,
+                                   W.stats + (size_t)row * kMaxSplits + slice, nullptr, nullptr, 0, true, nullptr,
+                                   nullptr, HEAD ? W.scaled + (size_t)row * kMaxSplits + slice : nullptr);
 }
 
 // Smallest key whose scaled logit (l - max)/T in f64 is >= -37.5 (the max's key when T <= 0:
@@ -1481,6 +1522,24 @@ __device__ __forceinline__ uint32_t head_threshold(float row_max, double T) {
     if (in_head(mid)) hi = mid; else lo = mid;
   }
   return hi;
+}
+
+// The entries among which a whole-vocabulary row's cut and draw lie: all with a weight of at
+// least (1 - p) S / n (S the row's total weight, n the vocabulary, p the top-p, or without a
+// cut the uniform), as the others together weigh less than (1 - p) S. S is a lower bound here
+// (the max's own weight, 1, where the first pass gave none), and the smallest weight's
+// logarithm is widened by 0.02, which covers that bound's 2^-16, its f32 logarithm and the
+// rounding of the value. On N(0, 2.5^2) logits with spikes, T = 1 and p = 0.95 that is one
+// entry in a hundred of the 37.5 T that can enter the sums.
+__device__ __forceinline__ uint32_t store_threshold(float row_max, const tabby_row_params &P, int vocab, double S,
+                                                    uint32_t weights_key) {
+  const double T = P.temperature;
+  const double p = P.top_p < 1.0 ? P.top_p : P.uniform;
+  const float share = (float)((1.0 - p) * ((S >= 0.99 && S < 1.0e30) ? S : 1.0) / (double)vocab);
+  if (greedy_temp(T) || !(share > 1.0e-37f)) return weights_key;
+  const double depth = 0.02 - 0.69314718055994530942 * (double)__builtin_amdgcn_logf(share);
+  const float v = (float)((double)row_max - depth * T);
+  return v == v ? max(weights_key, min(key_of(v), key_of(row_max))) : weights_key;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1624,9 +1683,8 @@ __global__ __launch_bounds__(kBlock) void merge_kernel(Launch L, Workspace W) {
   if (!finite) {
     // Whole-vocabulary row: hand max / sum-exp / the head threshold to the head kernels. The
     // candidates hold the row's top Nw = max(topk_cap, kHeadList) (slice_keep): when Nw fits a
-    // wave's register sort (<= 256) they go on sorted, with the sequential sum of their terms,
-    // to head_kernel and head_fast_kernel, as from finish_pool; the head also covers the
-    // caller's top-k list, the first topk_cap of them.
+    // wave's register sort (<= 256) they go on sorted to head_pick_kernel, as from finish_pool;
+    // the head also covers the caller's top-k list, the first topk_cap of them.
     const int Nw = min(max(L.topk_cap, kHeadList), V);
     const int need = min(L.topk_cap, V);
     uint32_t list_key = 0xffffffffu;
@@ -1668,24 +1726,15 @@ __global__ __launch_bounds__(kBlock) void merge_kernel(Launch L, Workspace W) {
         list_key = kNegInfKey;  // fewer candidates than the list: take the whole row
       }
     }
-    if (wave_id() != 0) return;
-    const double T = P.temperature;
-    double list_sum = 0.0;
-    if (handed > 0 && !greedy_temp(T)) {
-      double *terms = sm.u.tail.w;  // the histogram is no longer needed
-      for (int i = lane_id(); i < handed; i += kWaveSize)
-        terms[i] = fdlibm_exp(((double)value_of(composite_key(sm.sorted[i])) - (double)row_max) / T);
-      wave_lds_sync();
-      list_sum = wave_seq_sum(terms, handed, nullptr, INFINITY).total;
-    }
-    if (lane_id() == 0) {
+    if (threadIdx.x == 0) {
       RowState rs;
       rs.max = row_max;
       rs.sum_exp = sum_exp;
       rs.status = TABBY_OK;
       rs.handoff = (uint32_t)handed << 16;
-      rs.list_sum = list_sum;
-      rs.head_key = min(head_threshold(row_max, P.temperature), list_key);
+      const uint32_t weights_key = head_threshold(row_max, P.temperature);
+      rs.head_key = min(weights_key, list_key);
+      rs.store_key = store_threshold(row_max, P, V, 1.0, weights_key);
       W.row_state[row] = rs;
     }
     return;
@@ -1805,6 +1854,19 @@ __device__ __forceinline__ RowStats row_stats(const SliceStat *stats, int splits
       part += st[q].sum * (double)__builtin_amdgcn_exp2f((st[q].max - out.max) * kLog2e);
   out.sum_exp = wave_sum(part);
   return out;
+}
+
+// The slices' (or waves') sums of exp((x - max) / T), each against its own max, as one against
+// the row's: lane s holds slices s, s + 64, ...
+__device__ __forceinline__ double scaled_total(const SliceStat *stats, const double *scaled, int splits, float row_max,
+                                               double T) {
+  const float lt = scaled_log2e(T);
+  double part = 0.0;
+  for (int s = wave_lane(); s < splits; s += kWaveSize) {
+    const float m = stats[s].max;
+    if (m != -INFINITY) part += scaled[s] * (double)__builtin_amdgcn_exp2f((m - row_max) * lt);
+  }
+  return wave_sum(part);
 }
 
 // Length of slice s's list (s wave-uniform).
@@ -2073,10 +2135,72 @@ __device__ __forceinline__ RowPool row_pool(const Launch &L, const tabby_row_par
   return rp;
 }
 
-template <typename In, bool REG = false>
+// A whole-vocabulary row from its largest entries: sorted[0..K) descending, S the weight
+// exp((l - M)/T) of the whole row, known within `margin` (relative). True, with the drawn entry
+// and consideredCount, when the row is greedy or its cut lies within the first 64 entries and
+// every comparison that fixes the cut and the draw clears its threshold -- the cut's by
+// `margin`, the draw's, which compares sums of the list alone, by 2^-36 (as in reg_tail) -- so
+// that the reference decides the same way. By one wave.
+//
+// S from the f32 terms of the first pass (kScaledMargin): an exponent (x - M) * log2(e)/T of at
+// most 55 in size (smaller terms do not reach 2^-54 of the sum) carries the relative roundings
+// of log2(e), of log2(e)/T and of the fma, 2^-22.8 in all, so a term is within 55 * ln 2 *
+// 2^-22.8 = 2^-17.5 of its value; the exps and the sums add 2^-22. A sum that is not at least
+// nearly 1 (the max's own term) or not finite comes from exponents past f32: not decided here.
+constexpr double kScaledMargin = 1.0 / 65536.0;  // 2^-16
+__device__ __forceinline__ bool head_by_list(const uint64_t *sorted, int K, float row_max, const tabby_row_params &P,
+                                             double S, double margin, uint64_t &entry,
+                                             uint32_t &considered) {
+  const double T = P.temperature, top_p = P.top_p;
+  if (greedy_temp(T)) {
+    entry = sorted[0];
+    considered = 1u;
+    return true;
+  }
+  if (!(top_p < 1.0) || !(S >= 0.99) || !(S < 1.0e30)) return false;
+  const int lane = wave_lane();
+  const bool in = lane < min(K, kWaveSize);
+  const uint64_t v = in ? sorted[lane] : 0ull;
+  const double s = in ? exp_nonpos(((double)value_of(composite_key(v)) - (double)row_max) * (1.0 / T)) : 0.0;
+  const double run = wave_inclusive_scan(s), reach = top_p * S;
+  const uint64_t past = __ballot(in && run >= reach);
+  if (!past) return false;
+  const int cut = __ffsll((unsigned long long)past);
+  const double total = lane_f64(run, cut - 1), target = P.uniform * total;
+  const uint64_t hit = __ballot(lane < cut && target < run);
+  const int chosen = hit ? __ffsll((unsigned long long)hit) - 1 : cut - 1;
+  const double m1 = margin * total, m2 = 0x1p-36 * total;
+  const bool fail = (lane == cut - 1 && !(run > reach + m1)) || (lane == cut - 2 && !(run < reach - m1)) ||
+                    (lane == chosen && !(run > target + m2)) || (lane == chosen - 1 && !(run < target - m2));
+  if (__ballot(fail)) return false;
+  entry = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, chosen) |
+          ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), chosen) << 32);
+  considered = (uint32_t)cut;
+  return true;
+}
+
+// The result of a whole-vocabulary row decided without its sorted head (one lane).
+__device__ __forceinline__ void write_head_result(const Launch &L, int row, float row_max, double sum_exp,
+                                                  int topk_count, uint64_t entry, uint32_t considered) {
+  tabby_row_result res;
+  res.max_logit = row_max;
+  res.sum_exp = sum_exp;
+  // The pool is the whole row: poolMass = sum of exp(l_i - M) / sumExp over every element, 1
+  // up to rounding (a sequential sum of n such terms is within n * 2^-53 of it).
+  res.pool_mass = 1.0;
+  res.status = TABBY_OK;
+  res.topk_count = topk_count;
+  res.considered = considered;
+  res.pool_exhausted = 0;  // poolMass 1 is never below top_p
+  res.id = (int32_t)composite_index(entry);
+  res.probability = fdlibm_exp((double)value_of(composite_key(entry)) - (double)row_max) / sum_exp;
+  L.results[row] = res;
+}
+
+template <typename In, bool REG, bool HEAD>
 __device__ __forceinline__ void finish_pool(WaveMergeSmem &sm, const Launch &L, const Workspace &W, int row,
                                             const tabby_row_params &P, const RowPool &rp, float row_max,
-                                            double sum_exp);
+                                            double sum_exp, double scaled);
 
 template <typename In, class SumExp>
 __device__ __forceinline__ void reg_tail(uint64_t v, int K, const Launch &L, int row, const In *row_src,
@@ -2109,7 +2233,7 @@ __device__ __forceinline__ void merge_pool(WaveMergeSmem &sm, const RowLists &li
 
 // Merges row `row`'s sorted slice lists and statistics and finishes the row (at least four
 // waves; the lists and statistics are in global memory or in LDS; P is the row's parameters).
-template <typename In>
+template <typename In, bool HEAD>
 __device__ __forceinline__ void merge_row(WaveMergeSmem &sm, const Launch &L, const Workspace &W, int row,
                                           const tabby_row_params &P, const SliceStat *stats,
                                           const RowLists &lists) {
@@ -2121,7 +2245,11 @@ __device__ __forceinline__ void merge_row(WaveMergeSmem &sm, const Launch &L, co
   auto count_of = [&](int s) { return list_count(rs, s); };
   const RowPool rp = row_pool(L, P);
   merge_pool(sm, lists, m1, count_of, rp.K);
-  finish_pool<In, true>(sm, L, W, row, P, rp, rs.max, rs.sum_exp);
+  // A head pass's whole-vocabulary row (W.scaled is written for no other).
+  const double scaled = HEAD && rp.valid && !rp.finite
+                            ? scaled_total(stats, W.scaled + (size_t)row * kMaxSplits, lists.count, rs.max, P.temperature)
+                            : 0.0;
+  finish_pool<In, true, HEAD>(sm, L, W, row, P, rp, rs.max, rs.sum_exp, scaled);
 }
 
 // The rest of a row once its pool, sm.sorted[0..K), and its max and sum-exp are known: the
@@ -2129,10 +2257,10 @@ __device__ __forceinline__ void merge_row(WaveMergeSmem &sm, const Launch &L, co
 // and wave 1 work; every wave of the workgroup must call it. REG: finite pools take wave 0's
 // register tail (the merge kernels; row_kernel's small pools end in finish_small_pool, and
 // its general path keeps the two-wave form).
-template <typename In, bool REG>
+template <typename In, bool REG, bool HEAD>
 __device__ __forceinline__ void finish_pool(WaveMergeSmem &sm, const Launch &L, const Workspace &W, int row,
                                             const tabby_row_params &P, const RowPool &rp, float row_max,
-                                            double sum_exp) {
+                                            double sum_exp, double scaled) {
   const int lane = wave_lane();
   const int K = rp.K;
   const bool valid_params = rp.valid, finite = rp.finite;
@@ -2177,7 +2305,7 @@ __device__ __forceinline__ void finish_pool(WaveMergeSmem &sm, const Launch &L, 
     __syncthreads();
   }
   if (wave_id() != 0) return;
-  if (!valid_params || !in_domain || (!finite && !L.head_pass)) {
+  if (!valid_params || !in_domain || (!finite && !HEAD)) {
     const int32_t status = !valid_params ? TABBY_EINVAL : !in_domain ? TABBY_EDOMAIN : TABBY_EINVAL;
     if (lane == 0) {
       write_status(L, row, status, row_max, sum_exp);
@@ -2185,28 +2313,41 @@ __device__ __forceinline__ void finish_pool(WaveMergeSmem &sm, const Launch &L, 
     }
     return;
   }
-  if (!finite) {
-    // Whole-vocabulary row: hand max / sum-exp / the head threshold to the head kernels, and
-    // the row's top K, sorted[0..K), to head_kernel and head_fast_kernel. The head also
-    // covers the caller's top-k list, the first topk_cap of them.
-    uint64_t *list = W.head_sorted + (size_t)row * W.head_stride;
-    const double T = P.temperature;
-    for (int i = lane; i < K; i += kWaveSize) {
-      list[i] = sm.sorted[i];
-      if (!greedy_temp(T)) sm.b[i] = fdlibm_exp_inline(((double)value_of(composite_key(sm.sorted[i])) - (double)row_max) / T);
+  if constexpr (HEAD) if (!finite) {
+    // Whole-vocabulary row, K > 0 of its largest entries sorted: finished here when they decide
+    // it (head_by_list).
+    uint64_t entry = 0ull;
+    uint32_t considered = 0u;
+    if (K > 0 && head_by_list(sm.sorted, K, row_max, P, scaled, kScaledMargin, entry, considered)) {
+      if (lane == 0) {
+        write_head_result(L, row, row_max, sum_exp, min(L.topk_cap, L.vocab), entry, considered);
+        RowState st{};
+        st.status = TABBY_OK;
+        st.handoff = 1u;
+        W.row_state[row] = st;
+      }
+      for (int i = lane; i < min(L.topk_cap, K); i += kWaveSize) {
+        const uint32_t idx = composite_index(sm.sorted[i]);
+        L.topk_ids[(size_t)row * L.topk_cap + i] = (int32_t)idx;
+        L.topk_logits[(size_t)row * L.topk_cap + i] = load_one(row_src + min(idx, (uint32_t)(L.vocab - 1)));
+      }
+      return;
     }
-    wave_lds_sync();
-    const double list_sum = !greedy_temp(T) && K > 0 ? wave_seq_sum(sm.b, K, nullptr, INFINITY).total : 0.0;
+    // Otherwise hand max / sum-exp / the head threshold to the head kernels, and the list to
+    // head_pick_kernel. The head also covers the caller's top-k list, the first topk_cap of it.
+    uint64_t *list = W.head_sorted + (size_t)row * W.head_stride;
+    for (int i = lane; i < K; i += kWaveSize) list[i] = sm.sorted[i];
     if (lane == 0) {
       RowState st;
       st.max = row_max;
       st.sum_exp = sum_exp;
       st.status = TABBY_OK;
       st.handoff = (uint32_t)K << 16;
-      st.list_sum = list_sum;
       const int kt = min(L.topk_cap, K);  // the caller's top-k list must lie in the head
       const uint32_t list_key = kt > 0 ? composite_key(sm.sorted[kt - 1]) : 0xffffffffu;
-      st.head_key = min(head_threshold(row_max, P.temperature), list_key);
+      const uint32_t weights_key = head_threshold(row_max, P.temperature);
+      st.head_key = min(weights_key, list_key);
+      st.store_key = store_threshold(row_max, P, L.vocab, scaled, weights_key);
       W.row_state[row] = st;
     }
     return;
@@ -2214,13 +2355,13 @@ __device__ __forceinline__ void finish_pool(WaveMergeSmem &sm, const Launch &L, 
   wave_tail<In>(sm, K, L, row, row_src, row_max, sum_exp, P);
 }
 
-template <typename In>
+template <typename In, bool HEAD>
 __global__ __launch_bounds__(kBlock) void wave_merge_kernel(Launch L, Workspace W) {
   __shared__ WaveMergeSmem sm;
   const int row = (int)blockIdx.x;
   const RowLists lists{W.cands + (size_t)row * W.row_cand_stride, L.splits, L.list_stride, W.row_cand_stride};
   const tabby_row_params P = L.params[row];
-  merge_row<In>(sm, L, W, row, P, W.stats + (size_t)row * kMaxSplits, lists);
+  merge_row<In, HEAD>(sm, L, W, row, P, W.stats + (size_t)row * kMaxSplits, lists);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -2254,6 +2395,7 @@ struct RowSmem {
   uint32_t fin_mask;     // the waves finished streaming (the last one selects the take)
   uint32_t sel_take[2];  // the take's smallest key and its size
   uint32_t part_mask;    // the waves whose statistics the second-to-last one combined ...
+  double scaled[kRowWaves];  // each wave's sum of exp((x - max) / T) (whole-vocabulary rows)
   float part_max;        // ... their max
   double part_sum;       // ... and sum-exp against it
   uint32_t bound_key[2];  // the row's first bound and the largest key of its union
@@ -2628,7 +2770,7 @@ __global__ __launch_bounds__(kBlock) void lmhead_merge_kernel(Launch L, Workspac
   const RowLists lists{W.cands + (size_t)row * W.row_cand_stride, L.splits, L.list_stride, W.row_cand_stride};
   const int K = rp.K;
   if (!(rp.valid && rp.finite && K > 0 && K <= kWaveSize)) {
-    merge_row<float>(sm.m, L, W, row, P, stats, lists);  // statuses of out-of-contract rows
+    merge_row<float, false>(sm.m, L, W, row, P, stats, lists);  // statuses of out-of-contract rows
     return;
   }
   const uint64_t *list = lists.base + (size_t)s * L.list_stride;
@@ -2668,7 +2810,7 @@ __global__ __launch_bounds__(kBlock) void lmhead_merge_kernel(Launch L, Workspac
   const uint32_t before = block_exclusive_scan((uint32_t)take, sm.bs, &total_u);
   const int total = (int)total_u;
   if (total > 4 * kWaveSize) {
-    merge_row<float>(sm.m, L, W, row, P, stats, lists);
+    merge_row<float, false>(sm.m, L, W, row, P, stats, lists);
     return;
   }
   for (int i = 0; i < take; ++i) sm.surv[before + i] = list[i];
@@ -2711,12 +2853,12 @@ __global__ __launch_bounds__(kBlock) void lmhead_merge_kernel(Launch L, Workspac
 // its top K and statistics on to wave_merge_kernel. Returns false, with every wave's list
 // sorted in place and its count cut to K, when more than 64 entries would be taken (the
 // general merge then takes over). Every wave calls it.
-template <typename In>
+template <typename In, bool HEAD>
 __device__ __forceinline__ bool finish_small_pool(RowSmem &sm, const Launch &L, const Workspace &W, int row, int part,
                                   const tabby_row_params &P, const RowPool &rp, int nw);
 __device__ __forceinline__ void small_pool_select(RowSmem &sm, int K);
 
-template <typename In, int VEC>
+template <typename In, int VEC, bool HEAD>
 __global__ __launch_bounds__(kRowWaves * kWaveSize) void row_kernel(Launch L, Workspace W) {
   __shared__ RowSmem sm;
   int row = (int)blockIdx.x, part = 0;
@@ -2740,8 +2882,9 @@ __global__ __launch_bounds__(kRowWaves * kWaveSize) void row_kernel(Launch L, Wo
   }
   for (int i = (int)threadIdx.x; i < kSelBins; i += (int)blockDim.x) sm.sel_hist[i] = 0u;
   __syncthreads();
-  wave_slice<In, VEC, true>(sm.wave[w], L, P, row, w, part, sm.wave[w].list, &sm.stats[w], &sm.next_chunk,
-                            sm.bound_keys, nw, !small, sm.bound_key, small ? sm.sel_hist : nullptr);
+  wave_slice<In, VEC, true, HEAD>(sm.wave[w], L, P, row, w, part, sm.wave[w].list, &sm.stats[w], &sm.next_chunk,
+                                  sm.bound_keys, nw, !small, sm.bound_key, small ? sm.sel_hist : nullptr,
+                                  HEAD ? &sm.scaled[w] : nullptr);
   TABBY_STAMP(w);
   if (small) {
     // Each wave marks itself finished; the waves marked before it are in the returned mask.
@@ -2780,7 +2923,7 @@ __global__ __launch_bounds__(kRowWaves * kWaveSize) void row_kernel(Launch L, Wo
   }
   __syncthreads();
   if (w == 0) TABBY_STAMP(17);
-  if (small && finish_small_pool<In>(sm, L, W, row, part, P, rp, nw)) return;
+  if (small && finish_small_pool<In, HEAD>(sm, L, W, row, part, P, rp, nw)) return;
   constexpr int stride = (int)(sizeof(WaveSmem) / sizeof(uint64_t));
   const RowLists lists{sm.wave[0].list, nw, stride, (int64_t)nw * stride};
   ListMerger<1> m1 = lists_of_wave<1>(lists);
@@ -2810,10 +2953,15 @@ __global__ __launch_bounds__(kRowWaves * kWaveSize) void row_kernel(Launch L, Wo
         st.sum = sm.merge.row_sum;
         W.stats[(size_t)row * kMaxSplits + part] = st;
       }
+      if constexpr (HEAD) {
+        const double scaled = scaled_total(sm.stats, sm.scaled, nw, sm.merge.row_max, P.temperature);
+        if (wave_lane() == 0) W.scaled[(size_t)row * kMaxSplits + part] = scaled;
+      }
     }
     return;
   }
-  finish_pool<In>(sm.merge, L, W, row, P, rp, sm.merge.row_max, sm.merge.row_sum);
+  const double scaled = HEAD ? scaled_total(sm.stats, sm.scaled, nw, sm.merge.row_max, P.temperature) : 0.0;
+  finish_pool<In, false, HEAD>(sm.merge, L, W, row, P, rp, sm.merge.row_max, sm.merge.row_sum, scaled);
 }
 
 // The take of a row whose pool is at most kSmallPoolMax (finish_small_pool): the bin holding
@@ -2865,7 +3013,7 @@ __device__ __forceinline__ void small_pool_select(RowSmem &sm, int K) {
   }
 }
 
-template <typename In>
+template <typename In, bool HEAD>
 __device__ __forceinline__ bool finish_small_pool(RowSmem &sm, const Launch &L, const Workspace &W, int row, int part,
                                                   const tabby_row_params &P, const RowPool &rp, int nw) {
   const int w = wave_id(), lane = wave_lane();
@@ -2935,6 +3083,10 @@ __device__ __forceinline__ bool finish_small_pool(RowSmem &sm, const Launch &L, 
         st.sum = S1;
         W.stats[(size_t)row * kMaxSplits + part] = st;
       }
+      if constexpr (HEAD) {
+        const double scaled = scaled_total(sm.stats, sm.scaled, nw, M, P.temperature);
+        if (lane == 0) W.scaled[(size_t)row * kMaxSplits + part] = scaled;
+      }
       return;
     }
     if (!((M > -INFINITY) && (M < INFINITY))) {
@@ -2991,142 +3143,261 @@ __device__ __forceinline__ bool finish_small_pool(RowSmem &sm, const Launch &L, 
 // or, divided by that total, to a running weight sum (>= the first weight), below half an
 // ulp of either, so it cannot change them (head_threshold). The merge computes head_key, the
 // smallest key with (l - M)/T >= -37.5 in f64 (or the max's key when T <= 0). head_kernel
-// collects the head; head_fast_kernel finishes the row from the merge's sorted top list when
-// that provably decides it, else the sort and finish kernels sort the head and run the tail
-// (there poolMass takes the head's terms plus the rest of sum-exp).
+// collects the head with its weights binned; head_pick_kernel finishes the row by selection
+// when that provably decides it, else the sort and finish kernels sort the head and run the
+// tail (there poolMass takes the head's terms plus the rest of sum-exp).
 // ---------------------------------------------------------------------------------------
-__device__ __forceinline__ bool is_head_row(const tabby_row_params &P, const Launch &L) {
-  return params_valid(P, L.k_max) && effective_k(P, L.vocab) > L.kcap;
-}
+// Bins of a stored entry by its distance below the max, over the range that is stored: bin 0
+// holds the largest, so bins in order are the entries in descending order (unsorted within a
+// bin, equal logits together).
+constexpr int kPickBins = 1024;  // head_pick_kernel's, of up to kPickFew stored entries
+constexpr int kTableBins = 128;  // head_kernel's, a slice at a time
 
+struct PickBin {
+  float max, scale;  // bins per unit of M - l (finite: 0 * scale is 0)
+  float last;
+  __device__ __forceinline__ PickBin(const RowState &rs, int bins) : max(rs.max), last((float)(bins - 1)) {
+    const float span = rs.max - value_of(rs.store_key);
+    scale = span > 0.0f ? fminf((float)bins / span, 1.0e38f) : 0.0f;
+  }
+  // Non-increasing in x: one f32 subtraction and one product, each rounded monotonically.
+  __device__ __forceinline__ int of(float x) const { return (int)fminf((max - x) * scale, last); }
+};
 
-// The whole-vocabulary tail without sorting the head, when that is provably the same.
-// sampleFromTopK over the sorted head needs three sequential f64 sums: the scaled total S and
-// the running sums of w_i = s_i / S up to the cut (s_i = exp((l_i - M)/T), V8's exp). The
-// merge hands over the row's top N sorted (N = max(topk_cap, 64), finish_pool). Once a
-// partial sum P lies in [2^E, 2^(E+1)), adding a term s gives P + u * rint(s / u) exactly
-// (u = 2^(E-52)) unless s / u lies exactly halfway between integers (then the parity of P
-// decides). So if P_N, the sequential sum of the top N, is in binade E, every later term --
-// each smaller than the top N -- adds rint(s / u) ulps whatever the order, provided none ties
-// and the total stays below 2^(E+1), and then S = P_N + u * (sum of rint(s / u) over the
-// rest of the head). head_kernel counts those ulps (and the ties) for the head entries it
-// collects; both conditions are checked exactly (the counts are integers below 2^53, exact
-// in f64 in any order, and a total that reaches 2^53 stays there). A term's s / u comes from
-// the fast exp when it is below 2^36 and at least 2^-9 from a half: exp_nonpos is within 8
-// ulp of e^x and V8's exp within 1, so the two differ by under 9 * 2^-52 * 2^36 < 2^-12
-// there and round alike; other terms take V8's exp. When the running sums also reach the cut
-// within the top N (or the head holds nothing beyond them), head_fast_kernel finishes the
-// row -- bit for bit what the sorted head gives -- and marks it (RowState.handoff bit 0) so
-// that the sort and finish kernels skip it; otherwise it plans the sorted head. (Terms just
-// below P's binade tie often -- s in [2^(E-1), 2^E) has one bit below the ulp -- which is
-// why the top N are summed in order.)
-
-// 2^(52 - E) for P in [2^E, 2^(E+1)): s * ulp_scale(P) is s in ulps of P.
-__device__ __forceinline__ double ulp_scale(double P) {
-  const int E = (int)(((uint64_t)__double_as_longlong(P) >> 52) & 0x7ff) - 1023;
-  return __builtin_ldexp(1.0, 52 - E);
-}
-
-// Adds rint(s / u) for the term of composite v to r, and 1 to ties if s / u is a half-integer.
-__device__ __forceinline__ void add_ulps(uint64_t v, double M, double T, double scale, double &r, double &ties) {
-  const double dt = ((double)value_of(composite_key(v)) - M) / T;
-  double q = exp_nonpos(dt) * scale;
-  if (!(q < 68719476736.0 && __builtin_fabs(q - __builtin_floor(q) - 0.5) > 0x1p-9)) q = fdlibm_exp(dt) * scale;
-  ties += q - __builtin_floor(q) == 0.5 ? 1.0 : 0.0;
-  r += __builtin_rint(q);
+__device__ __forceinline__ void lds_add(double *p, double v) {
+  __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
 // head_kernel's slices: two wave chunks, both loaded before either is used.
 constexpr int kHeadSlice = 2 * kWChunk;
 
-// Collects the head (elements with key >= head_key) of one slice of a row into the row's head
-// buffer and, when the merge handed over the row's top N and T > 0, writes the slice's ulp
-// counts for head_fast_kernel: the sum of rint(s / u) over its head entries below the top N,
-// their number of ties, and their count.
+// exp(d / T) for the head's total weight, from y = d / T * 64 log2(e): y = 64 k + j + r with
+// |r| <= 1/2, and 2^(y/64) = 2^k * 2^(j/64) * e^(r ln2 / 64), the second factor from a table of
+// 64 (LDS) and the third a polynomial of degree 4 (truncation (ln2/128)^5 / 120 < 2^-44). The
+// rounding to an integer is an addition of 1.5 * 2^52, whose low bits are then 64 k + j. For
+// -64 * 1022 < y <= 0; other arguments give no meaningful value.
+constexpr int kExpSteps = 64;
+static_assert(kExpSteps == kWaveSize, "one table entry per lane");
+__device__ const double kExp2Steps[kExpSteps] = {  // 2^(j/64)
+    0x1.0000000000000p+0, 0x1.02c9a3e778061p+0, 0x1.059b0d3158574p+0, 0x1.0874518759bc8p+0,
+    0x1.0b5586cf9890fp+0, 0x1.0e3ec32d3d1a2p+0, 0x1.11301d0125b51p+0, 0x1.1429aaea92de0p+0,
+    0x1.172b83c7d517bp+0, 0x1.1a35beb6fcb75p+0, 0x1.1d4873168b9aap+0, 0x1.2063b88628cd6p+0,
+    0x1.2387a6e756238p+0, 0x1.26b4565e27cddp+0, 0x1.29e9df51fdee1p+0, 0x1.2d285a6e4030bp+0,
+    0x1.306fe0a31b715p+0, 0x1.33c08b26416ffp+0, 0x1.371a7373aa9cbp+0, 0x1.3a7db34e59ff7p+0,
+    0x1.3dea64c123422p+0, 0x1.4160a21f72e2ap+0, 0x1.44e086061892dp+0, 0x1.486a2b5c13cd0p+0,
+    0x1.4bfdad5362a27p+0, 0x1.4f9b2769d2ca7p+0, 0x1.5342b569d4f82p+0, 0x1.56f4736b527dap+0,
+    0x1.5ab07dd485429p+0, 0x1.5e76f15ad2148p+0, 0x1.6247eb03a5585p+0, 0x1.6623882552225p+0,
+    0x1.6a09e667f3bcdp+0, 0x1.6dfb23c651a2fp+0, 0x1.71f75e8ec5f74p+0, 0x1.75feb564267c9p+0,
+    0x1.7a11473eb0187p+0, 0x1.7e2f336cf4e62p+0, 0x1.82589994cce13p+0, 0x1.868d99b4492edp+0,
+    0x1.8ace5422aa0dbp+0, 0x1.8f1ae99157736p+0, 0x1.93737b0cdc5e5p+0, 0x1.97d829fde4e50p+0,
+    0x1.9c49182a3f090p+0, 0x1.a0c667b5de565p+0, 0x1.a5503b23e255dp+0, 0x1.a9e6b5579fdbfp+0,
+    0x1.ae89f995ad3adp+0, 0x1.b33a2b84f15fbp+0, 0x1.b7f76f2fb5e47p+0, 0x1.bcc1e904bc1d2p+0,
+    0x1.c199bdd85529cp+0, 0x1.c67f12e57d14bp+0, 0x1.cb720dcef9069p+0, 0x1.d072d4a07897cp+0,
+    0x1.d5818dcfba487p+0, 0x1.da9e603db3285p+0, 0x1.dfc97337b9b5fp+0, 0x1.e502ee78b3ff6p+0,
+    0x1.ea4afa2a490dap+0, 0x1.efa1bee615a27p+0, 0x1.f50765b6e4540p+0, 0x1.fa7c1819e90d8p+0,
+};
+__device__ __forceinline__ double exp_sum_term(double y, const double *table) {
+  const double shifted = y + 6755399441055744.0;
+  const int i = (int)(uint32_t)__double_as_longlong(shifted);  // 64 k + j
+  const double r = (y - (shifted - 6755399441055744.0)) * (6.93147180559945286227e-01 / kExpSteps);
+  const double p = __builtin_fma(r, __builtin_fma(r, __builtin_fma(r, __builtin_fma(r, 1.0 / 24.0, 1.0 / 6.0), 0.5), 1.0), 1.0);
+  const uint64_t bits = (uint64_t)__double_as_longlong(table[i & (kExpSteps - 1)] * p);
+  return __longlong_as_double((long long)(bits + ((uint64_t)(uint32_t)(i >> 6) << 52)));
+}
+
+// One slice of a whole-vocabulary row: its weight, sum_i exp((l_i - M)/T) over its part of the
+// head (elements with key >= head_key; f64 exps, added per lane), and its entries with key >=
+// store_key, in the slice's range of the row's head buffer (a row's slices appending to one
+// counter serialised on it).
+//
+// What bounds it: the f64 exps of the whole head (64 rows of 151,936 at T = 1: every element),
+// taken by exp_sum_term in half the instructions of exp_nonpos. A slice with at most
+// kHeadSparse elements in the head (most of a cold row's: T = 0.3) takes their exps from an LDS
+// list, eight or two to a lane instead of 32.
+//
+// A warm row stores several percent of its entries (store_threshold), more than head_pick_kernel
+// could search in one workgroup without order (64 rows at T = 1: 78 us there), so a slice that
+// stores more than kTableMin orders its entries by bin and writes each bin's weight and where
+// its entries start (18 us there and 17 us here, traced; storing the whole head in bin order, its
+// 8-byte stores scattered over each slice's 16 KB, took 26 us here). One 64-bit LDS add per
+// entry counts it (the low 12 bits) and adds its weight (the upper 52) in fixed point: bin b's
+// weights, below 2^-k, k = floor(b * width), are scaled by 2^(40 + k), so 2,048 of them stay
+// below 2^52 and each is rounded by at most 2^-41 of 2^-k, 2^-39 of its value (a bin is at most
+// 0.43 binary orders wide: the range stored is within 37.5 T of the max).
+constexpr int kHeadSparse = 8 * kWaveSize;
+constexpr int kTableMin = 32;
+constexpr int kWeightBits = 40;
+
 template <typename In, int VEC>
 __global__ __launch_bounds__(kWaveSize) void head_kernel(Launch L, Workspace W) {
-  __shared__ uint64_t list[kWListCap];
+  __shared__ unsigned long long bin_acc[kTableBins];
+  __shared__ uint32_t bin_at[kTableBins];
+  __shared__ uint64_t list[kHeadSparse];
+  __shared__ double exp_table[kExpSteps];
   int row, slice;
   row_slice_of((int)blockIdx.x, L.rows, L.h_splits, row, slice);
   const int V = L.vocab, lane = wave_lane();
   const int begin = slice * L.h_slice_len;
   const int n = min(L.h_slice_len, V - begin);
-  const int nchunks = (n + kWChunk - 1) / kWChunk;
-  const int full_chunks = n / kWChunk;
   const In *src = reinterpret_cast<const In *>(L.logits) + (size_t)row * V + begin;
   // Both chunks' loads at once (a slice's second chunk past the row's end reads zeros),
   // issued with the row's parameters and state rather than after them: one round trip for
   // all three (a row that turns out to need no head pass has read its slice for nothing).
-  float x[kWChunkPerLane], y[kWChunkPerLane];
-  const ChunkReader<In, VEC> rd(src, n);
-  rd.load(0, x);
-  rd.load(1, y);
-  const tabby_row_params P = L.params[row];
-  const RowState rs = W.row_state[row];
-  if (!is_head_row(P, L) || rs.status != TABBY_OK) return;
-  const float hv = value_of(rs.head_key);
-  // This slice's part of the head goes to its own range of the row's head buffer (no
-  // atomics: a row's slices appending to one counter serialised on it).
-  uint64_t *head = W.head + (size_t)row * W.head_stride + begin;
-  int stored = 0;
-  // The ulp of P_N (the sequential sum of the top N's terms, from the merge).
-  const int N = (int)(rs.handoff >> 16);
-  const double T = P.temperature, M = (double)rs.max;
-  const bool count_ulps = !greedy_temp(T) && N > 0 && N <= kWaveKcap;
-  const double scale = ulp_scale(rs.list_sum);
-  const uint64_t last = count_ulps ? W.head_sorted[(size_t)row * W.head_stride + N - 1] : 0ull;
-  double r = 0.0, ties = 0.0, outside = 0.0;
-  int count = 0;
-  auto flush = [&]() {
-    wave_lds_sync();
-    for (int i = lane; i < count; i += kWaveSize) {
-      const uint64_t v = list[i];
-      head[stored + i] = v;
-      if (count_ulps && v < last) {
-        add_ulps(v, M, T, scale, r, ties);
-        outside += 1.0;
-      }
-    }
-    stored += count;
-    count = 0;
-    wave_lds_sync();
-  };
-  auto collect = [&](int c, float(&cur)[kWChunkPerLane]) {
-    if (c >= full_chunks) {
-#pragma unroll
-      for (int e = 0; e < kWChunkPerLane; ++e)
-        if (wave_local<VEC>(c, e) >= n) cur[e] = __builtin_nanf("");  // fails cur >= hv
-    }
+  float x[2 * kWChunkPerLane];
+  {
+    float lo[kWChunkPerLane], hi[kWChunkPerLane];
+    const ChunkReader<In, VEC> rd(src, n);
+    rd.load(0, lo);
+    rd.load(1, hi);
 #pragma unroll
     for (int e = 0; e < kWChunkPerLane; ++e) {
-      if (count > kWListCap - kWaveSize) flush();
-      const bool take = cur[e] >= hv;
+      x[e] = lo[e];
+      x[kWChunkPerLane + e] = hi[e];
+    }
+  }
+  exp_table[lane] = kExp2Steps[lane];
+  const tabby_row_params P = L.params[row];
+  const RowState rs = W.row_state[row];
+  if (!is_head_row(P, L) || rs.status != TABBY_OK || (rs.handoff & 1u)) return;
+  const float hv = value_of(rs.head_key), sv = value_of(rs.store_key);
+  const double T = P.temperature, M = (double)rs.max;
+  const bool weigh = !greedy_temp(T);
+  const double inv_t = weigh ? 1.0 / T : 0.0;
+  const double per_unit = inv_t * (kExpSteps * 1.44269504088896338700e+00);
+  static_assert(kTableBins == 2 * kWaveSize, "two bins per lane");
+  bin_acc[lane] = bin_acc[kWaveSize + lane] = 0ull;
+  auto local_of = [&](int e) {
+    return e < kWChunkPerLane ? wave_local<VEC>(0, e) : wave_local<VEC>(1, e - kWChunkPerLane);
+  };
+  if (n < kHeadSlice) {  // the row's last slice
+#pragma unroll
+    for (int e = 0; e < 2 * kWChunkPerLane; ++e)
+      if (local_of(e) >= n) x[e] = __builtin_nanf("");  // fails every x >= v
+  }
+  // The slice's elements at or above `bound` into the list, as far as it goes; their number.
+  auto gather = [&](float bound) {
+    int count = 0;
+#pragma unroll
+    for (int e = 0; e < 2 * kWChunkPerLane; ++e) {
+      const bool take = x[e] >= bound;
       const uint64_t mask = __ballot(take);
       if (mask) {
-        if (take) list[count + (int)lanes_below(mask)] = composite(key_of(cur[e]), (uint32_t)(begin + wave_local<VEC>(c, e)));
+        const int at = count + (int)lanes_below(mask);
+        if (take && at < kHeadSparse) list[at] = raw_entry(x[e], (uint32_t)local_of(e));
         count = __builtin_amdgcn_readfirstlane(count + (int)__popcll(mask));
       }
     }
+    wave_lds_sync();
+    return count;
   };
-  static_assert(kHeadSlice == 2 * kWChunk, "head_kernel's slices are two chunks");
-  collect(0, x);
-  if (nchunks > 1) collect(1, y);
-  if (count > 0) flush();
-  if (lane == 0) W.head_slice_count[(size_t)row * W.acc_stride + slice] = (uint32_t)stored;
-  if (count_ulps) {
-    r = wave_sum(r);  // integers: exact below 2^53, and at least 2^53 once the total is
-    ties = wave_sum(ties);
-    outside = wave_sum(outside);
-    if (lane == 0) {
-      double *acc = W.head_acc + ((size_t)row * W.acc_stride + slice) * 3;
-      acc[0] = r;
-      acc[1] = ties;
-      acc[2] = outside;
+  const int in_head = gather(hv);
+  int stored = 0;
+  wave_lds_sync();  // the table and the cleared bins
+  uint64_t *head = W.head + (size_t)row * W.head_stride + begin;
+  double sum = 0.0;
+  // The weights of S elements of each lane that lie in the head (value(e); NaN: none).
+  auto weigh_head = [&](auto steps, auto value) {
+    constexpr int S = decltype(steps)::value;
+    if (!weigh) return;
+#pragma unroll
+    for (int e = 0; e < S; ++e) {
+      const double term = exp_sum_term(((double)value(e) - M) * per_unit, exp_table);
+      sum += value(e) >= hv ? term : 0.0;
     }
+  };
+  // The entries among them, at local(e): in bin order with the slice's table, or as they come.
+  auto store = [&](auto steps, auto value, auto local) {
+    constexpr int S = decltype(steps)::value;
+    if (stored <= kTableMin) {
+      int at = 0;
+#pragma unroll
+      for (int e = 0; e < S; ++e) {
+        const float v = value(e);
+        const uint64_t mask = __ballot(v >= sv);
+        if (v >= sv) head[at + (int)lanes_below(mask)] = composite(key_of(v), (uint32_t)(begin + local(e)));
+        at += (int)__popcll(mask);
+      }
+      return;
+    }
+    const PickBin bins(rs, kTableBins);
+    // Binary orders of weight per bin (0 where a greedy row has no weights).
+    const float width =
+        weigh ? fminf((float)(((double)rs.max - (double)sv) * inv_t * (1.4426950408889634 / kTableBins)), 1.0f) : 0.0f;
+    auto bin_shift = [&](int b) { return (int)((float)b * width); };
+#pragma unroll
+    for (int e = 0; e < S; ++e) {
+      const float v = value(e);
+      if (v >= sv) {
+        const int b = bins.of(v);
+        unsigned long long add = 1ull;
+        if (weigh) {
+          // rint of the scaled weight, below 2^52, by an addition to 2^52.
+          const double scaled = __builtin_ldexp(exp_nonpos(((double)v - M) * inv_t), kWeightBits + bin_shift(b));
+          add |= ((unsigned long long)__double_as_longlong(scaled + kTwo52) & 0xfffffffffffffull) << 12;
+        }
+        atomicAdd(&bin_acc[b], add);
+      }
+    }
+    wave_lds_sync();
+    // Each bin's start: an exclusive scan, lane i holding bins 2i and 2i + 1.
+    const unsigned long long a0 = bin_acc[2 * lane], a1 = bin_acc[2 * lane + 1];
+    const uint32_t c0 = (uint32_t)a0 & 0xfffu, c1 = (uint32_t)a1 & 0xfffu;
+    const uint32_t first = wave_inclusive_scan_u32(c0 + c1) - c0 - c1;
+    bin_at[2 * lane] = first;
+    bin_at[2 * lane + 1] = first + c0;
+    const size_t table = ((size_t)row * W.acc_stride + slice) * kTableBins + 2 * lane;
+    W.head_bin_start[table] = (uint16_t)first;
+    W.head_bin_start[table + 1] = (uint16_t)(first + c0);
+    W.head_bin_sum[table] = __builtin_ldexp((double)(a0 >> 12), -kWeightBits - bin_shift(2 * lane));
+    W.head_bin_sum[table + 1] = __builtin_ldexp((double)(a1 >> 12), -kWeightBits - bin_shift(2 * lane + 1));
+    wave_lds_sync();
+#pragma unroll
+    for (int e = 0; e < S; ++e) {
+      const float v = value(e);
+      if (v >= sv) head[atomicAdd(&bin_at[bins.of(v)], 1u)] = composite(key_of(v), (uint32_t)(begin + local(e)));
+    }
+  };
+  auto from_list = [&](auto steps, int count, bool sums) {
+    constexpr int S = decltype(steps)::value;
+    uint64_t v[S];
+#pragma unroll
+    for (int e = 0; e < S; ++e) {
+      const int i = e * kWaveSize + lane;
+      v[e] = i < count ? list[i] : raw_entry(__builtin_nanf(""), 0u);
+    }
+    auto value = [&](int e) { return __uint_as_float((uint32_t)(v[e] >> 32)); };
+    if (sums) {
+      weigh_head(steps, value);
+#pragma unroll
+      for (int e = 0; e < S; ++e) stored += (int)__popcll(__ballot(value(e) >= sv));
+    }
+    store(steps, value, [&](int e) { return (int)~(uint32_t)v[e]; });
+  };
+  using Few = std::integral_constant<int, 2>;
+  using Listed = std::integral_constant<int, kHeadSparse / kWaveSize>;
+  using All = std::integral_constant<int, 2 * kWChunkPerLane>;
+  auto own = [&](int e) { return x[e]; };
+  if (in_head <= kHeadSparse) {
+    if (in_head <= 2 * kWaveSize) from_list(Few{}, in_head, true);
+    else from_list(Listed{}, in_head, true);
+  } else {
+    weigh_head(All{}, own);
+    wave_lds_sync();
+    stored = gather(sv);
+    if (stored <= 2 * kWaveSize) from_list(Few{}, stored, false);
+    else if (stored <= kHeadSparse) from_list(Listed{}, stored, false);
+    else store(All{}, own, local_of);
+  }
+  sum = wave_sum(sum);
+  if (lane == 0) {
+    const size_t at = (size_t)row * W.acc_stride + slice;
+    W.head_slice_count[2 * at] = (uint32_t)stored;
+    W.head_slice_count[2 * at + 1] = (uint32_t)in_head;
+    W.head_slice_sum[at] = sum;
   }
 }
 
-// For a row that head_fast_kernel cannot finish, the sorted head is built in two steps.
+// For a row that head_pick_kernel cannot finish, the sorted head is built in two steps.
 // plan_head (that kernel's workgroup for the row) bins the head by key into 4096 buckets
 // (bucket = (max_key - key) >> shift, so bucket order is descending key order), scatters it
 // into bucket order, and cuts the bucket sequence into segments: a new segment starts at each
@@ -3146,29 +3417,45 @@ constexpr int kHeadBatch = 4096;
 __host__ __device__ __forceinline__ int plan_slots(int vocab_max) { return vocab_max / kSegCap + 2; }
 
 constexpr int kPlanThreads = 1024;  // a 13 K-entry head took 24.5 us on 256 lanes
-static_assert(kMaxSplits * kChunk <= kPlanThreads * kHeadSlice, "head_fast_kernel takes one slice per thread");
+static_assert(kMaxSplits * kChunk <= kPlanThreads * kHeadSlice, "head_pick_kernel takes one slice per thread");
 
 struct PlanSmem {
-  uint32_t starts[kPlanThreads + 1];  // head offset of each head_kernel slice's entries
   uint32_t wave_total[kPlanThreads / kWaveSize];
+  uint32_t slot;
   uint32_t hist[kHeadBuckets];
   uint32_t start[kHeadBuckets];
 };
 
-// The plan of one row's sorted head, by a workgroup of kPlanThreads (head_fast_kernel).
+// The plan of one row's sorted head, by a workgroup of kPlanThreads (head_pick_kernel): its
+// entries read from the row again (head_kernel stores only those the selection may need).
+template <typename In>
 __device__ __forceinline__ void plan_head(PlanSmem &sm, const Launch &L, const Workspace &W, int row,
                                           const RowState &rs, uint32_t *plan) {
-  const int H = (int)sm.starts[L.h_splits];
-  const uint64_t *head_base = W.head + (size_t)row * W.head_stride;
-  // Entry i of the head: in the slice s with starts[s] <= i < starts[s + 1].
-  auto head_at = [&](int i) {
-    int lo = 0, hi = L.h_splits;
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (sm.starts[mid] <= (uint32_t)i) lo = mid; else hi = mid;
+  uint64_t *head_base = W.head + (size_t)row * W.head_stride;
+  const In *src = reinterpret_cast<const In *>(L.logits) + (size_t)row * L.vocab;
+  constexpr int B = 8;  // global loads in flight per lane
+  if (threadIdx.x == 0) sm.slot = 0u;
+  __syncthreads();
+  for (int base0 = 0; base0 < L.vocab; base0 += B * kPlanThreads) {
+    float v[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int i = base0 + u * kPlanThreads + (int)threadIdx.x;
+      v[u] = i < L.vocab ? load_one(src + i) : 0.0f;
     }
-    return head_base[(size_t)lo * L.h_slice_len + (uint32_t)i - sm.starts[lo]];
-  };
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int i = base0 + u * kPlanThreads + (int)threadIdx.x;
+      const bool take = i < L.vocab && v[u] >= value_of(rs.head_key);
+      const uint32_t at = wave_slot(take, &sm.slot);
+      if (take) head_base[at] = composite(key_of(v[u]), (uint32_t)i);
+    }
+  }
+  __threadfence_block();
+  __syncthreads();
+  const int H = (int)sm.slot;
+  if (threadIdx.x == 0) W.head_count[row] = (uint32_t)H;
+  auto head_at = [&](int i) { return head_base[i]; };
   uint64_t *sorted = W.head_sorted + (size_t)row * W.head_stride;
   const uint32_t kmax = key_of(rs.max);
   const uint32_t range = kmax - min(rs.head_key, kmax);
@@ -3179,7 +3466,6 @@ __device__ __forceinline__ void plan_head(PlanSmem &sm, const Launch &L, const W
   };
   for (int b = threadIdx.x; b < kHeadBuckets; b += kPlanThreads) sm.hist[b] = 0u;
   __syncthreads();
-  constexpr int B = 8;  // global loads in flight per lane
   for (int base0 = 0; base0 < H; base0 += B * kPlanThreads) {
     uint64_t v[B];
 #pragma unroll
@@ -3341,28 +3627,11 @@ __device__ __forceinline__ void sort_segment(SortSmem &sm, const Launch &L, cons
   terms(out);
 }
 
-// Workgroups per row of head_sort_kernel; each sorts every kSortGroups-th segment. (One per
-// segment slot cost 7.5 us on config 4 when no row needed a sort: 171 slots per row, each
-// workgroup reserving 66 KB of LDS.)
-constexpr int kSortGroups = 8;
+// Heads up to this many entries run their sums from LDS (padded, no more than the sort's
+// buffer); larger ones from global memory.
+constexpr int kHeadLds = 7168;
 
-__global__ __launch_bounds__(kBlock) void head_sort_kernel(Launch L, Workspace W) {
-  __shared__ SortSmem sm;
-  const int row = (int)blockIdx.x / kSortGroups;
-  const int first = (int)blockIdx.x - row * kSortGroups;
-  const uint32_t *plan = W.head_plan + (size_t)row * W.plan_stride;
-  const int slots = (int)plan[0];
-  for (int g = first; g < slots; g += kSortGroups) {
-    sort_segment(sm, L, W, row, g, slots, plan);
-    __syncthreads();  // sm is reused by the next segment
-  }
-}
-
-// Heads up to this many entries run their sums from LDS (padded, 139 KB of the 160 KB a
-// gfx950 workgroup may use); larger ones from global memory.
-constexpr int kHeadLds = 16384;
-
-constexpr int kFinishThreads = 512;  // eight waves: the sums take 8,192 terms per step
+constexpr int kFinishThreads = kBlock;  // four waves: the sums take 4,096 terms per step
 
 struct HeadSmem {
   BlockScratch bs;
@@ -3403,13 +3672,9 @@ __device__ __forceinline__ int wave_first_above(C c, int n, double target) {
 // sampleFromTopK over the sorted head (see the comment on head_kernel): the head's terms,
 // the scaled total and the running sums (bit-exact sequential sums), the cut and the draw.
 template <typename In>
-__global__ __launch_bounds__(kFinishThreads) void head_finish_kernel(Launch L, Workspace W) {
-  __shared__ HeadSmem sm;
-  const int row = (int)blockIdx.x;
+__device__ __forceinline__ void head_finish(HeadSmem &sm, const Launch &L, const Workspace &W, int row) {
   const tabby_row_params P = L.params[row];
-  if (!is_head_row(P, L)) return;
   const RowState rs = W.row_state[row];
-  if (rs.status != TABBY_OK || (rs.handoff & 1u)) return;  // head_fast_kernel finished it
   const int V = L.vocab;
   const In *row_src = reinterpret_cast<const In *>(L.logits) + (size_t)row * V;
   const int H = (int)W.head_count[row];
@@ -3460,7 +3725,7 @@ __global__ __launch_bounds__(kFinishThreads) void head_finish_kernel(Launch L, W
     const double stop = top_p < 1.0 ? top_p : INFINITY;
     auto finish = [&](auto t, auto c) {
       // The weights are non-increasing: the sum may settle before the head's end. Both sums
-      // are taken by the whole workgroup (block_seq_sum_wide: 8,192 terms per step).
+      // are taken by the whole workgroup (block_seq_sum_wide).
       const double S = block_seq_sum_wide<kFinishThreads / kWaveSize>(t, H, c, false, INFINITY, true, sm.ss).total;
       for (int i = threadIdx.x; i < H; i += kFinishThreads) c[i] = t[i] / S;
       __syncthreads();
@@ -3516,145 +3781,481 @@ __global__ __launch_bounds__(kFinishThreads) void head_finish_kernel(Launch L, W
   }
 }
 
-// The fast finish of a whole-vocabulary row (see add_ulps above), by wave 0, with the top
-// list already in sm.top and this lane's share of head_kernel's counts (r, ties, outside):
-// true when the row is finished (result and top-k list written, RowState marked).
-struct HeadFastSmem {
-  uint64_t top[kWaveKcap];
-  double s[kWaveKcap];  // s_i = exp((l_i - M) / T) with V8's exp, then w_i = s_i / S
-  double c[kWaveKcap];  // running sums
-  int done;
+// Workgroups per row of head_sort_kernel; each sorts every kSortGroups-th segment. (One per
+// segment slot cost 7.5 us on 64 rows of 151,936 when no row needed a sort: 171 slots per row,
+// each workgroup reserving 66 KB of LDS.)
+constexpr int kSortGroups = 8;
+
+// The rows head_pick_kernel left (plan[0] > 0): the head's segments sorted, then the row's tail
+// by the last of its workgroups to arrive -- one launch, as in nearly every call no row is left
+// (each further launch, idle or not, costs the host about 3.6 us).
+union SortedSmem {
+  SortSmem sort;
+  HeadSmem finish;
 };
 
 template <typename In>
-__device__ __forceinline__ bool head_fast_finish(HeadFastSmem &sm, const Launch &L, const Workspace &W, int row,
-                                                 const tabby_row_params &P, const RowState &rs, int H, double r,
-                                                 double ties, double outside) {
-  const int N = (int)(rs.handoff >> 16);
-  if (N == 0 || N > kWaveKcap) return false;  // no list handed over (pools above 256)
-  const int V = L.vocab, lane = wave_lane();
-  const double M = (double)rs.max, S1 = rs.sum_exp, T = P.temperature, top_p = P.top_p;
-  int chosen = 0, cut = 1;
-  if (!greedy_temp(T)) {
-    for (int i = lane; i < N; i += kWaveSize)
-      sm.s[i] = fdlibm_exp(((double)value_of(composite_key(sm.top[i])) - M) / T);
-    const double PN = rs.list_sum;
-    // head_kernel's counts over the head entries below the top N.
-    r = wave_sum(r);
-    ties = wave_sum(ties);
-    outside = wave_sum(outside);
-    const double scale = ulp_scale(PN);
-    const double m = PN * scale;  // P_N in ulps: an integer in [2^52, 2^53)
-    if (ties > 0.0 || m + r >= 9007199254740992.0) return false;
-    const double S = (m + r) / scale;
-    for (int i = lane; i < N; i += kWaveSize) sm.s[i] = sm.s[i] / S;
-    wave_lds_sync();
-    const SeqSum run = wave_seq_sum(sm.s, N, sm.c, top_p < 1.0 ? top_p : INFINITY);
-    const bool reached = top_p < 1.0 && run.total >= top_p;
-    // Without the cut among the top N, the running sums must end there: nothing in the head
-    // beyond them (every smaller term is below half an ulp of every running sum).
-    if (!reached && outside > 0.0) return false;
-    wave_lds_sync();
-    chosen = wave_first_above(sm.c, run.count, P.uniform * run.total);
-    cut = reached ? run.count : V;
+__global__ __launch_bounds__(kBlock) void head_sort_kernel(Launch L, Workspace W) {
+  __shared__ __align__(16) unsigned char raw[sizeof(SortedSmem)];
+  __shared__ int last;
+  const int row = (int)blockIdx.x / kSortGroups;
+  const int first = (int)blockIdx.x - row * kSortGroups;
+  const uint32_t *plan = W.head_plan + (size_t)row * W.plan_stride;
+  const int slots = (int)plan[0];
+  if (slots == 0) return;  // the row is finished (or has no head): every workgroup of it ends here
+  SortSmem &sort = *reinterpret_cast<SortSmem *>(raw);
+  for (int g = first; g < slots; g += kSortGroups) {
+    sort_segment(sort, L, W, row, g, slots, plan);
+    __syncthreads();  // `sort` is reused by the next segment
   }
-  if (lane == 0) {
-    tabby_row_result res;
-    res.max_logit = rs.max;
-    res.sum_exp = S1;
-    // The pool is the whole row: poolMass = sum of exp(l_i - M) / sumExp over every element,
-    // 1 up to rounding (a sequential sum of n such terms is within n * 2^-53 of it).
-    res.pool_mass = 1.0;
-    res.status = TABBY_OK;
-    res.topk_count = min(H, L.topk_cap);
-    res.considered = (uint32_t)cut;
-    res.pool_exhausted = 0;  // poolMass 1 is never below top_p
-    res.id = (int32_t)composite_index(sm.top[chosen]);
-    res.probability = fdlibm_exp((double)value_of(composite_key(sm.top[chosen])) - M) / S1;
-    L.results[row] = res;
-    W.row_state[row].handoff = rs.handoff | 1u;
-  }
-  if (L.topk_cap > 0) {
-    // The caller's top-k list: the first topk_cap <= N entries (finish_pool).
-    const In *row_src = reinterpret_cast<const In *>(L.logits) + (size_t)row * V;
-    const int m = min(H, L.topk_cap);
-    for (int i = lane; i < m; i += kWaveSize) {
-      const uint32_t idx = composite_index(sm.top[i]);
-      L.topk_ids[(size_t)row * L.topk_cap + i] = (int32_t)idx;
-      L.topk_logits[(size_t)row * L.topk_cap + i] = load_one(row_src + min(idx, (uint32_t)(V - 1)));
-    }
-  }
-  return true;
+  // The workgroup's sorted entries, weights and sums are released with its arrival; the last to
+  // arrive has acquired every other's.
+  __syncthreads();
+  if (threadIdx.x == 0)
+    last = __hip_atomic_fetch_add(W.head_arrived + row, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+                   (uint32_t)(kSortGroups - 1)
+               ? 1
+               : 0;
+  __syncthreads();
+  if (last) head_finish<In>(*reinterpret_cast<HeadSmem *>(raw), L, W, row);
 }
 
-// One workgroup per whole-vocabulary row: the fast finish (wave 0), else the plan of the
-// sorted head for head_sort_kernel and head_finish_kernel.
+// ---------------------------------------------------------------------------------------
+// Finishing a whole-vocabulary row by selection (head_pick_kernel), without sorting its head.
+// sampleFromTopK needs two places in the sorted head: the cut, the first running sum to reach
+// top-p, and the draw, the first running sum above uniform * (the sum at the cut). Both are
+// searches for a partial sum of the weights in descending order, and need order only around
+// the place they find. The entries that can hold it (store_threshold) are binned by value, with
+// counts and weights: up to 4,096 of them here, held in the workgroup's registers throughout
+// (1,024 bins, LDS atomics), more by head_kernel's slices (128 bins; a search then reads its
+// bin's entries). A bin with more than 256 entries is refined over its range of composites,
+// 1,024-fold per pass, and one wave sorts and scans the at most 256 left.
+//
+// These sums are added in another order than the reference's and with exps within 8 ulp of
+// V8's, so their comparisons decide as the reference's only when they clear their threshold by
+// the errors of both, each rounding 2^-53 relative. The reference's running sum at place j,
+// c_j, carries n roundings of its scaled total (n the vocabulary) and j + 2 of its own. Here
+// the total carries fewer than 64 additions and the 2^-43 of exp_sum_term's terms, a partial
+// sum one addition for each entry of a bin, the 8 ulp of exp_nonpos's and the 2^-39 of a
+// table's, all of them an argument within 37.5 * 1.5 ulp (a product by 1/T). So the cut needs (n + 2 j + the place's bin +
+// kPickAdds) * 2^-53 on both sides: 2^-35.6 at 151,936 and a shallow cut, against gaps of about
+// 1e-6 between neighbouring sums. In the draw the scaled total cancels: the cut's place takes
+// the place of n. A row that does not clear them has its head sorted and summed bit for bit
+// (head_sort_kernel). poolMass is 1 (the pool is the whole row) within the n * 2^-53 of a
+// sequential sum.
+//
+// What bounds it: latency -- dependent rounds of loads, LDS atomics and barriers over a few
+// thousand entries of one row. Sorting the head took 983 us for 16 rows of 151,936 at T = 1,
+// top-p 0.95 (N(0, 2.5^2), cuts hundreds to thousands of entries deep) and 1,235 us for 64; by
+// selection the calls take 42 and 55 us, and one row's 28 us against 346.
+// ---------------------------------------------------------------------------------------
+constexpr int kPickList = 4 * kWaveSize;  // entries one wave sorts
+constexpr int kPickKept = 4;              // stored entries per thread kept in registers
+constexpr int kPickFew = kPickKept * kPlanThreads;
+constexpr int kPickAdds = 4096 + (1 << 14);  // 2^-39: head_kernel's fixed-point weights
+constexpr int kPlanWaves = kPlanThreads / kWaveSize;
+static_assert(kPickBins == kPlanThreads, "one bin per thread");
+
+struct PickSmem {
+  double cum[kPickBins + 1];    // weight of the bins before
+  uint32_t cumn[kPickBins + 1]; // their entries
+  double sub[kPlanThreads];     // a pass's weights and counts by (sub-)bin
+  uint32_t subn[kPlanThreads];
+  uint32_t dst[kPlanThreads + 1], off[kPlanThreads];  // stored entries by head slice
+  uint32_t wave_n[kPlanWaves], wave_h[kPlanWaves], wave_c[kPlanWaves];
+  double wave_s[kPlanWaves];
+  uint64_t list[kPickList];
+  uint64_t top[kWaveKcap];  // the merge's sorted list
+  int first;
+  uint32_t slot;
+  double before, through;
+  uint64_t entry;
+  uint32_t rank, count;
+  int ok;
+};
+
+// A row's stored entries as the workgroup reads them: entry i lies in the slice s with
+// dst[s] <= i < dst[s + 1], off[s] into what the slice stored.
+struct Stored {
+  const uint64_t *head;
+  const uint32_t *dst, *off;
+  int slices, slice_len;
+  uint32_t total;
+  bool kept;  // up to kPickFew entries stay in registers
+  uint64_t own[kPickKept];
+  __device__ __forceinline__ uint64_t at(uint32_t i) const {
+    int lo = 0, hi = slices;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (dst[mid] <= i) lo = mid; else hi = mid;
+    }
+    return head[(size_t)lo * slice_len + off[lo] + (i - dst[lo])];
+  }
+  // Slice threadIdx.x's `n` entries from `from` (0 past the last slice). All threads.
+  template <class Smem>
+  __device__ __forceinline__ void load(Smem &sm, uint32_t n, uint32_t from) {
+    const int lane = wave_lane(), w = wave_id();
+    const uint32_t incl = wave_inclusive_scan_u32(n);
+    __syncthreads();
+    if (lane == kWaveSize - 1) sm.wave_n[w] = incl;
+    __syncthreads();
+    uint32_t base = 0u;
+    total = 0u;
+    for (int k = 0; k < kPlanThreads / kWaveSize; ++k) {
+      base += k < w ? sm.wave_n[k] : 0u;
+      total += sm.wave_n[k];
+    }
+    sm.dst[threadIdx.x] = base + incl - n;
+    sm.off[threadIdx.x] = from;
+    if (threadIdx.x == 0) sm.dst[kPlanThreads] = total;
+    dst = sm.dst;
+    off = sm.off;
+    __syncthreads();
+    kept = total <= (uint32_t)kPickFew;
+#pragma unroll
+    for (int u = 0; u < kPickKept; ++u) {
+      const uint32_t i = threadIdx.x + (uint32_t)(u * kPlanThreads);
+      own[u] = kept && i < total ? at(i) : 0ull;
+    }
+  }
+  // f(entry) for every entry, and f(0) in the places past the last, all lanes together.
+  template <class F>
+  __device__ __forceinline__ void each(F f) const {
+    if (kept) {
+#pragma unroll
+      for (int u = 0; u < kPickKept; ++u)
+        if ((uint32_t)(u * kPlanThreads) < total) f(own[u]);
+      return;
+    }
+    for (uint32_t base = 0; base < total; base += kPickFew) {
+      uint64_t v[kPickKept];
+#pragma unroll
+      for (int u = 0; u < kPickKept; ++u) {
+        const uint32_t i = base + threadIdx.x + (uint32_t)(u * kPlanThreads);
+        v[u] = i < total ? at(i) : 0ull;
+      }
+#pragma unroll
+      for (int u = 0; u < kPickKept; ++u) f(v[u]);
+    }
+  }
+};
+
+struct Picked {
+  bool ok;
+  uint64_t entry;  // the first entry, in descending order, whose partial sum reaches the target
+  double through;  // that partial sum
+  uint32_t rank;   // entries before it
+};
+
+// Inclusive prefix sums of sub and subn over the workgroup (thread t's: bins 0..t).
+__device__ __forceinline__ void scan_bins(PickSmem &sm, double &weight, uint32_t &entries) {
+  const int lane = wave_lane(), w = wave_id();
+  const double s = wave_inclusive_scan(sm.sub[threadIdx.x]);
+  const uint32_t c = wave_inclusive_scan_u32(sm.subn[threadIdx.x]);
+  if (lane == kWaveSize - 1) {
+    sm.wave_s[w] = s;
+    sm.wave_n[w] = c;
+  }
+  __syncthreads();
+  const double totals = wave_inclusive_scan(lane < kPlanWaves ? sm.wave_s[lane] : 0.0);
+  const uint32_t counts = wave_inclusive_scan_u32(lane < kPlanWaves ? sm.wave_n[lane] : 0u);
+  weight = (w > 0 ? lane_f64(totals, w - 1) : 0.0) + s;
+  entries = (w > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)counts, w - 1) : 0u) + c;
+}
+
+// The search, by the row's whole workgroup, sm.cum and sm.cumn holding the bins' prefix sums
+// (those of kTableBins bins repeated past them). bin_entries(bin): `stored` now holds that bin's
+// entries (and may hold others).
+template <class BinEntries>
+__device__ __forceinline__ Picked pick_entry(PickSmem &sm, const Stored &stored, const PickBin &pb, const RowState &rs,
+                                             double T, double target, double adds, BinEntries bin_entries_of) {
+  const int lane = wave_lane(), w = wave_id(), tid = (int)threadIdx.x;
+  const double M = (double)rs.max, inv_t = 1.0 / T;
+  auto weight = [&](uint64_t v) { return exp_nonpos(((double)value_of(composite_key(v)) - M) * inv_t); };
+  const Picked none{false, 0ull, 0.0, 0u};
+  __syncthreads();  // the previous search's reads are done
+  if (tid == 0) {
+    sm.first = kPlanThreads;
+    sm.slot = 0u;
+  }
+  __syncthreads();
+  const uint64_t reached = __ballot(sm.cumn[tid + 1] > sm.cumn[tid] && sm.cum[tid + 1] >= target);
+  if (reached && lane == __ffsll((unsigned long long)reached) - 1) atomicMin(&sm.first, tid);
+  __syncthreads();
+  const int bin = sm.first;
+  if (bin == kPlanThreads) return none;
+  bin_entries_of(bin);
+  double before = sm.cum[bin];
+  uint32_t rank = sm.cumn[bin], count = sm.cumn[bin + 1] - rank;
+  const uint32_t bin_entries = count;
+  // The candidates are the bin's entries in [lo, hi]; sub-bins divide [rlo, rhi] (entries above
+  // rhi go to the first, below rlo to the last).
+  uint64_t lo = (uint64_t)rs.store_key << 32, hi = ((uint64_t)key_of(rs.max) << 32) | 0xffffffffull;
+  auto candidate = [&](uint64_t v) {
+    return v >= lo && v <= hi && pb.of(value_of(composite_key(v))) == bin;  // 0 lies below lo
+  };
+  const float vhi = fmaxf(rs.max - (float)bin / pb.scale, -3.0e38f);
+  const float vlo = fmaxf(rs.max - (float)(bin + 1) / pb.scale, -3.0e38f);
+  uint64_t rhi = tmin(hi, ((uint64_t)key_of(vhi) << 32) | (uint64_t)0xffffffffu);
+  uint64_t rlo = tmin(rhi, tmax(lo, (uint64_t)key_of(vlo) << 32));
+  for (int pass = 0; count > (uint32_t)kPickList; ++pass) {
+    if (pass == 8) return none;
+    const int bits = rhi == rlo ? 1 : 64 - __clzll((long long)(rhi - rlo));
+    const int shift = bits > 10 ? bits - 10 : 0;
+    __syncthreads();  // sm.first has been read
+    sm.sub[tid] = 0.0;
+    sm.subn[tid] = 0u;
+    if (tid == 0) sm.first = kPlanThreads;
+    __syncthreads();
+    stored.each([&](uint64_t v) {
+      if (candidate(v)) {
+        const int q = v >= rhi ? 0 : (int)tmin((rhi - v) >> shift, (uint64_t)(kPlanThreads - 1));
+        lds_add(&sm.sub[q], weight(v));
+        atomicAdd(&sm.subn[q], 1u);
+      }
+    });
+    __syncthreads();
+    double s_incl;
+    uint32_t c_incl;
+    scan_bins(sm, s_incl, c_incl);
+    const uint64_t hit = __ballot(sm.subn[tid] > 0u && before + s_incl >= target);
+    if (hit && lane == __ffsll((unsigned long long)hit) - 1) atomicMin(&sm.first, tid);
+    __syncthreads();
+    const int f = sm.first;
+    if (f == kPlanThreads) return none;
+    if (tid == f) {
+      sm.before = before + (s_incl - sm.sub[tid]);
+      sm.rank = rank + c_incl - sm.subn[tid];
+      sm.count = sm.subn[tid];
+    }
+    __syncthreads();
+    before = sm.before;
+    rank = sm.rank;
+    count = sm.count;
+    const uint64_t below = (uint64_t)(f + 1) << shift;
+    if (f > 0) hi = tmin(hi, rhi - ((uint64_t)f << shift));
+    if (f < kPlanThreads - 1 && below <= rhi) lo = tmax(lo, rhi - below + (uint64_t)1);
+    rhi = hi;
+    rlo = lo;
+  }
+  stored.each([&](uint64_t v) {
+    const bool take = candidate(v);
+    const uint32_t at = wave_slot(take, &sm.slot);
+    if (take && at < (uint32_t)kPickList) sm.list[at] = v;
+  });
+  __syncthreads();
+  if (w == 0) {
+    const int m = (int)min(sm.slot, (uint32_t)kPickList);
+    auto settle = [&](auto regs) {
+      constexpr int R = decltype(regs)::value;
+      uint64_t v[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = r * kWaveSize + lane < m ? sm.list[r * kWaveSize + lane] : 0ull;
+      wave_sort_desc<R>(v);
+      double carry = before;
+      bool found = false;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const bool in = r * kWaveSize + lane < m;
+        const double s = in ? weight(v[r]) : 0.0;
+        const double through = carry + wave_inclusive_scan(s);
+        const uint64_t hit = __ballot(in && through >= target);
+        if (!found && hit) {
+          found = true;
+          const int j = __ffsll((unsigned long long)hit) - 1;
+          const uint32_t place = rank + (uint32_t)(r * kWaveSize + j);
+          if (lane == j) {
+            // Both neighbours of the place clear the target.
+            const double rel = (adds + 2.0 * (double)place + (double)bin_entries + (double)kPickAdds) * 0x1p-53;
+            const bool ok = through > target + rel * through && (place == 0u || through - s < target - rel * through);
+            sm.entry = v[r];
+            sm.through = through;
+            sm.rank = place;
+            sm.ok = ok ? 1 : 0;
+          }
+        }
+        carry = lane_f64(through, kWaveSize - 1);
+      }
+      if (!found && lane == 0) sm.ok = 0;
+    };
+    if (m <= kWaveSize) settle(std::integral_constant<int, 1>{});
+    else settle(std::integral_constant<int, kPickList / kWaveSize>{});
+  }
+  __syncthreads();
+  return Picked{sm.ok != 0, sm.entry, sm.through, sm.rank};
+}
+
+// The row's drawn entry and consideredCount, when the merge's list or the selection decides
+// them; every thread of the workgroup returns the same. `slice_n`: what head slice threadIdx.x
+// stored (0 past the last), `stored_all` their total; H, S: the head's size and weight.
+__device__ __forceinline__ bool head_pick(PickSmem &sm, const Launch &L, const Workspace &W, int row,
+                                          uint32_t slice_n, uint32_t stored_all, const tabby_row_params &P,
+                                          const RowState &rs, int N, int H, double S, uint64_t &entry, uint32_t &considered) {
+  const double T = P.temperature, top_p = P.top_p;
+  const int lane = wave_lane(), tid = (int)threadIdx.x;
+  if (head_by_list(sm.top, N, rs.max, P, S, ((double)L.vocab + (double)kPickAdds) * 0x1p-53, entry, considered))
+    return true;  // every wave alike
+  if (H <= min(N, kWaveSize)) {
+    // The list is the whole head: the reference's sums bit for bit (as reg_tail takes them).
+    const bool in = lane < H;
+    const uint64_t v = in ? sm.top[lane] : 0ull;
+    const double se = in ? fdlibm_exp(((double)value_of(composite_key(v)) - (double)rs.max) / T) : 0.0;
+    double running;
+    const double S_seq = reg_seq_sum(se, H, INFINITY, &running).total;
+    const SeqSum run = reg_seq_sum(in ? se / S_seq : 0.0, H, top_p < 1.0 ? top_p : INFINITY, &running);
+    const uint64_t hit = __ballot(lane < run.count && P.uniform * run.total < running);
+    entry = sm.top[hit ? __ffsll((unsigned long long)hit) - 1 : run.count - 1];
+    considered = top_p < 1.0 && run.total >= top_p ? (uint32_t)run.count : (uint32_t)L.vocab;
+    return true;
+  }
+  const bool cuts = top_p < 1.0;
+  const double M = (double)rs.max, inv_t = 1.0 / T;
+  auto search = [&](const Stored &stored, const PickBin &pb, auto bin_entries_of) {
+    double total = S;
+    considered = (uint32_t)L.vocab;
+    if (cuts) {
+      const Picked c = pick_entry(sm, stored, pb, rs, T, top_p * S, (double)L.vocab, bin_entries_of);
+      if (!c.ok) return false;
+      total = c.through;
+      considered = c.rank + 1u;
+    }
+    const Picked d = pick_entry(sm, stored, pb, rs, T, P.uniform * total, (double)considered, bin_entries_of);
+    entry = d.entry;
+    return d.ok;
+  };
+  Stored stored;
+  stored.head = W.head + (size_t)row * W.head_stride;
+  stored.slices = L.h_splits;
+  stored.slice_len = L.h_slice_len;
+  sm.sub[tid] = 0.0;
+  sm.subn[tid] = 0u;
+  if (stored_all <= (uint32_t)kPickFew) {
+    // Every stored entry in registers, binned here.
+    const PickBin pb(rs, kPickBins);
+    stored.load(sm, slice_n, 0u);
+    stored.each([&](uint64_t v) {
+      if (v != 0ull) {
+        const float l = value_of(composite_key(v));
+        const int b = pb.of(l);
+        lds_add(&sm.sub[b], exp_nonpos(((double)l - M) * inv_t));
+        atomicAdd(&sm.subn[b], 1u);
+      }
+    });
+    __syncthreads();
+    scan_bins(sm, sm.cum[tid + 1], sm.cumn[tid + 1]);
+    if (tid == 0) {
+      sm.cum[0] = 0.0;
+      sm.cumn[0] = 0u;
+    }
+    return search(stored, pb, [](int) {});
+  }
+  // The bins from the slices' tables (thread (g, b) adds every eighth slice's bin b) and, for
+  // slices that stored too few for one, from their entries (a thread each).
+  const PickBin pb(rs, kTableBins);
+  const size_t tables = (size_t)row * W.acc_stride * kTableBins;
+  const bool tabled = slice_n > (uint32_t)kTableMin;
+  if (tid < kPlanThreads) sm.off[tid] = slice_n;
+  __syncthreads();
+  {
+    const int b = tid % kTableBins;
+    double weight = 0.0;
+    uint32_t entries = 0u;
+    for (int s = tid / kTableBins; s < L.h_splits; s += kPlanThreads / kTableBins) {
+      if (sm.off[s] <= (uint32_t)kTableMin) continue;
+      const size_t at = tables + (size_t)s * kTableBins + b;
+      weight += W.head_bin_sum[at];
+      entries += (b + 1 < kTableBins ? W.head_bin_start[at + 1] : sm.off[s]) - W.head_bin_start[at];
+    }
+    lds_add(&sm.sub[b], weight);
+    atomicAdd(&sm.subn[b], entries);
+  }
+  if (!tabled) {
+    const uint64_t *mine = stored.head + (size_t)tid * L.h_slice_len;
+    for (uint32_t i = 0; i < slice_n; ++i) {
+      const float l = value_of(composite_key(mine[i]));
+      lds_add(&sm.sub[pb.of(l)], exp_nonpos(((double)l - M) * inv_t));
+      atomicAdd(&sm.subn[pb.of(l)], 1u);
+    }
+  }
+  __syncthreads();
+  scan_bins(sm, sm.cum[tid + 1], sm.cumn[tid + 1]);
+  if (tid == 0) {
+    sm.cum[0] = 0.0;
+    sm.cumn[0] = 0u;
+  }
+  return search(stored, pb, [&](int bin) {
+    uint32_t from = 0u, n = slice_n;
+    if (tabled) {
+      const uint16_t *start = W.head_bin_start + tables + (size_t)tid * kTableBins;
+      from = start[bin];
+      n = (bin + 1 < kTableBins ? start[bin + 1] : slice_n) - from;
+    }
+    stored.load(sm, n, from);
+  });
+}
+
+// One workgroup per whole-vocabulary row: the selection, else the plan of the sorted head for
+// head_sort_kernel.
 template <typename In>
-__global__ __launch_bounds__(kPlanThreads) void head_fast_kernel(Launch L, Workspace W) {
+__global__ __launch_bounds__(kPlanThreads) void head_pick_kernel(Launch L, Workspace W) {
   __shared__ PlanSmem psm;
-  __shared__ HeadFastSmem sm;
-  const int row = (int)blockIdx.x;
+  __shared__ PickSmem sm;
+  const int row = (int)blockIdx.x, tid = (int)threadIdx.x, lane = wave_lane();
   uint32_t *plan = W.head_plan + (size_t)row * W.plan_stride;
   const tabby_row_params P = L.params[row];
   const RowState rs = W.row_state[row];
-  // Every slice's head count is requested with them (one slice per thread), and so are, by
-  // wave 0, the fast finish's inputs: the merge's top list (its first kWaveKcap slots, of
-  // which the row state then says how many hold it) and head_kernel's ulp counts, slice by
-  // slice -- one round trip for all.
-  const int ns = L.h_splits;
-  const uint32_t c = (int)threadIdx.x < ns ? W.head_slice_count[(size_t)row * W.acc_stride + threadIdx.x] : 0u;
-  constexpr int kTopRegs = kWaveKcap / kWaveSize;
-  uint64_t top[kTopRegs];
-  double r = 0.0, ties = 0.0, outside = 0.0;
-  if (wave_id() == 0) {
-    const uint64_t *list = W.head_sorted + (size_t)row * W.head_stride;
-#pragma unroll
-    for (int q = 0; q < kTopRegs; ++q) {
-      const int i = q * kWaveSize + wave_lane();
-      top[q] = i < W.head_stride ? list[i] : 0ull;
-    }
-    const double *acc = W.head_acc + (size_t)row * W.acc_stride * 3;
-    for (int i = wave_lane(); i < ns; i += kWaveSize) {
-      r += acc[3 * i];
-      ties += acc[3 * i + 1];
-      outside += acc[3 * i + 2];
-    }
-  }
-  if (!is_head_row(P, L) || rs.status != TABBY_OK) {
-    if (threadIdx.x == 0) plan[0] = 0u;
+  // Requested with them: every head slice's counts and weight (one slice per thread) and the
+  // merge's top list (its first kWaveKcap slots, of which the row state then says how many hold
+  // it).
+  const size_t slices = (size_t)row * W.acc_stride;
+  const bool slice = tid < L.h_splits;
+  const uint32_t c = slice ? W.head_slice_count[2 * (slices + tid)] : 0u;
+  const uint32_t c_head = slice ? W.head_slice_count[2 * (slices + tid) + 1] : 0u;
+  const double slice_sum = slice ? W.head_slice_sum[slices + tid] : 0.0;
+  const uint64_t listed = tid < kWaveKcap && tid < W.head_stride ? W.head_sorted[(size_t)row * W.head_stride + tid] : 0ull;
+  if (!is_head_row(P, L) || rs.status != TABBY_OK || (rs.handoff & 1u)) {
+    if (tid == 0) plan[0] = 0u;
     return;
   }
   const int N = (int)(rs.handoff >> 16);
-  if (wave_id() == 0) {
-    if (N > 0 && N <= kWaveKcap) {
-#pragma unroll
-      for (int q = 0; q < kTopRegs; ++q) {
-        const int i = q * kWaveSize + wave_lane();
-        if (i < N) sm.top[i] = top[q];
-      }
+  const bool has_list = N > 0 && N <= kWaveKcap;
+  if (has_list && tid < N) sm.top[tid] = listed;
+  // The head's size and weight.
+  const uint32_t h_incl = wave_inclusive_scan_u32(c_head), c_incl = wave_inclusive_scan_u32(c);
+  const double s_wave = wave_sum(slice_sum);
+  if (lane == kWaveSize - 1) {
+    sm.wave_h[wave_id()] = h_incl;
+    sm.wave_c[wave_id()] = c_incl;
+    sm.wave_s[wave_id()] = s_wave;
+  }
+  __syncthreads();
+  uint32_t H = 0u, C = 0u;
+  double S = 0.0;
+  for (int k = 0; k < kPlanWaves; ++k) {
+    H += sm.wave_h[k];
+    C += sm.wave_c[k];
+    S += sm.wave_s[k];
+  }
+  uint64_t entry = 0ull;
+  uint32_t considered = 0u;
+  if (has_list && head_pick(sm, L, W, row, c, C, P, rs, N, (int)H, S, entry, considered)) {
+    if (tid == 0) {
+      write_head_result(L, row, rs.max, rs.sum_exp, min(L.vocab, L.topk_cap), entry, considered);
+      W.row_state[row].handoff = rs.handoff | 1u;
+      plan[0] = 0u;
     }
-    if (!(N > 0 && N <= kWaveKcap) || greedy_temp(P.temperature)) r = ties = outside = 0.0;
-  }
-  // The head's size and where each slice's entries start (every thread holds one slice).
-  const uint32_t inc = wave_inclusive_scan_u32(c);
-  if (wave_lane() == kWaveSize - 1) psm.wave_total[wave_id()] = inc;
-  __syncthreads();
-  uint32_t below = inc;
-  for (int k = 0; k < wave_id(); ++k) below += psm.wave_total[k];
-  if ((int)threadIdx.x < ns) psm.starts[threadIdx.x + 1] = below;
-  if (threadIdx.x == 0) psm.starts[0] = 0u;
-  __syncthreads();
-  if (threadIdx.x == 0) W.head_count[row] = psm.starts[ns];
-  if (wave_id() == 0) {
-    const bool done = head_fast_finish<In>(sm, L, W, row, P, rs, (int)psm.starts[ns], r, ties, outside);
-    if (wave_lane() == 0) sm.done = done ? 1 : 0;
-  }
-  __syncthreads();
-  if (sm.done) {
-    if (threadIdx.x == 0) plan[0] = 0u;
+    // The caller's top-k list: the first topk_cap <= N entries (finish_pool).
+    const In *row_src = reinterpret_cast<const In *>(L.logits) + (size_t)row * L.vocab;
+    if (tid < min(L.topk_cap, N)) {
+      const uint32_t idx = composite_index(sm.top[tid]);
+      L.topk_ids[(size_t)row * L.topk_cap + tid] = (int32_t)idx;
+      L.topk_logits[(size_t)row * L.topk_cap + tid] = load_one(row_src + min(idx, (uint32_t)(L.vocab - 1)));
+    }
     return;
   }
-  plan_head(psm, L, W, row, rs, plan);
+  if (tid == 0) W.head_arrived[row] = 0u;
+  __syncthreads();
+  plan_head<In>(psm, L, W, row, rs, plan);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -3676,7 +4277,7 @@ __global__ __launch_bounds__(kWaveSize) void seq_sum_kernel(const double *t, int
   if (wave_lane() == 0) *count = r.count;
 }
 
-// The same by a workgroup of NW waves (block_seq_sum_wide; head_finish_kernel runs NW = 8).
+// The same by a workgroup of NW waves (block_seq_sum_wide; head_sort_kernel runs NW = 4).
 template <int NW>
 __global__ __launch_bounds__(NW * kWaveSize) void seq_sum_block_kernel(const double *t, int32_t n, double stop_at,
                                                                        double *out, int32_t *count) {
@@ -3685,7 +4286,7 @@ __global__ __launch_bounds__(NW * kWaveSize) void seq_sum_block_kernel(const dou
   if (threadIdx.x == 0) *count = r.count;
 }
 
-// Diagnostic kernel: the draw search of head_finish_kernel (wave_first_above), one wave per
+// Diagnostic kernel: the draw search of head_sort_kernel (wave_first_above), one wave per
 // target, over the non-decreasing c[0..n).
 __global__ __launch_bounds__(kWaveSize) void first_above_kernel(const double *c, int32_t n, const double *targets,
                                                                 int32_t *out) {
@@ -4474,17 +5075,23 @@ int row_parts(int rows, int vocab, int cus, int &part_len) {
   return (vocab + part_len - 1) / part_len;
 }
 
+template <typename In, int VEC, bool HEAD>
+void launch_first(const Launch &L, const Workspace &W, hipStream_t stream) {
+  const dim3 slices((unsigned)(L.rows * L.splits)), rows((unsigned)L.rows);
+  if (L.parts >= 1)
+    hipLaunchKernelGGL((row_kernel<In, VEC, HEAD>), L.parts == 1 ? rows : slices,
+                       dim3((unsigned)(L.row_waves * kWaveSize)), 0, stream, L, W);
+  else
+    hipLaunchKernelGGL((wave_kernel<In, VEC, HEAD>), slices, dim3(kWaveSize), 0, stream, L, W);
+  if (L.parts != 1) hipLaunchKernelGGL((wave_merge_kernel<In, HEAD>), rows, dim3(kBlock), 0, stream, L, W);
+}
+
 template <typename In, int VEC>
 hipError_t launch_pair(const Launch &L, const Workspace &W, int cus, hipStream_t stream) {
   const dim3 slices((unsigned)(L.rows * L.splits)), rows((unsigned)L.rows);
-  if (L.parts == 1) {
-    hipLaunchKernelGGL((row_kernel<In, VEC>), rows, dim3((unsigned)(L.row_waves * kWaveSize)), 0, stream, L, W);
-  } else if (L.parts > 1) {
-    hipLaunchKernelGGL((row_kernel<In, VEC>), slices, dim3((unsigned)(L.row_waves * kWaveSize)), 0, stream, L, W);
-    hipLaunchKernelGGL((wave_merge_kernel<In>), rows, dim3(kBlock), 0, stream, L, W);
-  } else if (L.kcap <= kWaveKcap) {
-    hipLaunchKernelGGL((wave_kernel<In, VEC>), slices, dim3(kWaveSize), 0, stream, L, W);
-    hipLaunchKernelGGL((wave_merge_kernel<In>), rows, dim3(kBlock), 0, stream, L, W);
+  if (L.kcap <= kWaveKcap) {
+    if (L.head_pass) launch_first<In, VEC, true>(L, W, stream);
+    else launch_first<In, VEC, false>(L, W, stream);
   } else if (L.pool_rows) {
     // pool_row_kernel ends every row but a head pass's whole-vocabulary ones, which
     // merge_kernel hands to the head kernels.
@@ -4502,9 +5109,8 @@ template <typename In, int VEC>
 hipError_t launch_head(const Launch &L, const Workspace &W, hipStream_t stream) {
   hipLaunchKernelGGL((head_kernel<In, VEC>), dim3((unsigned)(L.rows * L.h_splits)), dim3(kWaveSize), 0,
                      stream, L, W);
-  hipLaunchKernelGGL((head_fast_kernel<In>), dim3((unsigned)L.rows), dim3(kPlanThreads), 0, stream, L, W);
-  hipLaunchKernelGGL(head_sort_kernel, dim3((unsigned)(L.rows * kSortGroups)), dim3(kBlock), 0, stream, L, W);
-  hipLaunchKernelGGL((head_finish_kernel<In>), dim3((unsigned)L.rows), dim3(kFinishThreads), 0, stream, L, W);
+  hipLaunchKernelGGL((head_pick_kernel<In>), dim3((unsigned)L.rows), dim3(kPlanThreads), 0, stream, L, W);
+  hipLaunchKernelGGL((head_sort_kernel<In>), dim3((unsigned)(L.rows * kSortGroups)), dim3(kBlock), 0, stream, L, W);
   return hipGetLastError();
 }
 
@@ -4739,13 +5345,18 @@ int tabby_sampler_sample_device(tabby_sampler *h, const void *logits_dev, int32_
       const size_t plan_bytes = ((size_t)rows * plan_stride * 4 + 255) & ~(size_t)255;
       const size_t part_bytes = ((size_t)rows * (plan_stride - 2) * 16 + 255) & ~(size_t)255;
       const int acc_stride = (h->vocab_max + kHeadSlice - 1) / kHeadSlice;
-      const size_t acc_bytes = (size_t)rows * acc_stride * 24;
-      HIP_TRY(hipMalloc(&h->head_base, per * 32 + plan_bytes + part_bytes + acc_bytes + (size_t)rows * acc_stride * 4));
+      const size_t slices = (size_t)rows * acc_stride, bins = slices * kTableBins;
+      HIP_TRY(hipMalloc(&h->head_base, per * 32 + plan_bytes + part_bytes + bins * 10 + slices * 16 +
+                                           (size_t)rows * (kMaxSplits * 8 + 4)));
       char *b = (char *)h->head_base;
       h->ws.head_plan = (uint32_t *)(b + per * 32);
       h->ws.head_part = (double *)(b + per * 32 + plan_bytes);
-      h->ws.head_acc = (double *)(b + per * 32 + plan_bytes + part_bytes);
-      h->ws.head_slice_count = (uint32_t *)(b + per * 32 + plan_bytes + part_bytes + acc_bytes);
+      h->ws.head_bin_sum = (double *)(b + per * 32 + plan_bytes + part_bytes);
+      h->ws.head_slice_sum = h->ws.head_bin_sum + bins;
+      h->ws.scaled = h->ws.head_slice_sum + slices;
+      h->ws.head_slice_count = (uint32_t *)(h->ws.scaled + (size_t)rows * kMaxSplits);
+      h->ws.head_arrived = h->ws.head_slice_count + 2 * slices;
+      h->ws.head_bin_start = (uint16_t *)(h->ws.head_arrived + rows);
       h->ws.plan_stride = plan_stride;
       h->ws.acc_stride = acc_stride;
       h->ws.head = (uint64_t *)b;

@@ -562,6 +562,56 @@ def test_full_vocab_fast_finish_edges(oracle, dtype, topk_cap, k_max):
          compare(w, res, ids, vals, run_oracle(oracle, w, topk_cap), topk_cap))
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("vocab,k_max,topk_cap", [(2049, 64, 5), (40000, 64, 0), (40001, 1024, 3), (151936, 64, 0)])
+def test_full_vocab_selection(oracle, dtype, vocab, k_max, topk_cap):
+    # Whole-vocabulary rows finished by selection: cuts thousands of entries deep (the slices'
+    # tables), flat rows (slices that store from registers), tie groups of thousands (refined by
+    # index), draws without a cut, u = 0 and u near 1, masked rows of 20 equal entries whose sums
+    # meet top-p exactly (summed bit for bit from the list), equal rows at an exact boundary and
+    # draws placed on it (the sorted head), a large offset, and a cold row among them.
+    rows = 24
+    w = synth.random_workload(rows=rows, vocab=vocab, seed=77 + vocab, k_choices=(0,), temperatures=(1.0,),
+                              top_ps=(0.95,), sigma=2.5)
+    rng = np.random.default_rng(vocab + k_max)
+    for r in range(rows):
+        kind = r % 12
+        if kind == 1:
+            w.logits[r] = rng.normal(0, 0.2, vocab).astype(np.float32)
+            w.temperature[r], w.top_p[r] = 1.5, 0.9
+        elif kind == 2:
+            w.logits[r] = np.round(rng.normal(0, 2, vocab) * 2) * 0.5
+            w.top_p[r] = 0.8 if r < 12 else 0.35
+        elif kind == 3:
+            w.logits[r] = 1.25
+            w.top_p[r], w.uniform[r] = (0.5, 0.25) if r < 12 else (0.75, 0.9)
+        elif kind == 4:
+            w.logits[r] = -np.inf
+            w.logits[r, rng.choice(vocab, 20, replace=False)] = 3.0
+            w.top_p[r], w.uniform[r] = (0.5, 0.3) if r < 12 else (0.95, 0.5)
+        elif kind == 5:
+            w.top_p[r], w.uniform[r] = (1.0, 0.999) if r < 12 else (2.0, 1.0 - 2.0 ** -32)
+        elif kind == 6:
+            w.top_p[r], w.uniform[r] = 0.99, 0.0
+        elif kind == 7:
+            w.temperature[r] = 0.05
+        elif kind == 8:
+            w.logits[r] += 500.0
+            w.top_p[r] = 0.999
+        elif kind == 9:
+            w.temperature[r], w.top_p[r] = 50.0, 0.6
+        elif kind == 10:
+            w.logits[r, rng.choice(vocab, vocab // 2, replace=False)] = -np.inf
+            w.temperature[r], w.top_p[r] = 0.7, 0.9
+        elif kind == 11:
+            w.temperature[r] = 0.0
+    w.logits = w.logits.astype(dtype)
+    print(f"selection vocab={vocab} k_max={k_max} {dtype.__name__}", flush=True)
+    res, ids, vals = run_gpu(w, k_max=k_max, topk_cap=topk_cap)
+    _log(f"full vocab selection {vocab} {dtype.__name__} k_max={k_max}",
+         compare(w, res, ids, vals, run_oracle(oracle, w, topk_cap), topk_cap))
+
+
 def test_full_vocab_rejects_list_above_k_max():
     import torch
     x = torch.zeros(1, 5000, device="cuda")
