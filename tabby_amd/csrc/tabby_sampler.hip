@@ -1141,10 +1141,13 @@ __device__ __forceinline__ Pruned wave_prune_any(WaveSmem &sm, int count, int kk
 
 // Registers per lane (1, 2, 4 or 8) for the union of the row's published lane-maximum keys:
 // each of `waves` waves publishes m = min(64, 64 * regs / waves) keys, and the union must hold
-// at least kk of them (kk <= 256 here; 8 always suffices for 5 to 16 waves).
-__device__ __forceinline__ int bound_regs(int kk, int waves) {
+// at least kk keys of the `live` waves that have a chunk (kk <= 256 here; 8 always suffices for 5
+// to 16 live waves). Counting the idle waves' keys too, a part of 11 chunks on 16 waves
+// published 44 keys for k = 50: no bound, every element a candidate (one row of 50,257 in four
+// parts 26.7 us a call; now 13.8).
+__device__ __forceinline__ int bound_regs(int kk, int waves, int live) {
   for (int r = 1; r < 8; r *= 2)
-    if (waves * min(kWaveSize, kWaveSize * r / waves) >= kk) return r;
+    if (live * min(kWaveSize, kWaveSize * r / waves) >= kk) return r;
   return 8;
 }
 
@@ -1359,7 +1362,7 @@ __device__ __forceinline__ void wave_slice(WaveSmem &sm, const Launch &L, const 
     // one wave's offer: the row's top lane maxima are spread over the waves.) Every wave
     // passes the barrier once and computes the same bound.
     if (kk > 0) {
-      const int regs = bound_regs(kk, waves);
+      const int regs = bound_regs(kk, waves, min(waves, nchunks));
       const int m = min(kWaveSize, kWaveSize * regs / waves);
       float cm = -INFINITY;
       if (a < nchunks) {

@@ -562,6 +562,17 @@ def test_full_vocab_fast_finish_edges(oracle, dtype, topk_cap, k_max):
          compare(w, res, ids, vals, run_oracle(oracle, w, topk_cap), topk_cap))
 
 
+@pytest.mark.parametrize("vocab", [32769, 50257, 65537, 151937])
+def test_parts_with_idle_waves(oracle, vocab):
+    # Rows cut into parts of 16,384 elements or fewer: the last part has fewer chunks than its
+    # workgroup has waves, so the row's first bound comes from the waves that have one.
+    w = synth.random_workload(rows=5, vocab=vocab, seed=vocab, k_choices=(1, 50, 64, 100, 256), ties=False,
+                              temperatures=(0.0, 0.7, 1.0), top_ps=(0.9, 1.0))
+    w.logits[1, -3000:] += 9.0  # the row's top in the short part
+    res, ids, vals = run_gpu(w, k_max=256, topk_cap=100)
+    compare(w, res, ids, vals, run_oracle(oracle, w, 100), 100)
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
 @pytest.mark.parametrize("vocab,k_max,topk_cap", [(2049, 64, 5), (40000, 64, 0), (40001, 1024, 3), (151936, 64, 0)])
 def test_full_vocab_selection(oracle, dtype, vocab, k_max, topk_cap):
