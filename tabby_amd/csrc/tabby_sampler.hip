@@ -2382,11 +2382,14 @@ __global__ __launch_bounds__(kBlock) void wave_merge_kernel(Launch L, Workspace 
 // is a chain of dependent LDS round trips before its merge.)
 // ---------------------------------------------------------------------------------------
 constexpr int kRowWaves = 16;
+constexpr int kRowHalfWaves = 8;
 constexpr int kRowMinWaves = kWaves + 1;  // four merge the lists, one the statistics
 
+template <int NW>
 struct RowSmem {
-  WaveSmem wave[kRowWaves];
-  SliceStat stats[kRowWaves];
+  static constexpr int kWavesMax = NW;
+  WaveSmem wave[NW];
+  SliceStat stats[NW];
   WaveMergeSmem merge;
   int next_chunk;
   uint32_t bound_keys[8 * kWaveSize];
@@ -2398,7 +2401,7 @@ struct RowSmem {
   uint32_t fin_mask;     // the waves finished streaming (the last one selects the take)
   uint32_t sel_take[2];  // the take's smallest key and its size
   uint32_t part_mask;    // the waves whose statistics the second-to-last one combined ...
-  double scaled[kRowWaves];  // each wave's sum of exp((x - max) / T) (whole-vocabulary rows)
+  double scaled[NW];  // each wave's sum of exp((x - max) / T) (whole-vocabulary rows)
   float part_max;        // ... their max
   double part_sum;       // ... and sum-exp against it
   uint32_t bound_key[2];  // the row's first bound and the largest key of its union
@@ -2856,14 +2859,17 @@ __global__ __launch_bounds__(kBlock) void lmhead_merge_kernel(Launch L, Workspac
 // its top K and statistics on to wave_merge_kernel. Returns false, with every wave's list
 // sorted in place and its count cut to K, when more than 64 entries would be taken (the
 // general merge then takes over). Every wave calls it.
-template <typename In, bool HEAD>
-__device__ __forceinline__ bool finish_small_pool(RowSmem &sm, const Launch &L, const Workspace &W, int row, int part,
+template <typename In, bool HEAD, class Smem>
+__device__ __forceinline__ bool finish_small_pool(Smem &sm, const Launch &L, const Workspace &W, int row, int part,
                                   const tabby_row_params &P, const RowPool &rp, int nw);
-__device__ __forceinline__ void small_pool_select(RowSmem &sm, int K);
+template <class Smem>
+__device__ __forceinline__ void small_pool_select(Smem &sm, int K);
 
-template <typename In, int VEC, bool HEAD>
-__global__ __launch_bounds__(kRowWaves * kWaveSize) void row_kernel(Launch L, Workspace W) {
-  __shared__ RowSmem sm;
+// NW: the most waves a workgroup may have. kRowWaves (one workgroup per CU: 98 KB of LDS) for up
+// to as many rows as CUs, and for parts; kRowHalfWaves (two per CU: 60 KB) for more rows.
+template <typename In, int VEC, bool HEAD, int NW>
+__global__ __launch_bounds__(NW * kWaveSize, 4) void row_kernel(Launch L, Workspace W) {
+  __shared__ RowSmem<NW> sm;
   int row = (int)blockIdx.x, part = 0;
   if (L.parts > 1) row_slice_of((int)blockIdx.x, L.rows, L.parts, row, part);
   const int w = __builtin_amdgcn_readfirstlane(wave_id());
@@ -2973,7 +2979,8 @@ __global__ __launch_bounds__(kRowWaves * kWaveSize) void row_kernel(Launch L, Wo
 // (every list entry when the union is small enough to take whole). One wave computes it --
 // the row's last to finish streaming, while the others wait at the barrier -- and leaves
 // both in sm.sel_take.
-__device__ __forceinline__ void small_pool_select(RowSmem &sm, int K) {
+template <class Smem>
+__device__ __forceinline__ void small_pool_select(Smem &sm, int K) {
   const int lane = wave_lane();
   const SelBins sb = sel_bins(sm.bound_key[1], sm.bound_key[0]);
   uint32_t h[4], sum = 0;
@@ -3016,8 +3023,8 @@ __device__ __forceinline__ void small_pool_select(RowSmem &sm, int K) {
   }
 }
 
-template <typename In, bool HEAD>
-__device__ __forceinline__ bool finish_small_pool(RowSmem &sm, const Launch &L, const Workspace &W, int row, int part,
+template <typename In, bool HEAD, class Smem>
+__device__ __forceinline__ bool finish_small_pool(Smem &sm, const Launch &L, const Workspace &W, int row, int part,
                                                   const tabby_row_params &P, const RowPool &rp, int nw) {
   const int w = wave_id(), lane = wave_lane();
   const int K = rp.K;
@@ -5081,8 +5088,11 @@ int row_parts(int rows, int vocab, int cus, int &part_len) {
 template <typename In, int VEC, bool HEAD>
 void launch_first(const Launch &L, const Workspace &W, hipStream_t stream) {
   const dim3 slices((unsigned)(L.rows * L.splits)), rows((unsigned)L.rows);
-  if (L.parts >= 1)
-    hipLaunchKernelGGL((row_kernel<In, VEC, HEAD>), L.parts == 1 ? rows : slices,
+  if (L.parts >= 1 && L.row_waves <= kRowHalfWaves)
+    hipLaunchKernelGGL((row_kernel<In, VEC, HEAD, kRowHalfWaves>), L.parts == 1 ? rows : slices,
+                       dim3((unsigned)(L.row_waves * kWaveSize)), 0, stream, L, W);
+  else if (L.parts >= 1)
+    hipLaunchKernelGGL((row_kernel<In, VEC, HEAD, kRowWaves>), L.parts == 1 ? rows : slices,
                        dim3((unsigned)(L.row_waves * kWaveSize)), 0, stream, L, W);
   else
     hipLaunchKernelGGL((wave_kernel<In, VEC, HEAD>), slices, dim3(kWaveSize), 0, stream, L, W);
@@ -5164,6 +5174,15 @@ Plan plan_launch(int rows, int vocab, int dtype, const void *logits, int k_max, 
     // 31.2 us (151,936 f32, k = 50), 200 rows at k = 100 50.6 -> 29.4 us.
     L.parts = 1;
     L.row_waves = kRowWaves;
+  } else if (L.kcap <= kWaveKcap && rows > cus) {
+    // More rows than CUs: two eight-wave workgroups share a CU, so that 512 rows run at once, the
+    // tail of one row beside the stream of the other, and a batch that is not a multiple of the
+    // CUs does not end in a round of its own. Against one workgroup of 8 to 16 waves per CU at a
+    // time (f32, k = 50): 300 rows of 151,936 47.9 -> 44.0 us, 391 50.9 -> 45.6, 512 58.7 -> 52.1
+    // (47.9 at a plain read's rate), 600 86.0 -> 70.0; 391 rows of 50,257 28.5 -> 20.8; 300 of
+    // 32,000 23.2 -> 15.6. 256 rows keep sixteen waves each: one row per CU needs them all.
+    L.parts = 1;
+    L.row_waves = kRowHalfWaves;
   } else if (per_row_launch(L, cus)) {
     L.parts = 1;
     L.row_waves = std::max(L.splits, kRowMinWaves);  // at least the five the merge uses

@@ -562,6 +562,19 @@ def test_full_vocab_fast_finish_edges(oracle, dtype, topk_cap, k_max):
          compare(w, res, ids, vals, run_oracle(oracle, w, topk_cap), topk_cap))
 
 
+@pytest.mark.parametrize("rows,vocab,dtype", [(257, 1, np.float32), (300, 5000, np.float16), (391, 20001, np.float32),
+                                              (513, 8192, np.float32), (700, 33000, np.float16)])
+def test_more_rows_than_cus(oracle, rows, vocab, dtype):
+    # Eight-wave workgroups, two to a CU: every pool size up to 256, ties, -inf, greedy and
+    # whole-vocabulary rows, lists.
+    w = synth.random_workload(rows=rows, vocab=vocab, seed=rows, k_choices=(0, 1, 7, 64, 65, 200, 256), ties=True,
+                              neg_inf_frac=0.2 if vocab > 1 else 0.0)
+    w.logits = w.logits.astype(dtype)
+    cap = min(vocab, 40)
+    res, ids, vals = run_gpu(w, k_max=256, topk_cap=cap)
+    compare(w, res, ids, vals, run_oracle(oracle, w, cap), cap)
+
+
 @pytest.mark.parametrize("vocab", [32769, 50257, 65537, 151937])
 def test_parts_with_idle_waves(oracle, vocab):
     # Rows cut into parts of 16,384 elements or fewer: the last part has fewer chunks than its
