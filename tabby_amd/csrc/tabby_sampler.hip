@@ -1723,8 +1723,9 @@ __global__ __launch_bounds__(kBlock) void merge_kernel(Launch L, Workspace W) {
       if (C >= need) {  // the candidates hold the row's top `need`: select the need-th largest
         const SelectResult r = staged ? radix_select(from_lds, (uint32_t)need, sm.u.hist, sm.bs)
                                       : radix_select(from_global, (uint32_t)need, sm.u.hist, sm.bs);
-        // Every selected composite is >= r.prefix, whose low bits below r.shift are zero.
-        list_key = (uint32_t)(r.prefix >> 32);
+        // Every selected composite is >= r.prefix, whose low bits below r.shift are zero: with -inf
+        // in the list its key can fall below -inf's, where no value lies.
+        list_key = max((uint32_t)(r.prefix >> 32), kNegInfKey);
       } else {
         list_key = kNegInfKey;  // fewer candidates than the list: take the whole row
       }
