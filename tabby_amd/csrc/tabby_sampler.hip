@@ -12,19 +12,17 @@
 // exchange through global memory. A batch of up to half as many rows as CUs runs row_kernel
 // on parts of each row (one workgroup per part) and merges the parts' lists with
 // wave_merge_kernel, or, where that would give two or three parts, one workgroup per row.
-// Other batches, and pools above 256, take two kernels:
-//   * wave_kernel (slice_kernel for pools above 256): grid = rows x splits; each wave
-//     (workgroup) owns one slice of one row and reads it from HBM exactly once with 16-byte
-//     nontemporal loads into registers. From registers it keeps the slice max, the slice sum
-//     of exp(x - max) (f32 terms, f64 accumulation), and a superset of the slice's top-k: every
-//     element at or above a bound that never exceeds the slice's k-th largest value, held in a
-//     wave-private LDS list (pruned by histogram when it fills) and written unsorted to the
-//     slice's candidate region. Waves of a row share the best bound any of them has proven.
-//   * merge_kernel: grid = rows; each 256-lane workgroup combines its row's slices: max,
-//     sum-exp (slice sums rescaled in f64, in slice order), an exact radix select over the
-//     64-bit (value key, ~index) composites -- the lower index wins ties, as in sampler.ts:28 --
-//     a sort, and sampleFromTopK's f64 tail in the reference's exact order of operations
-//     (sequential sums; V8's exp by the fdlibm method).
+// Other batches take two kernels:
+//   * wave_kernel: grid = rows x splits; each wave (workgroup) owns one slice of one row and
+//     reads it from HBM exactly once with 16-byte nontemporal loads into registers. From
+//     registers it keeps the slice max, the slice sum of exp(x - max) (f32 terms, f64
+//     accumulation), and a superset of the slice's top-k: every element at or above a bound that
+//     never exceeds the slice's k-th largest value, held in a wave-private LDS list (pruned by
+//     histogram when it fills), sorted at the end and written to the slice's candidate region.
+//   * wave_merge_kernel: grid = rows; each 256-lane workgroup combines its row's slices: max,
+//     sum-exp, the exact top-k over the 64-bit (value key, ~index) composites -- the lower index
+//     wins ties, as in sampler.ts:28 -- and sampleFromTopK's f64 tail.
+// Pools above 256 take pool_row_kernel, one workgroup per row from the first element to the draw.
 // The kernel boundary orders the first kernel's writes before the second's reads; no
 // workgroup waits on another. Rows whose pool is the whole vocabulary (top_k = 0 beyond the
 // pool capacity) end in the merge when their largest entries decide them, else in two more
@@ -111,6 +109,7 @@ __device__ __forceinline__ double rebase_sum(double sum, float lane_max, float m
 }
 constexpr int kKcapSmall = 256;
 constexpr int kKcapLarge = 1024;
+constexpr int kMaxVocab = 1 << 20;
 
 struct SliceStat {
   float max;      // slice max (f32, exact)
@@ -118,7 +117,7 @@ struct SliceStat {
   double sum;     // sum over the slice of exp(x - max)
 };
 // SliceStat.count of a row that pool_row_kernel ended itself (sampled, or its status written):
-// merge_kernel skips the row.
+// pool_handoff_kernel skips the row.
 constexpr uint32_t kPoolRowDone = 0xffffffffu;
 
 // Per-row hand-over from the sampling kernel to the head kernel (whole-vocabulary rows).
@@ -181,7 +180,6 @@ struct Launch {
   int32_t parts;      // row_kernel: 1 = one workgroup per row; > 1 = workgroups per row (each
                       // a part of slice_len elements, finished by wave_merge_kernel); 0 = unused
   int32_t row_waves;  // row_kernel: waves per workgroup
-  int32_t pool_rows;  // 1: pool_row_kernel streams each row (pools above 256, rows >= CUs)
   int32_t list_stride;  // pools <= 256: entries between the sorted lists of consecutive slices
                         // (or parts) of a row in cands -- slice_len, or kWaveKcap when the
                         // lists are packed (a list never holds more than the pool)
@@ -474,118 +472,6 @@ __device__ __forceinline__ void finish_row(Smem &sm, const Launch &L, int row, c
   }
 }
 
-// sampleFromTopK (src/engine/sampler.ts:147-212) for a pool of at most 64*R candidates, by
-// one wave, in registers: element i of the pool is register i/64 of lane i%64. The
-// per-element terms are computed lane-parallel; each sum is sequential in index order,
-// lane by lane through readlane, as the reference's left-to-right reduce. The running sums
-// of the draw equal the top-p cumulative sums, so they are kept (writelane) from the
-// top-p scan (each lane keeps its own element's) and the draw is a ballot over
-// "target < running".
-template <int R, typename In>
-__device__ __forceinline__ void wave_finish(const uint64_t *pool_in, int count, const Launch &L, int row,
-                            const In *row_src, float max_logit, double sum_exp,
-                            const tabby_row_params &P) {
-  const int lane = wave_lane();
-  uint64_t v[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int i = r * kWaveSize + lane;
-    v[r] = i < count ? pool_in[i] : 0ull;
-  }
-  wave_sort_desc<R>(v);
-  const double T = P.temperature;
-  double exact[R], w[R];
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    exact[r] = 0.0;
-    w[r] = 0.0;
-    if (r * kWaveSize + lane < count) {
-      const double d = (double)value_of(composite_key(v[r])) - (double)max_logit;
-      exact[r] = fdlibm_exp(d) / sum_exp;
-      if (!greedy_temp(T)) w[r] = fdlibm_exp(d / T);
-    }
-  }
-  double pool = 0.0, scaled = 0.0;
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int m = min(kWaveSize, count - r * kWaveSize);
-    for (int j = 0; j < m; ++j) {
-      pool += readlane_f64(exact[r], j);
-      scaled += readlane_f64(w[r], j);
-    }
-  }
-  tabby_row_result res;
-  res.max_logit = max_logit;
-  res.sum_exp = sum_exp;
-  res.pool_mass = pool;
-  res.status = TABBY_OK;
-  res.topk_count = min(count, L.topk_cap);
-  int chosen = 0;
-  if (greedy_temp(T)) {
-    res.considered = 1;
-    res.pool_exhausted = 0;
-  } else {
-#pragma unroll
-    for (int r = 0; r < R; ++r) w[r] = w[r] / scaled;
-    const double top_p = P.top_p;
-    double c = 0.0, running[R];
-    int cut = count;
-    bool cut_found = false;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      running[r] = 0.0;
-      const int m = min(kWaveSize, count - r * kWaveSize);
-      for (int j = 0; j < m && !cut_found; ++j) {
-        c += readlane_f64(w[r], j);
-        running[r] = lane == j ? c : running[r];
-        if (top_p < 1.0 && c >= top_p) {
-          cut = r * kWaveSize + j + 1;
-          cut_found = true;
-        }
-      }
-    }
-    const double target = P.uniform * c;  // c is the running sum at cut - 1: the reference's total
-    chosen = cut - 1;
-    bool done = false;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int i = r * kWaveSize + lane;
-      const uint64_t hit = __ballot(i < cut && target < running[r]);
-      if (!done && hit) {
-        chosen = r * kWaveSize + __ffsll((unsigned long long)hit) - 1;
-        done = true;
-      }
-    }
-    res.considered = (uint32_t)cut;
-    res.pool_exhausted = (top_p < 1.0 && pool < top_p) ? 1 : 0;
-  }
-  // The chosen candidate's id and probability live in lane chosen%64, register chosen/64.
-  uint64_t cv = 0;
-  double cp = 0.0;
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    if (r == chosen / kWaveSize) {
-      cv = (uint64_t)__builtin_amdgcn_readlane((int)v[r], chosen % kWaveSize) |
-           ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(v[r] >> 32), chosen % kWaveSize) << 32);
-      cp = readlane_f64(exact[r], chosen % kWaveSize);
-    }
-  }
-  res.id = (int32_t)composite_index(cv);
-  res.probability = cp;
-  if (lane == 0) L.results[row] = res;
-  if (L.topk_cap > 0) {
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int i = r * kWaveSize + lane;
-      if (i < count && i < L.topk_cap) {
-        const uint32_t idx = composite_index(v[r]);
-        L.topk_ids[(size_t)row * L.topk_cap + i] = (int32_t)idx;
-        L.topk_logits[(size_t)row * L.topk_cap + i] = load_one(row_src + min(idx, (uint32_t)(L.vocab - 1)));
-      }
-    }
-  }
-}
-
 __device__ __forceinline__ void write_status(const Launch &L, int row, int32_t status, float mx,
                                              double se) {
   tabby_row_result r;
@@ -596,36 +482,6 @@ __device__ __forceinline__ void write_status(const Launch &L, int row, int32_t s
   r.status = status;
   L.results[row] = r;
 }
-
-// ---------------------------------------------------------------------------------------
-// Kernel 1 (slices): grid = rows x splits; each workgroup streams one slice of a row from
-// HBM exactly once, in chunks of 16 elements per lane (4096 per workgroup) with the next
-// chunk's loads in flight while the current one is processed. Per lane it keeps an online
-// max and an f64 sum of exp(x - max). It also collects the slice's candidates: every
-// element >= theta, where theta starts at a lower bound on the first chunk's kk-th largest
-// element (a radix select on the top 22 bits of the key) -- so at least kk distinct elements
-// reach it, and it never exceeds the slice's kk-th largest value. Candidates go to an LDS list with one atomic per
-// wave; a list that would overflow is flushed to the slice's region of global memory. The
-// exact selection happens once per row, in the merge.
-//
-// There is no cross-workgroup communication: the merge is the next kernel on the stream,
-// so the kernel boundary orders these writes before its reads (an agent-scope fence per
-// workgroup costs an L2 writeback + invalidate each, measured slower than the whole read).
-// ---------------------------------------------------------------------------------------
-constexpr int kChunkPerLane = 16;
-constexpr int kChunk = kChunkPerLane * kBlock;
-constexpr int kListCap = kChunk;  // a whole chunk always fits after a flush
-
-struct SliceSmem {
-  BlockScratch bs;
-  uint32_t list_count;  // list length after a prune or flush
-  uint32_t committed;   // list_count as of the last chunk boundary (stable between barriers)
-  uint32_t flushed;     // candidates already written to global memory
-  uint32_t wave_count[2][kWaves];  // by chunk parity: chunk c+1 writes while c is read
-  float theta;
-  uint32_t hist[kBins];       // radix-select histograms (first-chunk theta, list pruning)
-  uint64_t list[kListCap];
-};
 
 // theta from a selection threshold key, clamped to [-inf, +inf]: an early-exit prefix can
 // fall below the key of -inf (or above +inf), where keys decode to NaN.
@@ -654,247 +510,6 @@ __device__ __forceinline__ uint32_t wave_slot(bool take, uint32_t *slot) {
 
 // Raw loads of chunk `chunk` (no masking, so nothing consumes them until the next
 // iteration and they stay in flight). Lanes past the end reread the slice's last vector.
-template <typename In, int VEC>
-__device__ __forceinline__ void load_chunk(const In *src, int n, int chunk, float (&x)[kChunkPerLane]) {
-  constexpr int ITEMS = kChunkPerLane / VEC;
-#pragma unroll
-  for (int j = 0; j < ITEMS; ++j) {
-    const int le = chunk * kChunk + (j * kBlock + (int)threadIdx.x) * VEC;
-    float v[VEC];
-    Loader<In, VEC>::load(src + min(le, n - VEC), v);
-#pragma unroll
-    for (int c = 0; c < VEC; ++c) x[j * VEC + c] = v[c];
-  }
-}
-
-// Padding lanes of chunk `chunk` become -inf, which no statistic or candidate test admits.
-template <int VEC>
-__device__ __forceinline__ void mask_chunk(int n, int chunk, float (&x)[kChunkPerLane]) {
-  constexpr int ITEMS = kChunkPerLane / VEC;
-#pragma unroll
-  for (int j = 0; j < ITEMS; ++j) {
-    const bool valid = chunk * kChunk + (j * kBlock + (int)threadIdx.x) * VEC < n;
-#pragma unroll
-    for (int c = 0; c < VEC; ++c) x[j * VEC + c] = valid ? x[j * VEC + c] : -INFINITY;
-  }
-}
-
-template <int VEC>
-__device__ __forceinline__ int chunk_local(int chunk, int e) {
-  // Slice-local index of register element e of this lane in chunk `chunk`.
-  return chunk * kChunk + ((e / VEC) * kBlock + (int)threadIdx.x) * VEC + e % VEC;
-}
-
-// Copies the LDS list to the slice's global region and empties it. Whole workgroup.
-__device__ __forceinline__ void flush_list(SliceSmem &sm, uint64_t *region, uint32_t count) {
-  const uint32_t at = sm.flushed;
-  for (uint32_t i = threadIdx.x; i < count; i += kBlock) region[at + i] = sm.list[i];
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    sm.flushed = at + count;
-    sm.list_count = 0u;
-    sm.committed = 0u;
-  }
-  __syncthreads();
-}
-
-// Drops from the LDS list every entry below the key of its kk-th largest composite and
-// raises sm.theta to that key. Whole workgroup; returns the new length (>= kk).
-__device__ __forceinline__ uint32_t prune_list(SliceSmem &sm, uint32_t have, uint32_t kk) {
-  auto each = [&](auto &&f) {
-    for (uint32_t i = threadIdx.x; i < have; i += kBlock) f(sm.list[i]);
-  };
-  // Two radix passes (the key's top 22 bits) suffice: entries tied on the key are kept anyway.
-  const SelectResult r = radix_select(each, kk, sm.hist, sm.bs, 2);
-  const uint32_t key = min(max((uint32_t)(r.prefix >> 32), kNegInfKey), 0xff800000u);
-  constexpr int kPer = kListCap / kBlock;
-  uint64_t v[kPer];
-#pragma unroll
-  for (int q = 0; q < kPer; ++q) {
-    const uint32_t i = (uint32_t)(q * kBlock) + threadIdx.x;
-    v[q] = i < have ? sm.list[i] : 0ull;
-  }
-  if (threadIdx.x == 0) sm.bs.slot = 0u;
-  __syncthreads();
-#pragma unroll
-  for (int q = 0; q < kPer; ++q) {
-    const uint32_t i = (uint32_t)(q * kBlock) + threadIdx.x;
-    const bool keep = i < have && composite_key(v[q]) >= key;
-    const uint32_t at = wave_slot(keep, &sm.bs.slot);
-    if (keep) sm.list[at] = v[q];
-  }
-  __syncthreads();
-  const uint32_t kept = sm.bs.slot;
-  if (threadIdx.x == 0) {
-    sm.theta = fmaxf(sm.theta, value_of(key));
-    sm.list_count = kept;
-    sm.committed = kept;
-  }
-  __syncthreads();
-  return kept;
-}
-
-template <typename In, int VEC>
-__global__ __launch_bounds__(kBlock) void slice_kernel(Launch L, Workspace W) {
-  constexpr int ITEMS = kChunkPerLane / VEC;
-  __shared__ SliceSmem sm;
-
-  int row, slice;
-  row_slice_of((int)blockIdx.x, L.rows, L.splits, row, slice);
-  const int V = L.vocab;
-  const int begin = slice * L.slice_len;
-  const int n = min(L.slice_len, V - begin);
-  const int nchunks = (n + kChunk - 1) / kChunk;
-  const tabby_row_params P = L.params[row];
-  const bool valid_params = params_valid(P, L.k_max);
-  const int keff = effective_k(P, V);
-  const int kk = slice_keep(valid_params, keff, n, L.kcap, L.head_pass, L.topk_cap);
-  const In *src = reinterpret_cast<const In *>(L.logits) + (size_t)row * V + begin;
-  // The slice's candidate region: room for every element of the slice.
-  uint64_t *region = W.cands + (size_t)row * W.row_cand_stride + (size_t)begin;
-
-  if (threadIdx.x == 0) {
-    sm.list_count = 0u;
-    sm.committed = 0u;
-    sm.flushed = 0u;
-    sm.theta = -INFINITY;
-  }
-  __syncthreads();
-  float lane_max = -INFINITY;
-  float lane_ml = 0.0f;   // fl(lane_max * L): the reference of lane_sum's terms (rebase_sum)
-  double lane_sum = 0.0;  // sum of 2^(x*L - lane_ml) over this lane's elements so far
-
-  // Chunk c held in x, with the next chunk's loads in flight (issued unconditionally on each
-  // path of the loop below and into their own registers, so the compiler's wait before
-  // chunk c leaves them in flight).
-  auto body = [&](int c, float(&x)[kChunkPerLane]) {
-    mask_chunk<VEC>(n, c, x);
-
-    // Online max / sum-exp for this lane.
-    float cm = x[0];
-#pragma unroll
-    for (int e = 1; e < kChunkPerLane; ++e) cm = fmaxf(cm, x[e]);
-    const float nm = fmaxf(lane_max, cm);
-    if (nm != -INFINITY) {
-      const float ml = nm * kLog2e;
-      float t[kChunkPerLane];  // summed pairwise, as in the wave kernel
-#pragma unroll
-      for (int e = 0; e < kChunkPerLane; ++e) t[e] = __builtin_amdgcn_exp2f(fmaf(x[e], kLog2e, -ml));
-#pragma unroll
-      for (int h = kChunkPerLane / 2; h > 0; h >>= 1) {
-#pragma unroll
-        for (int e = 0; e < h; ++e) t[e] += t[e + h];
-      }
-      const float part = t[0];
-      const double rescale = lane_max == -INFINITY ? 0.0 : (double)__builtin_amdgcn_exp2f(lane_ml - ml);
-      lane_sum = lane_sum * rescale + (double)part;
-      lane_max = nm;
-      lane_ml = ml;
-    }
-
-    if (kk > 0) {
-      if (c == 0 && kk < min(n, kChunk)) {
-        // theta: a lower bound on the kk-th largest element of the first chunk (its padding
-        // excluded).
-        auto elems = [&](auto &&f) {
-#pragma unroll
-          for (int e = 0; e < kChunkPerLane; ++e) {
-            const int local = chunk_local<VEC>(0, e);
-            if (local < n) f(composite(key_of(x[e]), (uint32_t)local));
-          }
-        };
-        // Two passes: the top 22 bits of the key. The bin's lower edge still has kk
-        // elements at or above it (ties on the key would need the index digits).
-        const SelectResult r = radix_select(elems, (uint32_t)kk, sm.hist, sm.bs, 2);
-        if (threadIdx.x == 0) sm.theta = theta_of(r.prefix);
-        __syncthreads();
-      }
-      const float theta = sm.theta;
-      const bool check_index = !(theta > -INFINITY);
-      // Count first (ballots, kept for the appends), so that a list that would overflow is
-      // pruned or flushed before anything is appended; each wave's slots then follow from
-      // the per-wave counts, with no atomics.
-      uint64_t masks[kChunkPerLane];
-      uint32_t mine = 0;
-#pragma unroll
-      for (int e = 0; e < kChunkPerLane; ++e) {
-        masks[e] = __ballot(x[e] >= theta && (!check_index || chunk_local<VEC>(c, e) < n));
-        mine += (uint32_t)__popcll(masks[e]);
-      }
-      if (lane_id() == 0) sm.wave_count[c & 1][wave_id()] = mine;
-      __syncthreads();
-      uint32_t incoming = 0, before = 0;
-#pragma unroll
-      for (int w = 0; w < kWaves; ++w) {
-        const uint32_t wc = sm.wave_count[c & 1][w];
-        before += w < wave_id() ? wc : 0u;
-        incoming += wc;
-      }
-      uint32_t have = sm.committed;
-      if (incoming > 0) {
-        if (have + incoming > (uint32_t)kListCap && have >= (uint32_t)kk) {
-          // Prune: keep the entries whose key reaches the list's kk-th largest, and raise
-          // theta to it. Only massive ties can leave the list too full; it is then flushed.
-          have = prune_list(sm, have, (uint32_t)kk);
-        }
-        if (have + incoming > (uint32_t)kListCap) {
-          flush_list(sm, region, have);
-          have = 0;
-        }
-        uint32_t at = have + before;  // a chunk holds at most kChunk <= kListCap candidates
-#pragma unroll
-        for (int e = 0; e < kChunkPerLane; ++e) {
-          const uint64_t mask = masks[e];
-          if (mask) {
-            if ((mask >> lane_id()) & 1ull)
-              sm.list[at + lanes_below(mask)] =
-                  composite(key_of(x[e]), (uint32_t)(begin + chunk_local<VEC>(c, e)));
-            at += (uint32_t)__popcll(mask);
-          }
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) sm.committed = have + incoming;  // read after the next barrier
-      }
-    }
-  };
-  float x[kChunkPerLane], y[kChunkPerLane];
-  load_chunk<In, VEC>(src, n, 0, x);
-  for (int c = 0; c < nchunks; c += 2) {
-    if (c + 1 >= nchunks) {
-      body(c, x);
-      break;
-    }
-    load_chunk<In, VEC>(src, n, c + 1, y);
-    body(c, x);
-    if (c + 2 >= nchunks) {
-      body(c + 1, y);
-      break;
-    }
-    load_chunk<In, VEC>(src, n, c + 2, x);
-    body(c + 1, y);
-  }
-
-  // Slice statistics (their barriers also publish `committed`).
-  const float ms = block_max(lane_max, sm.bs);
-  const double ss = block_sum(rebase_sum(lane_sum, lane_max, lane_ml, ms), sm.bs);
-  uint32_t total = 0;
-  if (kk > 0) {
-    uint32_t have = sm.committed;
-    // A last prune keeps the merge's candidate set small (about kk plus ties per slice).
-    if (have > (uint32_t)kk + (uint32_t)kk / 4u) have = prune_list(sm, have, (uint32_t)kk);
-    total = sm.flushed + have;
-    const uint32_t at = sm.flushed;
-    for (uint32_t i = threadIdx.x; i < have; i += kBlock) region[at + i] = sm.list[i];
-  }
-  if (threadIdx.x == 0) {
-    SliceStat st_out;
-    st_out.max = ms;
-    st_out.count = total;
-    st_out.sum = ss;
-    W.stats[(size_t)row * kMaxSplits + slice] = st_out;
-  }
-}
-
 // ---------------------------------------------------------------------------------------
 // Kernel 1 for pools of at most 256 (wave_kernel): grid = rows x splits, one wave per
 // workgroup, so nothing in it waits at a barrier. Each wave streams its slice of a row from
@@ -1546,235 +1161,41 @@ __device__ __forceinline__ uint32_t store_threshold(float row_max, const tabby_r
 }
 
 // ---------------------------------------------------------------------------------------
-// Kernel 2 (merge): one workgroup per row. Row max and sum-exp from the slice statistics
-// (in slice order, so the result does not depend on scheduling), the exact top-keff of the
-// slices' candidates, an LDS bitonic sort, and sampleFromTopK.
+// A head pass's whole-vocabulary rows in a batch of large pools (pool_row_kernel ends every
+// other row): the row's top Nw = max(topk_cap, kHeadList) (slice_keep), unsorted in its
+// candidate region, sorted; its statistics, head key and, when Nw fits a wave's register sort
+// (<= 256), the list handed on to head_kernel and head_pick_kernel, as from finish_pool. The
+// head also covers the caller's top-k list, the first topk_cap of them.
 // ---------------------------------------------------------------------------------------
-constexpr int kCandLds = 4096;  // candidate lists up to this size are staged in LDS (two workgroups fit a CU)
-
-template <int KCAP>
-struct MergeSmem {
-  BlockScratch bs;
-  float row_max;
-  double sum_exp;
-  double pool_mass;
-  double scaled_total;
-  uint32_t slice_first[kMaxSplits];
-  double slice_term[kMaxSplits];
-  uint64_t sorted[KCAP];
-  uint64_t cand[kCandLds];
-  union {
-    uint32_t hist[kBins];
-    struct {
-      double exact[KCAP];
-      double w[KCAP];
-    } tail;
-  } u;
-};
-
-template <int KCAP, typename In>
-__global__ __launch_bounds__(kBlock) void merge_kernel(Launch L, Workspace W) {
-  __shared__ MergeSmem<KCAP> sm;
+__global__ __launch_bounds__(kBlock) void pool_handoff_kernel(Launch L, Workspace W) {
+  __shared__ uint64_t sorted[kKcapLarge];
   const int row = (int)blockIdx.x;
-  if (L.pool_rows && W.stats[(size_t)row * kMaxSplits].count == kPoolRowDone) return;
-  const int splits = L.splits;
-  const int V = L.vocab;
+  const SliceStat st = W.stats[(size_t)row * kMaxSplits];
+  if (st.count == kPoolRowDone) return;
   const tabby_row_params P = L.params[row];
-  const bool valid_params = params_valid(P, L.k_max);
-  const int keff = effective_k(P, V);
-  const bool finite = valid_params && keff <= L.kcap;
-  const In *row_src = reinterpret_cast<const In *>(L.logits) + (size_t)row * V;
-
-  // 0. Candidate counts per slice (in the statistics) and their offsets; then the
-  //    candidate loads are issued together, ahead of the statistics math.
-  const SliceStat *stats = W.stats + (size_t)row * kMaxSplits;
-  SliceStat mine;
-  mine.max = -INFINITY;
-  mine.count = 0u;
-  mine.sum = 0.0;
-  if ((int)threadIdx.x < splits) mine = stats[threadIdx.x];
-  uint32_t total_u;
-  const bool collects = valid_params && (finite || L.head_pass);
-  const uint32_t first = block_exclusive_scan(collects ? mine.count : 0u, sm.bs, &total_u);
-  if ((int)threadIdx.x < splits) sm.slice_first[threadIdx.x] = first;
-  __syncthreads();
-  const int C = (int)total_u;
+  const int C = min((int)st.count, kKcapLarge);
   const uint64_t *cands = W.cands + (size_t)row * W.row_cand_stride;
-  // Flat candidate i lives in slice s (the last with slice_first[s] <= i), at
-  // cands[s*slice_len + i - slice_first[s]].
-  auto cand_addr = [&](int i) {
-    int lo = 0, hi = splits - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if ((int)sm.slice_first[mid] <= i) lo = mid; else hi = mid - 1;
-    }
-    return cands + (size_t)lo * L.slice_len + (i - (int)sm.slice_first[lo]);
-  };
-  const bool staged = C <= kCandLds;
-  if (staged) {
-    constexpr int B = 8;
-    for (int base = 0; base < C; base += B * kBlock) {
-      uint64_t v[B];
-#pragma unroll
-      for (int u = 0; u < B; ++u) {
-        const int i = base + u * kBlock + (int)threadIdx.x;
-        v[u] = i < C ? *cand_addr(i) : 0ull;
-      }
-#pragma unroll
-      for (int u = 0; u < B; ++u) {
-        const int i = base + u * kBlock + (int)threadIdx.x;
-        if (i < C) sm.cand[i] = v[u];
-      }
-    }
-  }
+  const int npow = next_pow2(C);
+  for (int i = threadIdx.x; i < npow; i += kBlock) sorted[i] = i < C ? cands[i] : 0ull;
+  __syncthreads();
+  if (npow > 1) block_sort_desc(sorted, npow);
+  const int Nw = min(max(L.topk_cap, kHeadList), L.vocab);
+  const int handed = Nw <= kWaveKcap && C >= Nw ? Nw : 0;
+  uint64_t *list = W.head_sorted + (size_t)row * W.head_stride;
+  for (int i = threadIdx.x; i < handed; i += kBlock) list[i] = sorted[i];
   if (threadIdx.x == 0) {
-    sm.bs.slot = 0u;
+    const int need = min(L.topk_cap, L.vocab);
+    const uint32_t list_key = need == 0 ? 0xffffffffu : C >= need ? composite_key(sorted[need - 1]) : kNegInfKey;
+    const uint32_t weights_key = head_threshold(st.max, P.temperature);
+    RowState rs;
+    rs.max = st.max;
+    rs.sum_exp = st.sum;
+    rs.status = TABBY_OK;
+    rs.handoff = (uint32_t)handed << 16;
+    rs.head_key = min(weights_key, list_key);
+    rs.store_key = store_threshold(st.max, P, L.vocab, 1.0, weights_key);
+    W.row_state[row] = rs;
   }
-
-  // 1. Row max and sum-exp, in slice order.
-  const float M = block_max(mine.max, sm.bs);
-  if ((int)threadIdx.x < splits)
-    sm.slice_term[threadIdx.x] =
-        mine.max == -INFINITY ? 0.0 : mine.sum * fdlibm_exp((double)mine.max - (double)M);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    double S = 0.0;
-    for (int s = 0; s < splits; ++s) S += sm.slice_term[s];
-    sm.sum_exp = S;
-  }
-  __syncthreads();
-  const float row_max = M;
-  const double sum_exp = sm.sum_exp;
-  const bool in_domain = (row_max > -INFINITY) && (row_max < INFINITY) && (sum_exp > 0.0) &&
-                         (sum_exp < INFINITY);
-
-  if (!valid_params || !in_domain) {
-    if (threadIdx.x == 0) {
-      write_status(L, row, !valid_params ? TABBY_EINVAL : TABBY_EDOMAIN, row_max, sum_exp);
-      W.row_state[row].status = !valid_params ? TABBY_EINVAL : TABBY_EDOMAIN;
-    }
-    return;
-  }
-  if (!finite && !L.head_pass) {
-    if (threadIdx.x == 0) write_status(L, row, TABBY_EINVAL, row_max, sum_exp);
-    return;
-  }
-  // 2. The exact top-keff of the row's candidates, sorted. The candidates include every
-  //    element of the row's top-keff (each slice kept all elements >= a lower bound of its
-  //    own kk-th largest value).
-  const uint32_t floor_key = kNegInfKey;
-  auto from_lds = [&](auto &&f) {
-    for (int i = threadIdx.x; i < C; i += kBlock) {
-      const uint64_t v = sm.cand[i];
-      if (composite_key(v) >= floor_key) f(v);
-    }
-  };
-  auto from_global = [&](auto &&f) {
-    constexpr int B = 8;  // loads in flight per lane before the first use
-    for (int base = 0; base < C; base += B * kBlock) {
-      uint64_t v[B];
-#pragma unroll
-      for (int u = 0; u < B; ++u) {
-        const int i = base + u * kBlock + (int)threadIdx.x;
-        v[u] = i < C ? *cand_addr(i) : 0ull;
-      }
-#pragma unroll
-      for (int u = 0; u < B; ++u)
-        if (base + u * kBlock + (int)threadIdx.x < C && composite_key(v[u]) >= floor_key) f(v[u]);
-    }
-  };
-  if (!finite) {
-    // Whole-vocabulary row: hand max / sum-exp / the head threshold to the head kernels. The
-    // candidates hold the row's top Nw = max(topk_cap, kHeadList) (slice_keep): when Nw fits a
-    // wave's register sort (<= 256) they go on sorted to head_pick_kernel, as from finish_pool;
-    // the head also covers the caller's top-k list, the first topk_cap of them.
-    const int Nw = min(max(L.topk_cap, kHeadList), V);
-    const int need = min(L.topk_cap, V);
-    uint32_t list_key = 0xffffffffu;
-    int handed = 0;
-    if (Nw <= kWaveKcap && C >= Nw) {
-      auto pick = [&](auto &&each) {
-        if (threadIdx.x == 0) sm.bs.slot = 0u;
-        __syncthreads();
-        if (C > Nw) {
-          const SelectResult r = radix_select(each, (uint32_t)Nw, sm.u.hist, sm.bs);
-          each([&](uint64_t v) {
-            const bool take = selected(v, r);
-            const uint32_t at = wave_slot(take, &sm.bs.slot);
-            if (take && at < (uint32_t)Nw) sm.sorted[at] = v;
-          });
-        } else {
-          each([&](uint64_t v) {
-            const uint32_t at = wave_slot(true, &sm.bs.slot);
-            if (at < (uint32_t)Nw) sm.sorted[at] = v;
-          });
-        }
-      };
-      if (staged) pick(from_lds); else pick(from_global);
-      const int npow = next_pow2(Nw);
-      for (int i = Nw + (int)threadIdx.x; i < npow; i += kBlock) sm.sorted[i] = 0ull;
-      __syncthreads();
-      block_sort_desc(sm.sorted, npow);
-      uint64_t *list = W.head_sorted + (size_t)row * W.head_stride;
-      for (int i = threadIdx.x; i < Nw; i += kBlock) list[i] = sm.sorted[i];
-      if (need > 0) list_key = composite_key(sm.sorted[need - 1]);
-      handed = Nw;
-    } else if (need > 0) {
-      if (C >= need) {  // the candidates hold the row's top `need`: select the need-th largest
-        const SelectResult r = staged ? radix_select(from_lds, (uint32_t)need, sm.u.hist, sm.bs)
-                                      : radix_select(from_global, (uint32_t)need, sm.u.hist, sm.bs);
-        // Every selected composite is >= r.prefix, whose low bits below r.shift are zero: with -inf
-        // in the list its key can fall below -inf's, where no value lies.
-        list_key = max((uint32_t)(r.prefix >> 32), kNegInfKey);
-      } else {
-        list_key = kNegInfKey;  // fewer candidates than the list: take the whole row
-      }
-    }
-    if (threadIdx.x == 0) {
-      RowState rs;
-      rs.max = row_max;
-      rs.sum_exp = sum_exp;
-      rs.status = TABBY_OK;
-      rs.handoff = (uint32_t)handed << 16;
-      const uint32_t weights_key = head_threshold(row_max, P.temperature);
-      rs.head_key = min(weights_key, list_key);
-      rs.store_key = store_threshold(row_max, P, V, 1.0, weights_key);
-      W.row_state[row] = rs;
-    }
-    return;
-  }
-  auto gather = [&](auto &&each) {
-    if (C > keff) {
-      const SelectResult r = radix_select(each, (uint32_t)keff, sm.u.hist, sm.bs);
-      each([&](uint64_t v) {
-        const bool take = selected(v, r);
-        const uint32_t at = wave_slot(take, &sm.bs.slot);
-        if (take && at < (uint32_t)keff) sm.sorted[at] = v;
-      });
-    } else {
-      each([&](uint64_t v) {
-        const uint32_t at = wave_slot(true, &sm.bs.slot);
-        if (at < (uint32_t)keff) sm.sorted[at] = v;
-      });
-    }
-  };
-  if (staged) gather(from_lds); else gather(from_global);
-  __syncthreads();
-
-  // 3. Sort and sampleFromTopK: by wave 0 in registers for pools up to 256, else by the
-  //    workgroup through LDS.
-  if (keff <= kWaveKcap) {
-    if (wave_id() != 0) return;
-    if (keff <= 64) wave_finish<1, In>(sm.sorted, keff, L, row, row_src, row_max, sum_exp, P);
-    else if (keff <= 128) wave_finish<2, In>(sm.sorted, keff, L, row, row_src, row_max, sum_exp, P);
-    else wave_finish<4, In>(sm.sorted, keff, L, row, row_src, row_max, sum_exp, P);
-    return;
-  }
-  const int npow = next_pow2(keff);
-  for (int i = keff + (int)threadIdx.x; i < npow; i += kBlock) sm.sorted[i] = 0ull;
-  __syncthreads();
-  block_sort_desc(sm.sorted, npow);
-  finish_row<KCAP, In>(sm, L, row, row_src, keff, row_max, sum_exp, P);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -3428,7 +2849,7 @@ constexpr int kHeadBatch = 4096;
 __host__ __device__ __forceinline__ int plan_slots(int vocab_max) { return vocab_max / kSegCap + 2; }
 
 constexpr int kPlanThreads = 1024;  // a 13 K-entry head took 24.5 us on 256 lanes
-static_assert(kMaxSplits * kChunk <= kPlanThreads * kHeadSlice, "head_pick_kernel takes one slice per thread");
+static_assert(kMaxVocab <= kPlanThreads * kHeadSlice, "head_pick_kernel takes one slice per thread");
 
 struct PlanSmem {
   uint32_t wave_total[kPlanThreads / kWaveSize];
@@ -4325,9 +3746,9 @@ __global__ void exp_kernel(const double *x, double *y, int64_t n) {
 // the first chunk's kk-th largest -- a quarter of that chunk at kk = 1,024 -- and pruned its
 // list with two workgroup barriers per chunk: config 5 took 135 us there.) At the end the
 // workgroup selects the row's exact top kk from the list (pool_select), gathers it into LDS,
-// sorts it and samples it (finish_row over its 16 waves), as merge_kernel would have; a row
+// sorts it and samples it (finish_row over its 16 waves); a row
 // outside the contract gets its status here too. Only a head pass's whole-vocabulary rows
-// leave their top list, unsorted, with the row's statistics, as slice 0 for merge_kernel.
+// leave their top list, unsorted, with the row's statistics, as slice 0 for pool_handoff_kernel.
 // ---------------------------------------------------------------------------------------
 constexpr int kPoolWaves = 16;
 constexpr int kPoolThreads = kPoolWaves * kWaveSize;
@@ -4846,17 +4267,16 @@ __global__ __launch_bounds__(kPoolThreads, 8) void pool_row_kernel(Launch L, Wor
   }
   // The row's exact top kk of the candidates, unsorted: to `sorted` in LDS for a row this
   // workgroup samples itself (valid parameters, a pool of at most kcap, finite statistics:
-  // every row that merge_kernel would sample from the pool), else to region[0 .. kept) for
-  // merge_kernel (statuses and whole-vocabulary rows).
+  // every finite pool), else to region[0 .. kept) for pool_handoff_kernel (whole-vocabulary rows).
   if (w == 0) {
     TABBY_STAMP(17);
     TABBY_RECORD(31, C);
     TABBY_RECORD(29, rescan ? 1 : 0);
   }
   const RowStats rs = row_stats(sm.stats, kPoolWaves);
-  // The row's outcome, as merge_kernel decides it: a status (parameters outside the contract,
+  // The row's outcome: a status (parameters outside the contract,
   // statistics outside the domain, a whole-vocabulary row with no head pass), a pool this
-  // workgroup samples (`here`), or a whole-vocabulary row for merge_kernel and the head
+  // workgroup samples (`here`), or a whole-vocabulary row for pool_handoff_kernel and the head
   // kernels. (C >= kk >= 1 for a pool in the domain: theta has kk elements at or above it --
   // the floor always, a guessed bound once the count above has shown it.)
   const bool in_domain = rs.max > -INFINITY && rs.max < INFINITY && rs.sum_exp > 0.0 && rs.sum_exp < INFINITY;
@@ -4918,8 +4338,7 @@ __global__ __launch_bounds__(kPoolThreads, 8) void pool_row_kernel(Launch L, Wor
     kept = C;
   }
   if (here) {
-    // sampleFromTopK over the pool, as merge_kernel would: the statistics are this row's one
-    // slice's (the merge's sum in slice order is that slice's sum), the pool sorted descending.
+    // sampleFromTopK over the pool, sorted descending.
     const int count = (int)kept;
     const int npow = next_pow2(count);
     for (int i = count + (int)threadIdx.x; i < npow; i += kPoolThreads) sm.sorted[i] = 0ull;
@@ -5032,32 +4451,26 @@ struct Plan {
   int vec;
 };
 
-// Enough slices per row that the batch fills the chip about once: 256 CUs x 3 resident
-// 256-lane workgroups of the slice kernel (its 41.5 KB of LDS leaves room for three; a
-// larger grid ran in two rounds -- config 5, 512 rows: 3 slices per row took 225 us, one
-// 200 us), rounded down, or 256 CUs x 4 SIMDs x 4 one-wave workgroups for the wave kernel
-// (measured at 256 rows: 16 slices per row, 39.9 us per call, beat 12 per row, 41.4 us --
-// the SIMDs issue their oldest wave first and a fourth wave hides more of the others'
-// waits -- and 18 or 20 per row, which no longer fit at once, ~50 us). Each
-// slice is at least one chunk long (two for the wave kernel) and aligned to the vector
-// loads. A row's wave slices are capped at kMaxWaveSplits: with few rows the chip is idle
-// anyway and the latency is one slice's chain plus the merge, whose cost grows with the
-// number of lists (measured on one row: 24 slices of 2048 beat 12 of 4096 and 48 of 1024
-// at vocab 49152; 37 slices of 4096 beat 46 and 74 at vocab 151936).
-constexpr int kTargetGroups = 768;
+// Enough one-wave slices per row (wave_kernel) that the batch fills the chip about once: 256 CUs
+// x 4 SIMDs x 4 waves (measured at 256 rows: 16 slices per row, 39.9 us per call, beat 12 per
+// row, 41.4 us -- the SIMDs issue their oldest wave first and a fourth wave hides more of the
+// others' waits -- and 18 or 20 per row, which no longer fit at once, ~50 us). Each slice is at
+// least two chunks long and aligned to the vector loads. A row's slices are capped at
+// kMaxWaveSplits: with few rows the chip is idle anyway and the latency is one slice's chain
+// plus the merge, whose cost grows with the number of lists (measured on one row: 24 slices of
+// 2048 beat 12 of 4096 and 48 of 1024 at vocab 49152; 37 slices of 4096 beat 46 and 74 at
+// vocab 151936).
 constexpr int kTargetWaves = 4096;
 constexpr int kMaxWaveSplits = 36;
 
-Plan make_plan(int rows, int vocab, int dtype, const void *logits, bool wave) {
+Plan make_plan(int rows, int vocab, int dtype, const void *logits) {
   Plan p;
   const int vec_elems = dtype == TABBY_F32 ? 4 : 8;
   const bool aligned = ((uintptr_t)logits % 16u) == 0 && vocab % vec_elems == 0;
   p.vec = aligned ? vec_elems : 1;
-  const int chunk = wave ? 2 * kWChunk : kChunk;
-  const int target = wave ? kTargetWaves : kTargetGroups;
-  const int most = std::min(wave ? kMaxWaveSplits : kMaxSplits, (vocab + chunk - 1) / chunk);
-  const int want = std::max(1, std::min(most, wave ? (target + rows - 1) / rows : target / rows));
-  const int granule = (wave ? kWaveSize : kBlock) * p.vec;
+  const int most = std::min(kMaxWaveSplits, (vocab + 2 * kWChunk - 1) / (2 * kWChunk));
+  const int want = std::max(1, std::min(most, (kTargetWaves + rows - 1) / rows));
+  const int granule = kWaveSize * p.vec;
   const int per = (vocab + want - 1) / want;
   p.slice_len = (per + granule - 1) / granule * granule;
   p.splits = (vocab + p.slice_len - 1) / p.slice_len;
@@ -5106,15 +4519,10 @@ hipError_t launch_pair(const Launch &L, const Workspace &W, int cus, hipStream_t
   if (L.kcap <= kWaveKcap) {
     if (L.head_pass) launch_first<In, VEC, true>(L, W, stream);
     else launch_first<In, VEC, false>(L, W, stream);
-  } else if (L.pool_rows) {
-    // pool_row_kernel ends every row but a head pass's whole-vocabulary ones, which
-    // merge_kernel hands to the head kernels.
-    hipLaunchKernelGGL((pool_row_kernel<In, VEC>), rows, dim3(kPoolThreads), 0, stream, L, W);
-    if (L.head_pass)
-      hipLaunchKernelGGL((merge_kernel<kKcapLarge, In>), rows, dim3(kBlock), 0, stream, L, W);
   } else {
-    hipLaunchKernelGGL((slice_kernel<In, VEC>), slices, dim3(kBlock), 0, stream, L, W);
-    hipLaunchKernelGGL((merge_kernel<kKcapLarge, In>), rows, dim3(kBlock), 0, stream, L, W);
+    // pool_row_kernel ends every row but a head pass's whole-vocabulary ones.
+    hipLaunchKernelGGL((pool_row_kernel<In, VEC>), rows, dim3(kPoolThreads), 0, stream, L, W);
+    if (L.head_pass) hipLaunchKernelGGL(pool_handoff_kernel, rows, dim3(kBlock), 0, stream, L, W);
   }
   return hipGetLastError();
 }
@@ -5146,7 +4554,7 @@ hipError_t dispatch(int dtype, const Plan &p, const Launch &L, const Workspace &
 Plan plan_launch(int rows, int vocab, int dtype, const void *logits, int k_max, int topk_cap, int cus,
                  bool head_pass, Launch &L) {
   const int kcap = k_max <= kKcapSmall ? kKcapSmall : kKcapLarge;
-  const Plan p = make_plan(rows, vocab, dtype, logits, kcap <= kWaveKcap);
+  const Plan p = make_plan(rows, vocab, dtype, logits);
   L = Launch{};
   L.logits = logits;
   L.rows = rows;
@@ -5161,11 +4569,12 @@ Plan plan_launch(int rows, int vocab, int dtype, const void *logits, int k_max, 
   L.h_splits = (vocab + kHeadSlice - 1) / kHeadSlice;
   L.parts = 0;
   L.row_waves = 0;
-  L.pool_rows = 0;
-  if (kcap > kWaveKcap && rows >= cus) {
-    // One pool_row_kernel workgroup per row (merge_kernel, for a head pass, reads a
-    // whole-vocabulary row's list as slice 0).
-    L.pool_rows = 1;
+  if (kcap > kWaveKcap) {
+    // One pool_row_kernel workgroup per row, however few rows (pool_handoff_kernel, for a head
+    // pass, reads a whole-vocabulary row's list as slice 0). Fewer rows than CUs, cut into 256-lane
+    // slices whose candidates a second kernel selected and sorted, took 495 us for one row of 151,936
+    // (k = 1,024, ties; 265 without), 551 for 16, 186 for 64, 107 for 255; now 34, 36, 37 and 46.
+    // One row of 32,000 at k = 512: 35 -> 19.5.
     L.splits = 1;
     L.slice_len = vocab;
   } else if (L.kcap <= kWaveKcap && rows * 2 > cus && rows < cus) {
@@ -5271,8 +4680,8 @@ int tabby_sampler_create(int device, int32_t vocab_max, int32_t rows_max, int32_
                          tabby_sampler **out) {
   if (!out) return fail(TABBY_EINVAL, "out pointer is null");
   *out = nullptr;
-  if (vocab_max < 1 || vocab_max > kMaxSplits * kChunk)
-    return fail(TABBY_EINVAL, "vocab_max must be between 1 and " + std::to_string(kMaxSplits * kChunk));
+  if (vocab_max < 1 || vocab_max > kMaxVocab)
+    return fail(TABBY_EINVAL, "vocab_max must be between 1 and " + std::to_string(kMaxVocab));
   if (rows_max < 1 || rows_max > (1 << 20)) return fail(TABBY_EINVAL, "rows_max must be between 1 and 1048576");
   if (k_max < 1 || k_max > kKcapLarge)
     return fail(TABBY_ECAPACITY, "k_max must be between 1 and " + std::to_string(kKcapLarge));
@@ -5535,8 +4944,8 @@ int tabby_sampler_sample_device_noalloc(const void *logits_dev, int32_t dtype, i
   if (!logits_dev) return fail(TABBY_EINVAL, "logits pointer is null");
   if (dtype != TABBY_F32 && dtype != TABBY_F16) return fail(TABBY_EINVAL, "dtype must be TABBY_F32 or TABBY_F16");
   if (rows < 1 || rows > (1 << 20)) return fail(TABBY_EINVAL, "rows must be between 1 and 1048576, got " + std::to_string(rows));
-  if (vocab < 1 || vocab > kMaxSplits * kChunk)
-    return fail(TABBY_EINVAL, "vocab must be between 1 and " + std::to_string(kMaxSplits * kChunk) + ", got " + std::to_string(vocab));
+  if (vocab < 1 || vocab > kMaxVocab)
+    return fail(TABBY_EINVAL, "vocab must be between 1 and " + std::to_string(kMaxVocab) + ", got " + std::to_string(vocab));
   if (k_max < 1 || k_max > kWaveKcap)
     return fail(TABBY_ECAPACITY, "k_max must be between 1 and " + std::to_string(kWaveKcap) +
                                      " for the allocation-free entry, got " + std::to_string(k_max));

@@ -575,6 +575,21 @@ def test_more_rows_than_cus(oracle, rows, vocab, dtype):
     compare(w, res, ids, vals, run_oracle(oracle, w, cap), cap)
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("rows,vocab", [(1, 1025), (3, 300), (5, 2047), (2, 16385), (7, 33001), (130, 4096), (1, 151936)])
+def test_large_pools_few_rows(oracle, rows, vocab, dtype):
+    # pool_row_kernel on fewer rows than CUs: rows of one to 149 chunks, pools around and above
+    # 256 and the whole (short) row, ties, -inf, greedy rows, whole-vocabulary rows and lists.
+    w = synth.random_workload(rows=rows, vocab=vocab, seed=rows + vocab, k_choices=(257, 1024, 1000, 0, 3),
+                              ties=rows % 2 == 1, neg_inf_frac=0.25 if rows > 2 else 0.0, top_ps=(0.98, 1.0))
+    if rows == 1:
+        w.top_k[0] = 1024
+    w.logits = w.logits.astype(dtype)
+    cap = min(vocab, 300)
+    res, ids, vals = run_gpu(w, k_max=1024, topk_cap=cap)
+    compare(w, res, ids, vals, run_oracle(oracle, w, cap), cap)
+
+
 @pytest.mark.parametrize("vocab", [32769, 50257, 65537, 151937])
 def test_parts_with_idle_waves(oracle, vocab):
     # Rows cut into parts of 16,384 elements or fewer: the last part has fewer chunks than its
