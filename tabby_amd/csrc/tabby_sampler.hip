@@ -1809,7 +1809,6 @@ constexpr int kRowMinWaves = kWaves + 1;  // four merge the lists, one the stati
 
 template <int NW>
 struct RowSmem {
-  static constexpr int kWavesMax = NW;
   WaveSmem wave[NW];
   SliceStat stats[NW];
   WaveMergeSmem merge;
@@ -4514,8 +4513,8 @@ void launch_first(const Launch &L, const Workspace &W, hipStream_t stream) {
 }
 
 template <typename In, int VEC>
-hipError_t launch_pair(const Launch &L, const Workspace &W, int cus, hipStream_t stream) {
-  const dim3 slices((unsigned)(L.rows * L.splits)), rows((unsigned)L.rows);
+hipError_t launch_pair(const Launch &L, const Workspace &W, hipStream_t stream) {
+  const dim3 rows((unsigned)L.rows);
   if (L.kcap <= kWaveKcap) {
     if (L.head_pass) launch_first<In, VEC, true>(L, W, stream);
     else launch_first<In, VEC, false>(L, W, stream);
@@ -4536,14 +4535,14 @@ hipError_t launch_head(const Launch &L, const Workspace &W, hipStream_t stream) 
   return hipGetLastError();
 }
 
-hipError_t dispatch(int dtype, const Plan &p, const Launch &L, const Workspace &W, int cus, hipStream_t s) {
+hipError_t dispatch(int dtype, const Plan &p, const Launch &L, const Workspace &W, hipStream_t s) {
   hipError_t e;
   if (dtype == TABBY_F32) {
-    e = p.vec == 4 ? launch_pair<float, 4>(L, W, cus, s) : launch_pair<float, 1>(L, W, cus, s);
+    e = p.vec == 4 ? launch_pair<float, 4>(L, W, s) : launch_pair<float, 1>(L, W, s);
     if (e == hipSuccess && L.head_pass) e = p.vec == 4 ? launch_head<float, 4>(L, W, s) : launch_head<float, 1>(L, W, s);
     return e;
   }
-  e = p.vec == 8 ? launch_pair<uint16_t, 8>(L, W, cus, s) : launch_pair<uint16_t, 1>(L, W, cus, s);
+  e = p.vec == 8 ? launch_pair<uint16_t, 8>(L, W, s) : launch_pair<uint16_t, 1>(L, W, s);
   if (e == hipSuccess && L.head_pass) e = p.vec == 8 ? launch_head<uint16_t, 8>(L, W, s) : launch_head<uint16_t, 1>(L, W, s);
   return e;
 }
@@ -4808,7 +4807,7 @@ int tabby_sampler_sample_device(tabby_sampler *h, const void *logits_dev, int32_
   L.topk_ids = topk_ids_dev;
   L.topk_logits = topk_logits_dev;
   HIP_TRY(hipSetDevice(h->device));
-  HIP_TRY(dispatch(dtype, p, L, h->ws, h->cus, (hipStream_t)stream));
+  HIP_TRY(dispatch(dtype, p, L, h->ws, (hipStream_t)stream));
   return TABBY_OK;
 }
 
@@ -4985,7 +4984,7 @@ int tabby_sampler_sample_device_noalloc(const void *logits_dev, int32_t dtype, i
     return fail(TABBY_ECAPACITY, std::to_string(rows) + " rows of " + std::to_string(vocab) + " need " +
                                      std::to_string(off) + " bytes of scratch; the allocation-free entry has " +
                                      std::to_string(kNoAllocScratchBytes));
-  HIP_TRY(dispatch(dtype, p, L, W, cus, (hipStream_t)stream));
+  HIP_TRY(dispatch(dtype, p, L, W, (hipStream_t)stream));
   return TABBY_OK;
 }
 
