@@ -45,7 +45,7 @@ __device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
 // The composite of the first maximum among this lane's elements, scanned in index order with
 // the reference's strict `>`: a NaN never compares greater, so it is skipped. A lane whose
 // elements are all -inf or NaN offers -inf at an arbitrary index; the row's answer is then
-// decided without it (see row_answer).
+// decided without it (see write_answer).
 template <typename In, int VEC, int BLOCK>
 __device__ __forceinline__ uint64_t lane_first_max(const In *row, int begin, int end) {
   const int lane = (int)threadIdx.x;
@@ -90,14 +90,21 @@ __device__ __forceinline__ uint64_t lane_first_max(const In *row, int begin, int
   return composite(key_of(best), (uint32_t)at);
 }
 
-// The reference's answer from the row's largest composite: the composite's index, unless the
-// first entry is NaN (nothing compares greater than it, sampler.ts:14-18) or nothing in the
-// row lies above -inf (nothing compares greater than the first entry, -inf or NaN): then 0.
+// The reference's answer from the row's largest composite and its first entry: the composite's
+// index, unless the first entry is NaN (nothing compares greater than it, sampler.ts:14-18) or
+// nothing in the row lies above -inf (nothing compares greater than the first entry, -inf or NaN):
+// then 0. The value comes from the key, which leaves no load to wait for, except a zero's (the key
+// has no sign of zero).
 template <typename In>
-__device__ __forceinline__ int row_answer(const In *src, uint64_t best) {
-  const float first = load_one(src);
-  if (first != first || composite_key(best) <= kNegInfKey) return 0;
-  return (int)composite_index(best);
+__device__ __forceinline__ void write_answer(const In *src, float first, uint64_t best, int row, int32_t *ids,
+                                             float *max_logits) {
+  const bool none = first != first || composite_key(best) <= kNegInfKey;
+  const int id = none ? 0 : (int)composite_index(best);
+  ids[row] = id;
+  if (!max_logits) return;
+  float v = none ? first : value_of(composite_key(best));
+  if (v == 0.0f) v = load_one(src + id);
+  max_logits[row] = v;
 }
 
 template <typename In, int VEC, int BLOCK>
@@ -109,6 +116,7 @@ __global__ __launch_bounds__(BLOCK) void argmax_kernel(const In *logits, int voc
   const In *src = logits + (size_t)row * (size_t)vocab;
   const int begin = split * split_len;
   const int end = min(vocab, begin + split_len);
+  const float first = load_one(src);
   uint64_t c = lane_first_max<In, VEC, BLOCK>(src, begin, end);
   c = wave_max_u64(c);
   const int w = (int)threadIdx.x / kWaveSize;
@@ -118,30 +126,29 @@ __global__ __launch_bounds__(BLOCK) void argmax_kernel(const In *logits, int voc
     uint64_t b = wave_best[0];
 #pragma unroll
     for (int i = 1; i < BLOCK / kWaveSize; ++i) b = tmax(b, wave_best[i]);
-    if (splits == 1) {
-      const int id = row_answer(src, b);
-      ids[row] = id;
-      if (max_logits) max_logits[row] = load_one(src + id);
-    } else {
-      partial[(size_t)row * splits + split] = b;
-    }
+    if (splits == 1) write_answer(src, first, b, row, ids, max_logits);
+    else partial[(size_t)row * splits + split] = b;
   }
 }
 
-// One lane per row: the row's splits combined (largest composite), then the answer.
+// One wave per row, a lane per split. What bounds it is its chain of loads: the partials and the
+// row's first entry come in one round trip. 32 rows of 151,936 f32, a call that is waited for: 27.7
+// us, against 31.2 with a lane per row that read its partials, then the first entry, then the
+// answer's own; back to back 10.8 against 11.3, where two runs of one build differ by more.
+// (A row finished by the last of its workgroups to arrive, with no second launch, took 13.9 us:
+// the store, the count and the partials then wait on memory one after another.)
 template <typename In>
 __global__ __launch_bounds__(kArgBlock) void argmax_finish_kernel(const In *logits, int rows, int vocab, int splits,
                                                                   const uint64_t *partial, int32_t *ids,
                                                                   float *max_logits) {
-  const int row = (int)(blockIdx.x * kArgBlock + threadIdx.x);
+  static_assert(kArgMaxSplits <= kWaveSize, "a lane per split");
+  const int row = (int)(blockIdx.x * (kArgBlock / kWaveSize)) + (int)threadIdx.x / kWaveSize;
   if (row >= rows) return;
-  const uint64_t *p = partial + (size_t)row * splits;
-  uint64_t b = p[0];
-  for (int s = 1; s < splits; ++s) b = tmax(b, p[s]);
+  const int lane = wave_lane();
   const In *src = logits + (size_t)row * (size_t)vocab;
-  const int id = row_answer(src, b);
-  ids[row] = id;
-  if (max_logits) max_logits[row] = load_one(src + id);
+  const float first = load_one(src);
+  const uint64_t b = wave_max_u64(lane < splits ? partial[(size_t)row * splits + lane] : 0ull);
+  if (lane == 0) write_answer(src, first, b, row, ids, max_logits);
 }
 
 template <typename In, int VEC>
@@ -173,7 +180,7 @@ int launch_argmax(const HandleView &hv, const In *logits, int rows, int vocab, i
                      stream, logits, vocab, splits, split_len, partial, ids, max_logits);
   TABBY_HIP_CHECK(hipGetLastError());
   if (splits > 1) {
-    hipLaunchKernelGGL((argmax_finish_kernel<In>), dim3((unsigned)((rows + kArgBlock - 1) / kArgBlock)),
+    hipLaunchKernelGGL((argmax_finish_kernel<In>), dim3((unsigned)((rows * kWaveSize + kArgBlock - 1) / kArgBlock)),
                        dim3(kArgBlock), 0, stream, logits, rows, vocab, splits, partial, ids, max_logits);
     TABBY_HIP_CHECK(hipGetLastError());
   }

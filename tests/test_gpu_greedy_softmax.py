@@ -88,6 +88,32 @@ def test_argmax_f16(oracle, rows, vocab):
     assert np.array_equal(mx, wide[np.arange(rows), want])
 
 
+@pytest.mark.parametrize("dtype", ["f32", "f16"])
+@pytest.mark.parametrize("rows,vocab", [(1, 524289), (7, 4096), (9, 4097), (33, 151936), (255, 16384), (257, 5000)])
+def test_argmax_values(oracle, dtype, rows, vocab):
+    # One split to 64 per row and rows that fill no workgroup: the value comes with its bits, a
+    # zero's sign, infinities and denormals among them.
+    rng = np.random.default_rng(rows + vocab)
+    x = (-rng.integers(1, 9, (rows, vocab))).astype(np.float16 if dtype == "f16" else np.float32)
+    tops = [-0.0, 0.0, 6e-8, -6e-8, np.inf, -np.inf, np.nan, 2.5]
+    for r in range(rows):
+        top = tops[r % 8]
+        if np.isinf(top) and top < 0:
+            x[r] = -np.inf
+        elif np.isnan(top):
+            x[r, 0] = np.nan
+        else:
+            x[r, rng.integers(0, vocab, 3)] = top
+    print(f"argmax values rows={rows} vocab={vocab} {dtype}", flush=True)
+    ids, mx = _gpu_argmax(x, dtype)
+    wide = x.astype(np.float32)
+    want = np.array([oracle.argmax(wide[r]) for r in range(rows)])
+    assert np.array_equal(ids, want)
+    got, exact = mx.view(np.uint32), wide[np.arange(rows), want]
+    assert np.array_equal(np.isnan(mx), np.isnan(exact))
+    assert np.array_equal(got[~np.isnan(exact)], exact.view(np.uint32)[~np.isnan(exact)])
+
+
 def test_argmax_agrees_with_greedy_sampling(oracle):
     # The one-candidate pool's id (sampleFromTopK at T = 0) is the argmax.
     torch = _torch()
