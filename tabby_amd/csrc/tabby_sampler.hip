@@ -123,9 +123,10 @@ constexpr uint32_t kPoolRowDone = 0xffffffffu;
 // Per-row hand-over from the sampling kernel to the head kernel (whole-vocabulary rows).
 struct RowState {
   float max;
-  uint32_t head_key;  // elements with key >= head_key form the row's head
-  uint32_t store_key; // >= head_key: those with key >= store_key hold the cut and the draw, and lie
-                      // within 37.5 T of the max
+  uint32_t head_key;  // elements with key >= head_key form the row's head: those within 37.5 T of
+                      // the max, and the caller's top-k list
+  uint32_t weights_key;  // elements with key >= weights_key: those within 37.5 T of the max
+  uint32_t store_key; // >= weights_key: those with key >= store_key hold the cut and the draw
   double sum_exp;
   int32_t status;
   uint32_t handoff;   // bits 16..: length N of the row's sorted top list in head_sorted (0: none);
@@ -1193,6 +1194,7 @@ __global__ __launch_bounds__(kBlock) void pool_handoff_kernel(Launch L, Workspac
     rs.status = TABBY_OK;
     rs.handoff = (uint32_t)handed << 16;
     rs.head_key = min(weights_key, list_key);
+    rs.weights_key = weights_key;
     rs.store_key = store_threshold(st.max, P, L.vocab, 1.0, weights_key);
     W.row_state[row] = rs;
   }
@@ -1772,6 +1774,7 @@ __device__ __forceinline__ void finish_pool(WaveMergeSmem &sm, const Launch &L, 
       const uint32_t list_key = kt > 0 ? composite_key(sm.sorted[kt - 1]) : 0xffffffffu;
       const uint32_t weights_key = head_threshold(row_max, P.temperature);
       st.head_key = min(weights_key, list_key);
+      st.weights_key = weights_key;
       st.store_key = store_threshold(row_max, P, L.vocab, scaled, weights_key);
       W.row_state[row] = st;
     }
@@ -2636,10 +2639,11 @@ __device__ __forceinline__ double exp_sum_term(double y, const double *table) {
   return __longlong_as_double((long long)(bits + ((uint64_t)(uint32_t)(i >> 6) << 52)));
 }
 
-// One slice of a whole-vocabulary row: its weight, sum_i exp((l_i - M)/T) over its part of the
-// head (elements with key >= head_key; f64 exps, added per lane), and its entries with key >=
-// store_key, in the slice's range of the row's head buffer (a row's slices appending to one
-// counter serialised on it).
+// One slice of a whole-vocabulary row: its weight, sum_i exp((l_i - M)/T) over its elements with key
+// >= weights_key (f64 exps, added per lane; below that key a top-k list may reach past
+// exp_sum_term's range, to -inf, and no term changes the reference's sums), the size of its part of
+// the head, and its entries with key >= store_key, in the slice's range of the row's head buffer (a
+// row's slices appending to one counter serialised on it).
 //
 // What bounds it: the f64 exps of the whole head (64 rows of 151,936 at T = 1: every element),
 // taken by exp_sum_term in half the instructions of exp_nonpos. A slice with at most
@@ -2690,7 +2694,7 @@ __global__ __launch_bounds__(kWaveSize) void head_kernel(Launch L, Workspace W) 
   const tabby_row_params P = L.params[row];
   const RowState rs = W.row_state[row];
   if (!is_head_row(P, L) || rs.status != TABBY_OK || (rs.handoff & 1u)) return;
-  const float hv = value_of(rs.head_key), sv = value_of(rs.store_key);
+  const float hv = value_of(rs.head_key), wv = value_of(rs.weights_key), sv = value_of(rs.store_key);
   const double T = P.temperature, M = (double)rs.max;
   const bool weigh = !greedy_temp(T);
   const double inv_t = weigh ? 1.0 / T : 0.0;
@@ -2726,14 +2730,14 @@ __global__ __launch_bounds__(kWaveSize) void head_kernel(Launch L, Workspace W) 
   wave_lds_sync();  // the table and the cleared bins
   uint64_t *head = W.head + (size_t)row * W.head_stride + begin;
   double sum = 0.0;
-  // The weights of S elements of each lane that lie in the head (value(e); NaN: none).
+  // The weights of S elements of each lane (value(e); below wv or NaN: none).
   auto weigh_head = [&](auto steps, auto value) {
     constexpr int S = decltype(steps)::value;
     if (!weigh) return;
 #pragma unroll
     for (int e = 0; e < S; ++e) {
       const double term = exp_sum_term(((double)value(e) - M) * per_unit, exp_table);
-      sum += value(e) >= hv ? term : 0.0;
+      sum += value(e) >= wv ? term : 0.0;
     }
   };
   // The entries among them, at local(e): in bin order with the slice's table, or as they come.
@@ -3539,6 +3543,9 @@ __device__ __forceinline__ bool head_pick(PickSmem &sm, const Launch &L, const W
     considered = top_p < 1.0 && run.total >= top_p ? (uint32_t)run.count : (uint32_t)L.vocab;
     return true;
   }
+  // S holds the max's own weight, 1; a total that does not comes from a T whose reciprocal is not
+  // finite.
+  if (!(S >= 0.99) || !(S < 1.0e30)) return false;
   const bool cuts = top_p < 1.0;
   const double M = (double)rs.max, inv_t = 1.0 / T;
   auto search = [&](const Stored &stored, const PickBin &pb, auto bin_entries_of) {

@@ -651,6 +651,41 @@ def test_full_vocab_selection(oracle, dtype, vocab, k_max, topk_cap):
          compare(w, res, ids, vals, run_oracle(oracle, w, topk_cap), topk_cap))
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("topk_cap,k_max", [(40, 64), (100, 256), (256, 256), (100, 1024), (300, 1024)])
+def test_full_vocab_cold_rows_with_lists(oracle, dtype, topk_cap, k_max):
+    # Cold whole-vocabulary rows whose top-k list reaches far below the entries that have a weight
+    # (scaled logits of -700 to -7,000, and -inf), so the row's total weight is of a part of what it
+    # collects. The maxima are tied or nearly so and the uniforms draw the later ones; tied list ends
+    # lengthen short lists; some rows have fewer finite entries than the list.
+    rows, vocab = 36, 6000
+    w = synth.random_workload(rows=rows, vocab=vocab, seed=901 + topk_cap, k_choices=(0,), temperatures=(0.01,),
+                              top_ps=(1.0,), sigma=6.0)
+    rng = np.random.default_rng(topk_cap + k_max)
+    for r in range(rows):
+        row = w.logits[r]
+        kind = r % 3
+        if kind == 1:    # a list ending in a tie of 150
+            row[rng.choice(vocab, 150, replace=False)] = np.ceil(np.sort(row)[-30]) if r % 2 else row.max() - 8.0
+        elif kind == 2:  # thirty finite entries
+            keep = rng.choice(vocab, 30, replace=False)
+            kept = row[keep].copy()
+            row[:] = -np.inf
+            row[keep] = kept
+        T = (0.005, 0.01, 0.02, 0.002)[(r // 3) % 4]
+        top = np.float32(np.ceil(row.max()) + 1.0)
+        at = np.sort(rng.choice(vocab, 3, replace=False))
+        row[at] = top if dtype == np.float16 else [top, np.float32(top - 0.2 * T), np.float32(top - 0.5 * T)]
+        w.temperature[r] = T
+        w.top_p[r] = (1.0, 0.9, np.nan)[(r // 12) % 3]
+        w.uniform[r] = (0.9, 0.45, 0.1, 0.6)[r % 4]
+    w.logits = w.logits.astype(dtype)
+    print(f"cold rows with lists cap={topk_cap} k_max={k_max} {dtype.__name__}", flush=True)
+    res, ids, vals = run_gpu(w, k_max=k_max, topk_cap=topk_cap)
+    _log(f"full vocab cold rows with lists {dtype.__name__} cap={topk_cap} k_max={k_max}",
+         compare(w, res, ids, vals, run_oracle(oracle, w, topk_cap), topk_cap))
+
+
 def test_full_vocab_rejects_list_above_k_max():
     import torch
     x = torch.zeros(1, 5000, device="cuda")
