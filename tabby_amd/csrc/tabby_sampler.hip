@@ -755,19 +755,23 @@ __device__ __forceinline__ Pruned wave_prune_any(WaveSmem &sm, int count, int kk
   return wave_prune<8>(sm, count, kk, floor_key);
 }
 
-// Registers per lane (1, 2, 4 or 8) for the union of the row's published lane-maximum keys:
-// each of `waves` waves publishes m = min(64, 64 * regs / waves) keys, and the union must hold
-// at least kk keys of the `live` waves that have a chunk (kk <= 256 here; 8 always suffices for 5
-// to 16 live waves). Counting the idle waves' keys too, a part of 11 chunks on 16 waves
-// published 44 keys for k = 50: no bound, every element a candidate (one row of 50,257 in four
-// parts 26.7 us a call; now 13.8).
-__device__ __forceinline__ int bound_regs(int kk, int waves, int live) {
+// Keys that each of the `live` waves that have a chunk publishes for the row's first bound, their
+// union being sorted in `regs` registers per lane, and the smallest regs (1, 2, 4 or 8) whose union
+// holds at least kk keys (kk <= 256 here; 8 always suffices for 4 to 16 live waves: a wave has 64
+// keys to publish). Waves with no chunk take no part: with their keys counted and their share of the
+// union kept for them, a part of 11 chunks on 16 waves published 44 keys for k = 50, so that it had
+// no bound and every element was a candidate (one row of 50,257 in four parts 26.7 us a call, 13.8
+// now), and 5 chunks on 8 waves published 40, eight a wave: too few of a wave that holds most of
+// a masked row's entries.
+__device__ __forceinline__ int bound_share(int regs, int live) { return min(kWaveSize, kWaveSize * regs / live); }
+__device__ __forceinline__ int bound_regs(int kk, int live) {
   for (int r = 1; r < 8; r *= 2)
-    if (live * min(kWaveSize, kWaveSize * r / waves) >= kk) return r;
+    if (live * bound_share(r, live) >= kk) return r;
   return 8;
 }
 
-// The kk-th largest (1 <= kk <= total <= 64 * R) of keys[0..total), on every lane.
+// The kk-th largest (1 <= kk, total <= 64 * R) of keys[0..total), on every lane; 0, below every key,
+// when there are fewer.
 template <int R>
 __device__ __forceinline__ uint32_t union_kth(const uint32_t *keys, int total, int kk, uint32_t &largest) {
   uint32_t v[R];
@@ -972,14 +976,15 @@ __device__ __forceinline__ void wave_slice(WaveSmem &sm, const Launch &L, const 
     int b = next();
     rd.load(b, y);
     // The row's first bound, shared by its waves. A wave's 64 lane maxima over its first two
-    // chunks are 64 distinct elements of the row; each wave publishes its m largest, and the
-    // kk-th largest of the union (waves * m >= kk keys) has kk distinct elements at or above
+    // chunks are 64 distinct elements of the row; each wave with a chunk publishes its m largest, and
+    // the kk-th largest of the union (no bound if it holds fewer) has kk distinct elements at or above
     // it, so it never exceeds the row's kk-th largest. (The union is much tighter than any
     // one wave's offer: the row's top lane maxima are spread over the waves.) Every wave
     // passes the barrier once and computes the same bound.
     if (kk > 0) {
-      const int regs = bound_regs(kk, waves, min(waves, nchunks));
-      const int m = min(kWaveSize, kWaveSize * regs / waves);
+      const int live = min(waves, nchunks);
+      const int regs = bound_regs(kk, live);
+      const int m = bound_share(regs, live);
       float cm = -INFINITY;
       if (a < nchunks) {
         if (a >= full_chunks) {
@@ -1001,14 +1006,14 @@ __device__ __forceinline__ void wave_slice(WaveSmem &sm, const Launch &L, const 
       }
       uint32_t k1[1] = {key_of(cm)};
       wave_sort_desc<1>(k1);
-      if (wave_lane() < m) bound_keys[slice * m + wave_lane()] = min(max(k1[0], kNegInfKey), 0xff800000u);
+      if (slice < live && wave_lane() < m) bound_keys[slice * m + wave_lane()] = min(max(k1[0], kNegInfKey), 0xff800000u);
       __syncthreads();
       uint32_t t;
       switch (regs) {
-        case 1: t = union_kth<1>(bound_keys, waves * m, kk, union_top); break;
-        case 2: t = union_kth<2>(bound_keys, waves * m, kk, union_top); break;
-        case 4: t = union_kth<4>(bound_keys, waves * m, kk, union_top); break;
-        default: t = union_kth<8>(bound_keys, waves * m, kk, union_top); break;
+        case 1: t = union_kth<1>(bound_keys, live * m, kk, union_top); break;
+        case 2: t = union_kth<2>(bound_keys, live * m, kk, union_top); break;
+        case 4: t = union_kth<4>(bound_keys, live * m, kk, union_top); break;
+        default: t = union_kth<8>(bound_keys, live * m, kk, union_top); break;
       }
       theta_key = max(theta_key, t);
       theta = value_of(theta_key);
