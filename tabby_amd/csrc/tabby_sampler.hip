@@ -177,6 +177,7 @@ struct Launch {
   int32_t kcap;      // largest pool the sampling kernel finishes itself
   int32_t head_pass; // 1 when the head kernels run after this launch
   int32_t h_splits;  // slices per row of the head kernel
+  int32_t sort_groups;  // workgroups per row of head_sort_kernel
   int32_t h_slice_len;
   int32_t parts;      // row_kernel: 1 = one workgroup per row; > 1 = workgroups per row (each
                       // a part of slice_len elements, finished by wave_merge_kernel); 0 = unused
@@ -2963,8 +2964,12 @@ __device__ __forceinline__ void plan_head(PlanSmem &sm, const Launch &L, const W
   }
 }
 
+// Eight waves: 16 rows of 32,000 equal logits took 2.00 ms with four, 1.80 with eight.
+constexpr int kSortWaves = 8;
+constexpr int kSortThreads = kSortWaves * kWaveSize;
+
 struct SortSmem {
-  BlockScratch bs;
+  BlockScratchT<kSortWaves> bs;
   uint32_t hist[kBins];
   uint64_t buf[kSegLds];
 };
@@ -2993,7 +2998,7 @@ __device__ __forceinline__ void sort_segment(SortSmem &sm, const Launch &L, cons
   double *part = W.head_part + ((size_t)row * slots_max + g) * 2;
   auto terms = [&](const uint64_t *src) {
     double pool_part = 0.0, e_part = 0.0;
-    for (int i = threadIdx.x; i < n; i += kBlock) {
+    for (int i = threadIdx.x; i < n; i += kSortThreads) {
       const double d = (double)value_of(composite_key(src[i])) - (double)rs.max;
       // poolMass and the head's share of sum-exp are compared within 1e-5: an f32 exp2 will
       // do (the exact V8 exp is kept for the weights, which decide the draw).
@@ -3011,10 +3016,10 @@ __device__ __forceinline__ void sort_segment(SortSmem &sm, const Launch &L, cons
   };
   if (n <= kSegLds) {
     const int npow = next_pow2(n);
-    for (int i = threadIdx.x; i < npow; i += kBlock) sm.buf[i] = i < n ? seg[i] : 0ull;
+    for (int i = threadIdx.x; i < npow; i += kSortThreads) sm.buf[i] = i < n ? seg[i] : 0ull;
     __syncthreads();
-    if (n > 1) block_sort_desc(sm.buf, npow);
-    for (int i = threadIdx.x; i < n; i += kBlock) seg[i] = sm.buf[i];
+    if (n > 1) block_sort_desc<kSortWaves>(sm.buf, npow);
+    for (int i = threadIdx.x; i < n; i += kSortThreads) seg[i] = sm.buf[i];
     terms(sm.buf);
     return;
   }
@@ -3029,11 +3034,11 @@ __device__ __forceinline__ void sort_segment(SortSmem &sm, const Launch &L, cons
     __syncthreads();
     auto below = [&](auto &&f) {
       constexpr int B = 8;
-      for (int base = 0; base < n; base += B * kBlock) {
+      for (int base = 0; base < n; base += B * kSortThreads) {
         uint64_t v[B];
 #pragma unroll
         for (int u = 0; u < B; ++u) {
-          const int i = base + u * kBlock + (int)threadIdx.x;
+          const int i = base + u * kSortThreads + (int)threadIdx.x;
           v[u] = i < n ? seg[i] : ~0ull;
         }
 #pragma unroll
@@ -3055,26 +3060,26 @@ __device__ __forceinline__ void sort_segment(SortSmem &sm, const Launch &L, cons
       });
     }
     const int npow = next_pow2(b);
-    for (int i = b + (int)threadIdx.x; i < npow; i += kBlock) sm.buf[i] = 0ull;
+    for (int i = b + (int)threadIdx.x; i < npow; i += kSortThreads) sm.buf[i] = 0ull;
     __syncthreads();
-    block_sort_desc(sm.buf, npow);
-    for (int i = threadIdx.x; i < b; i += kBlock) out[pos + i] = sm.buf[i];
+    block_sort_desc<kSortWaves>(sm.buf, npow);
+    for (int i = threadIdx.x; i < b; i += kSortThreads) out[pos + i] = sm.buf[i];
     upper = sm.buf[b - 1];
     pos += b;
     __syncthreads();
   }
-  for (int i = threadIdx.x; i < n; i += kBlock) seg[i] = out[i];
+  for (int i = threadIdx.x; i < n; i += kSortThreads) seg[i] = out[i];
   terms(out);
 }
 
-// Heads up to this many entries run their sums from LDS (padded, no more than the sort's
-// buffer); larger ones from global memory.
-constexpr int kHeadLds = 7168;
+// Heads up to this many entries run their sums from LDS (padded, 139 KB of the 160 KB a gfx950
+// workgroup may use); larger ones from global memory (16 rows of 12,000 equal logits: 656 us from
+// global memory, 562 from LDS; a launch that finds no row to sort takes the same).
+constexpr int kHeadLds = 16384;
 
-constexpr int kFinishThreads = kBlock;  // four waves: the sums take 4,096 terms per step
+constexpr int kFinishThreads = kSortThreads;  // the sums take 8,192 terms per step
 
 struct HeadSmem {
-  BlockScratch bs;
   SeqScratch<kFinishThreads / kWaveSize> ss;
   double pool, e;
   int cut;
@@ -3221,10 +3226,12 @@ __device__ __forceinline__ void head_finish(HeadSmem &sm, const Launch &L, const
   }
 }
 
-// Workgroups per row of head_sort_kernel; each sorts every kSortGroups-th segment. (One per
-// segment slot cost 7.5 us on 64 rows of 151,936 when no row needed a sort: 171 slots per row,
-// each workgroup reserving 66 KB of LDS.)
-constexpr int kSortGroups = 8;
+// Workgroups per row of head_sort_kernel; each sorts every sort_groups-th segment. At most eight (one
+// per segment slot cost 7.5 us on 64 rows of 151,936 when no row needed a sort: 171 slots per row,
+// each workgroup reserving its LDS), and no more in all than run at once, one to a CU: the last of a
+// row's workgroups to arrive finishes the row, and holds a place that another row's wait for (300
+// rows of 5,000 equal logits: 1,461 us in eight each, 580 in one; 64: 421 and, in four, 320).
+static int sort_groups(int rows, int cus) { return std::max(1, std::min(8, cus / rows)); }
 
 // The rows head_pick_kernel left (plan[0] > 0): the head's segments sorted, then the row's tail
 // by the last of its workgroups to arrive -- one launch, as in nearly every call no row is left
@@ -3235,16 +3242,19 @@ union SortedSmem {
 };
 
 template <typename In>
-__global__ __launch_bounds__(kBlock) void head_sort_kernel(Launch L, Workspace W) {
+__global__ __launch_bounds__(kSortThreads) void head_sort_kernel(Launch L, Workspace W) {
   __shared__ __align__(16) unsigned char raw[sizeof(SortedSmem)];
   __shared__ int last;
-  const int row = (int)blockIdx.x / kSortGroups;
-  const int first = (int)blockIdx.x - row * kSortGroups;
+  const int row = (int)blockIdx.x / L.sort_groups;
+  // Rotated by row: a head that is one segment long is sorted, and mostly finished, by the workgroup
+  // that takes segment 0, and eight workgroups per row put them all on one XCD (64 rows of 5,000 equal
+  // logits took 498 us, with four workgroups each and rotated 320).
+  const int first = ((int)blockIdx.x + row) % L.sort_groups;
   const uint32_t *plan = W.head_plan + (size_t)row * W.plan_stride;
   const int slots = (int)plan[0];
   if (slots == 0) return;  // the row is finished (or has no head): every workgroup of it ends here
   SortSmem &sort = *reinterpret_cast<SortSmem *>(raw);
-  for (int g = first; g < slots; g += kSortGroups) {
+  for (int g = first; g < slots; g += L.sort_groups) {
     sort_segment(sort, L, W, row, g, slots, plan);
     __syncthreads();  // `sort` is reused by the next segment
   }
@@ -3253,7 +3263,7 @@ __global__ __launch_bounds__(kBlock) void head_sort_kernel(Launch L, Workspace W
   __syncthreads();
   if (threadIdx.x == 0)
     last = __hip_atomic_fetch_add(W.head_arrived + row, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
-                   (uint32_t)(kSortGroups - 1)
+                   (uint32_t)(L.sort_groups - 1)
                ? 1
                : 0;
   __syncthreads();
@@ -3720,7 +3730,7 @@ __global__ __launch_bounds__(kWaveSize) void seq_sum_kernel(const double *t, int
   if (wave_lane() == 0) *count = r.count;
 }
 
-// The same by a workgroup of NW waves (block_seq_sum_wide; head_sort_kernel runs NW = 4).
+// The same by a workgroup of NW waves (block_seq_sum_wide; head_sort_kernel runs NW = 8).
 template <int NW>
 __global__ __launch_bounds__(NW * kWaveSize) void seq_sum_block_kernel(const double *t, int32_t n, double stop_at,
                                                                        double *out, int32_t *count) {
@@ -4543,7 +4553,7 @@ hipError_t launch_head(const Launch &L, const Workspace &W, hipStream_t stream) 
   hipLaunchKernelGGL((head_kernel<In, VEC>), dim3((unsigned)(L.rows * L.h_splits)), dim3(kWaveSize), 0,
                      stream, L, W);
   hipLaunchKernelGGL((head_pick_kernel<In>), dim3((unsigned)L.rows), dim3(kPlanThreads), 0, stream, L, W);
-  hipLaunchKernelGGL((head_sort_kernel<In>), dim3((unsigned)(L.rows * kSortGroups)), dim3(kBlock), 0, stream, L, W);
+  hipLaunchKernelGGL((head_sort_kernel<In>), dim3((unsigned)(L.rows * L.sort_groups)), dim3(kSortThreads), 0, stream, L, W);
   return hipGetLastError();
 }
 
@@ -4578,6 +4588,7 @@ Plan plan_launch(int rows, int vocab, int dtype, const void *logits, int k_max, 
   L.head_pass = head_pass ? 1 : 0;
   L.h_slice_len = kHeadSlice;
   L.h_splits = (vocab + kHeadSlice - 1) / kHeadSlice;
+  L.sort_groups = sort_groups(rows, cus);
   L.parts = 0;
   L.row_waves = 0;
   if (kcap > kWaveKcap) {
