@@ -42,6 +42,8 @@ namespace {
 
 constexpr int kSmWaves = 4;  // rows per workgroup, one wave each
 constexpr int kBlockMinRows = 256;       // rows of up to 512 entries: a lane adds a row from here on
+constexpr int kTinyCols = 64;            // one group of one entry per lane
+constexpr int kElementCols = 384;        // one entry per lane at a time up to here
 constexpr int kBlockMinLongRows = 1024;  // rows of 513-1,024 entries
 constexpr int kChunkCols = 16384;        // longest row held in a workgroup's registers
 constexpr double kTwo24 = 16777216.0;
@@ -421,13 +423,21 @@ __global__ __launch_bounds__(NW == 1 ? kSmWaves * kWaveSize : NW * kWaveSize) vo
 // element loads and stores and the exps read back from LDS. 14 x 1,024 of 1,024 (88 MB): 27.4
 // us, by chunks 33.0, in steps of 256 73. Eight rows per workgroup took 33 us there: fewer
 // workgroups of a CU are then in different phases.
-template <int COLS>
+//
+// VEC: consecutive entries per lane. Four (16-byte loads and stores) take the row in groups of 256,
+// whose exps -- what the kernel issues most of -- cost the same however few of them lie in the row;
+// one takes it in groups of 64. 28,672 rows of 32, 128, 257 and 384 entries: 14.4, 16.6, 26.0 and
+// 26.8 us by fours, 7.9, 12.6, 22.8 and 25.6 by ones (rows of up to 64 in a tile of their own that
+// reads eight entries ahead: 9.6 in the tile of 512); of 448: 28.0 against 28.9.
+template <int COLS, int VEC>
 __global__ __launch_bounds__(kSmWaves *kWaveSize) void softmax_rows_block_kernel(const float *x, float *out,
                                                                                  RowDims d) {
   // Row pitch: four pad words put the four rows the sum reads at once on different banks.
   constexpr int kPitch = COLS + 4;
-  constexpr int kGroups = COLS / 256;
-  constexpr int kStep = 32;  // entries the sum reads ahead of its adds
+  constexpr int kGroup = VEC * kWaveSize;
+  constexpr int kGroups = COLS / kGroup;
+  static_assert(kGroups * VEC <= 32, "a bit per entry of a lane");
+  constexpr int kStep = COLS <= kTinyCols ? 8 : 32;  // entries the sum reads ahead of its adds
   __shared__ __align__(16) float tile[kSmWaves * kPitch + kStep];
   __shared__ float inv[kSmWaves];
   const int lane = wave_lane();
@@ -437,18 +447,18 @@ __global__ __launch_bounds__(kSmWaves *kWaveSize) void softmax_rows_block_kernel
   const int row = row0 + wave;
   const int valid = wave < rows ? valid_of(d, row) : 0;
   const float *src = x + (size_t)row * d.row_len;
-  float *mine = tile + wave * kPitch + 4 * lane;
-  float v[kGroups][4];
+  float *mine = tile + wave * kPitch + VEC * lane;
+  float v[kGroups][VEC];
 #pragma unroll
   for (int k = 0; k < kGroups; ++k) {
-    const int i = 4 * (k * kWaveSize + lane);
-    if (i + 4 <= valid) {
+    const int i = k * kGroup + VEC * lane;
+    if (VEC == 4 && i + VEC <= valid) {
       const sm_f32x4u f = __builtin_nontemporal_load(reinterpret_cast<const sm_f32x4u *>(src + i));
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[k][j] = f[j];
+      for (int j = 0; j < VEC; ++j) v[k][j] = f[j];
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) v[k][j] = i + j < valid ? src[i + j] : -INFINITY;
+      for (int j = 0; j < VEC; ++j) v[k][j] = i + j < valid ? src[i + j] : -INFINITY;
     }
   }
   float mx = -INFINITY;
@@ -456,7 +466,7 @@ __global__ __launch_bounds__(kSmWaves *kWaveSize) void softmax_rows_block_kernel
 #pragma unroll
   for (int k = 0; k < kGroups; ++k)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < VEC; ++j) {
       mx = fmaxf(mx, v[k][j]);
       nan |= v[k][j] != v[k][j];
     }
@@ -465,36 +475,39 @@ __global__ __launch_bounds__(kSmWaves *kWaveSize) void softmax_rows_block_kernel
   uint32_t slow = 0u;
 #pragma unroll
   for (int k = 0; k < kGroups; ++k) {
-    if (k * 256 < valid) {  // uniform: groups past a causal prefix cost nothing
+    if (k * kGroup < valid) {  // uniform: groups past the row's end or its causal prefix cost nothing
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
+      for (int j = 0; j < VEC; ++j) {
         const float a = v[k][j] - mx;
         bool s;
         const float e = exp_to_f32_fast(a, s);
-        const bool in = 4 * (k * kWaveSize + lane) + j < valid;
-        slow |= in && s ? 1u << (4 * k + j) : 0u;
+        const bool in = k * kGroup + VEC * lane + j < valid;
+        slow |= in && s ? 1u << (VEC * k + j) : 0u;
         v[k][j] = !in ? 0.0f : s ? a : e;
       }
-      *reinterpret_cast<sm_f32x4 *>(mine + k * 256) = sm_f32x4{v[k][0], v[k][1], v[k][2], v[k][3]};
+      if constexpr (VEC == 4) {
+        *reinterpret_cast<sm_f32x4 *>(mine + k * kGroup) = sm_f32x4{v[k][0], v[k][1], v[k][2], v[k][3]};
+      } else {
+        mine[k * kGroup] = v[k][0];
+      }
     }
   }
   if (__ballot(slow != 0u)) {  // V8's method, once for all entries, through LDS
     for (uint32_t b = slow; b != 0u; b &= b - 1u) {
       const int k = __ffs((int)b) - 1;
-      float *at = mine + (k >> 2) * 256 + (k & 3);
+      float *at = mine + (k / VEC) * kGroup + k % VEC;
       *at = exp_to_f32_slow(*at);
     }
 #pragma unroll
     for (int k = 0; k < kGroups; ++k)
-      if (k * 256 < valid) {
-        const sm_f32x4 f = *reinterpret_cast<const sm_f32x4 *>(mine + k * 256);
+      if (k * kGroup < valid) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[k][j] = f[j];
+        for (int j = 0; j < VEC; ++j) v[k][j] = mine[k * kGroup + j];
       }
   }
   __syncthreads();
   if (wave == 0 && lane < rows) {
-    // The row's exps left to right (zeros past its end change nothing); the next 32 are read
+    // The row's exps left to right (zeros past its end change nothing); the next kStep are read
     // while these are added.
     const int n = valid_of(d, row0 + lane);
     const sm_f32x4 *t4 = reinterpret_cast<const sm_f32x4 *>(tile + lane * kPitch);
@@ -522,16 +535,20 @@ __global__ __launch_bounds__(kSmWaves *kWaveSize) void softmax_rows_block_kernel
   float *dst = out + (size_t)row * d.row_len;
 #pragma unroll
   for (int k = 0; k < kGroups; ++k) {
-    const int i = 4 * (k * kWaveSize + lane);
-    sm_f32x4u o;
+    const int i = k * kGroup + VEC * lane;
+    if constexpr (VEC == 4) {
+      sm_f32x4u o;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o[j] = i + j < valid ? v[k][j] * q : 0.0f;
-    if (i + 4 <= d.row_len) {
-      __builtin_nontemporal_store(o, reinterpret_cast<sm_f32x4u *>(dst + i));
+      for (int j = 0; j < 4; ++j) o[j] = i + j < valid ? v[k][j] * q : 0.0f;
+      if (i + 4 <= d.row_len) {
+        __builtin_nontemporal_store(o, reinterpret_cast<sm_f32x4u *>(dst + i));
+      } else {
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+          if (i + j < d.row_len) dst[i + j] = o[j];
+      }
     } else {
-#pragma unroll
-      for (int j = 0; j < 3; ++j)
-        if (i + j < d.row_len) dst[i + j] = o[j];
+      if (i < d.row_len) __builtin_nontemporal_store(i < valid ? v[k][0] * q : 0.0f, dst + i);
     }
   }
 }
@@ -616,13 +633,16 @@ extern "C" int tabby_softmax_rows_device(const float *x_dev, float *out_dev, int
   const dim3 grid((unsigned)((n_rows + kSmWaves - 1) / kSmWaves)), block(kSmWaves * kWaveSize);
   // Rows of up to kChunkCols entries are held in registers from the load to the store; longer
   // ones take three passes. Enough rows to fill the chip share the instructions of their sums
-  // (softmax_rows_block_kernel, four rows per wave's adds), up to 1,024 entries: 14 x 1,024
+  // (softmax_rows_block_kernel, four rows per wave's adds; an entry per lane at a time up to
+  // kElementCols, four beyond), up to 1,024 entries: 14 x 1,024
   // causal rows of 1,024 took 27.4 us against 33.0 by chunks, but 280 rows of 920 took 9.6 us
   // against 7.1, and 14 x 512 rows of 2,048 took 44.2 us (with room for 2,048) against 41.7.
   if (row_len <= 512 && n_rows >= kBlockMinRows) {
-    hipLaunchKernelGGL(softmax_rows_block_kernel<512>, grid, block, 0, s, x_dev, out_dev, d);
+    if (row_len <= kTinyCols) hipLaunchKernelGGL((softmax_rows_block_kernel<kTinyCols, 1>), grid, block, 0, s, x_dev, out_dev, d);
+    else if (row_len <= kElementCols) hipLaunchKernelGGL((softmax_rows_block_kernel<512, 1>), grid, block, 0, s, x_dev, out_dev, d);
+    else hipLaunchKernelGGL((softmax_rows_block_kernel<512, 4>), grid, block, 0, s, x_dev, out_dev, d);
   } else if (row_len <= 1024 && n_rows >= kBlockMinLongRows) {
-    hipLaunchKernelGGL(softmax_rows_block_kernel<1024>, grid, block, 0, s, x_dev, out_dev, d);
+    hipLaunchKernelGGL((softmax_rows_block_kernel<1024, 4>), grid, block, 0, s, x_dev, out_dev, d);
   } else if (row_len <= 512) {
     launch_chunks<1, 2>(x_dev, out_dev, d, s);
   } else if (row_len <= 1024) {

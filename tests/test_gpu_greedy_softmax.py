@@ -265,6 +265,13 @@ def test_softmax_chunk_edges(oracle, n_rows, row_len):
     _check_softmax(oracle, x, n_rows, row_len, period, 0)         # short causal prefixes
 
 
+@pytest.mark.parametrize("row_len", [1, 2, 7, 8, 9, 63, 64, 65, 128, 193, 256, 257, 383, 384, 385, 511, 512])
+def test_softmax_short_row_edges(oracle, row_len):
+    # Batches of short rows, a lane adding each: one entry per lane at a time up to 384 (a tile of its
+    # own up to 64), four beyond, on the same inputs.
+    test_softmax_chunk_edges(oracle, 259, row_len)
+
+
 def test_softmax_special_rows(oracle):
     row_len = 300
     x = np.random.default_rng(9).normal(0, 1, (6, row_len)).astype(np.float32)
