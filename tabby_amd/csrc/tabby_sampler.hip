@@ -1170,9 +1170,10 @@ __device__ __forceinline__ uint32_t store_threshold(float row_max, const tabby_r
 // ---------------------------------------------------------------------------------------
 // A head pass's whole-vocabulary rows in a batch of large pools (pool_row_kernel ends every
 // other row): the row's top Nw = max(topk_cap, kHeadList) (slice_keep), unsorted in its
-// candidate region, sorted; its statistics, head key and, when Nw fits a wave's register sort
-// (<= 256), the list handed on to head_kernel and head_pick_kernel, as from finish_pool. The
-// head also covers the caller's top-k list, the first topk_cap of them.
+// candidate region, sorted; its statistics, head key and the list handed on to head_kernel and
+// head_pick_kernel, as from finish_pool. The head also covers the caller's top-k list, the first
+// topk_cap of them. (A list of more than 256 was not handed on for a while, which left the row to the
+// sorted head: 64 rows of 151,936, T 0.3, a list of 300, 176 us; now 48.)
 // ---------------------------------------------------------------------------------------
 __global__ __launch_bounds__(kBlock) void pool_handoff_kernel(Launch L, Workspace W) {
   __shared__ uint64_t sorted[kKcapLarge];
@@ -1187,7 +1188,7 @@ __global__ __launch_bounds__(kBlock) void pool_handoff_kernel(Launch L, Workspac
   __syncthreads();
   if (npow > 1) block_sort_desc(sorted, npow);
   const int Nw = min(max(L.topk_cap, kHeadList), L.vocab);
-  const int handed = Nw <= kWaveKcap && C >= Nw ? Nw : 0;
+  const int handed = C >= Nw ? Nw : 0;
   uint64_t *list = W.head_sorted + (size_t)row * W.head_stride;
   for (int i = threadIdx.x; i < handed; i += kBlock) list[i] = sorted[i];
   if (threadIdx.x == 0) {
@@ -3315,7 +3316,7 @@ struct PickSmem {
   uint32_t wave_n[kPlanWaves], wave_h[kPlanWaves], wave_c[kPlanWaves];
   double wave_s[kPlanWaves];
   uint64_t list[kPickList];
-  uint64_t top[kWaveKcap];  // the merge's sorted list
+  uint64_t top[kKcapLarge];  // the merge's sorted list
   int first;
   uint32_t slot;
   double before, through;
@@ -3658,21 +3659,21 @@ __global__ __launch_bounds__(kPlanThreads) void head_pick_kernel(Launch L, Works
   const tabby_row_params P = L.params[row];
   const RowState rs = W.row_state[row];
   // Requested with them: every head slice's counts and weight (one slice per thread) and the
-  // merge's top list (its first kWaveKcap slots, of which the row state then says how many hold
-  // it).
+  // merge's top list (its first kcap slots, of which the row state then says how many hold it).
   const size_t slices = (size_t)row * W.acc_stride;
   const bool slice = tid < L.h_splits;
   const uint32_t c = slice ? W.head_slice_count[2 * (slices + tid)] : 0u;
   const uint32_t c_head = slice ? W.head_slice_count[2 * (slices + tid) + 1] : 0u;
   const double slice_sum = slice ? W.head_slice_sum[slices + tid] : 0.0;
-  const uint64_t listed = tid < kWaveKcap && tid < W.head_stride ? W.head_sorted[(size_t)row * W.head_stride + tid] : 0ull;
+  const uint64_t listed = tid < L.kcap && tid < W.head_stride ? W.head_sorted[(size_t)row * W.head_stride + tid] : 0ull;
   if (!is_head_row(P, L) || rs.status != TABBY_OK || (rs.handoff & 1u)) {
     if (tid == 0) plan[0] = 0u;
     return;
   }
   const int N = (int)(rs.handoff >> 16);
-  const bool has_list = N > 0 && N <= kWaveKcap;
-  if (has_list && tid < N) sm.top[tid] = listed;
+  static_assert(kKcapLarge <= kPlanThreads, "an entry of the list per thread");
+  const bool has_list = N > 0;
+  if (tid < N) sm.top[tid] = listed;
   // The head's size and weight.
   const uint32_t h_incl = wave_inclusive_scan_u32(c_head), c_incl = wave_inclusive_scan_u32(c);
   const double s_wave = wave_sum(slice_sum);

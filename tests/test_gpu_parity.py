@@ -652,6 +652,13 @@ def test_full_vocab_selection(oracle, dtype, vocab, k_max, topk_cap):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("vocab,topk_cap", [(2049, 257), (40001, 1024)])
+def test_full_vocab_selection_long_lists(oracle, dtype, vocab, topk_cap):
+    # The same rows with lists of more than 256, handed on whole by pool_handoff_kernel.
+    test_full_vocab_selection(oracle, dtype, vocab, 1024, topk_cap)
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
 @pytest.mark.parametrize("topk_cap,k_max", [(40, 64), (100, 256), (256, 256), (100, 1024), (300, 1024)])
 def test_full_vocab_cold_rows_with_lists(oracle, dtype, topk_cap, k_max):
     # Cold whole-vocabulary rows whose top-k list reaches far below the entries that have a weight
