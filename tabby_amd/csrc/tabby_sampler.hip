@@ -3794,6 +3794,11 @@ constexpr int kPoolBoundKeys = 4 * kPoolThreads;
 // Rows of at least this many chunks (the sample then at most a quarter of the row) stream at a
 // guessed first bound (pool_row_kernel).
 constexpr int kPoolGuessChunks = 128;
+// Rows of at most this many elements have no first bound. One row of 1,025, k = 300: 24.6 us with a
+// bound, 15.1 without (18.4 in the two kernels that served few rows before); of 2,000, k = 1,000 23.9 and
+// 14.9; of 5,000 22.7 and 20.3; of 6,144 20.3 and 20.9, of 8,192 19.8 and 21.6.
+constexpr int kPoolAllRow = 5 * kWChunk;
+static_assert(kPoolAllRow <= kPoolListCap, "their candidates stay in LDS");
 static_assert((kPoolWaves & (kPoolWaves - 1)) == 0, "pool_row_kernel's claim order takes v mod kPoolWaves by a mask");
 
 // The spacing of pool_row_kernel's sample chunks: the largest power of two s with
@@ -4162,12 +4167,16 @@ __global__ __launch_bounds__(kPoolThreads, 8) void pool_row_kernel(Launch L, Wor
   // fifth of a 151,936 row, so it leaves ~6 kk there; rows of at least kPoolGuessChunks
   // chunks (a sample of at most a quarter) stream at the (kk/2)-th largest group maximum
   // instead -- ~2.5 kk candidates when the sample stands for the row -- and take their
-  // candidates again at the certain bound if the guess leaves fewer than kk.
+  // candidates again at the certain bound if the guess leaves fewer than kk. Rows of at most
+  // kPoolAllRow elements take every element as a candidate: the list holds them, and a sample of
+  // theirs is the row or nearly so, and its select costs more than the candidates that it keeps out.
   const bool guess = kk > 1 && kk < n && nchunks >= kPoolGuessChunks;
   float theta = -INFINITY;
-  if (kk > 0 && kk < n) {
+  if (kk > 0 && kk < n && n > kPoolAllRow) {
     theta = sample_bound(guess ? (uint32_t)kk / 2u : (uint32_t)kk);
     if (w == 0) TABBY_STAMP(22);
+  } else {
+    pool_hist_clear(sm);  // for the selection's passes, behind the stream's barrier
   }
 
   float lane_max = -INFINITY;
