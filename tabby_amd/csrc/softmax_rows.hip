@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <string>
 
 #include "abi_internal.h"
@@ -46,6 +47,8 @@ constexpr int kTinyCols = 64;            // one group of one entry per lane
 constexpr int kElementCols = 384;        // one entry per lane at a time up to here
 constexpr int kBlockMinLongRows = 1024;  // rows of 513-1,024 entries
 constexpr int kChunkCols = 16384;        // longest row held in a workgroup's registers
+constexpr int kMaxRowThreads = 1024;     // of softmax_rows_chunk_kernel
+constexpr int kLaunchRows = (int)(((int64_t)1 << 32) / kMaxRowThreads) - 1;
 constexpr double kTwo24 = 16777216.0;
 constexpr double kTwo25 = 33554432.0;
 
@@ -588,9 +591,42 @@ __global__ __launch_bounds__(kSmWaves *kWaveSize) void softmax_rows_stream_kerne
 template <int NW, int Q>
 void launch_chunks(const float *x, float *out, const RowDims &d, hipStream_t s) {
   static_assert(NW * Q * 256 <= kChunkCols, "no wider than the widest rows held in registers");
+  static_assert(NW * kWaveSize <= kMaxRowThreads, "kLaunchRows");
   const int per_group = NW == 1 ? kSmWaves : 1;
   hipLaunchKernelGGL((softmax_rows_chunk_kernel<NW, Q>), dim3((unsigned)((d.n_rows + per_group - 1) / per_group)),
                      dim3((unsigned)(NW * per_group * kWaveSize)), 0, s, x, out, d);
+}
+
+// One launch (at most kLaunchRows rows).
+void launch_rows(const float *x, float *out, const RowDims &d, hipStream_t s) {
+  const dim3 grid((unsigned)((d.n_rows + kSmWaves - 1) / kSmWaves)), block(kSmWaves * kWaveSize);
+  // Rows of up to kChunkCols entries are held in registers from the load to the store; longer
+  // ones take three passes. Enough rows to fill the chip share the instructions of their sums
+  // (softmax_rows_block_kernel, four rows per wave's adds; an entry per lane at a time up to
+  // kElementCols, four beyond), up to 1,024 entries: 14 x 1,024
+  // causal rows of 1,024 took 27.4 us against 33.0 by chunks, but 280 rows of 920 took 9.6 us
+  // against 7.1, and 14 x 512 rows of 2,048 took 44.2 us (with room for 2,048) against 41.7.
+  if (d.row_len <= 512 && d.n_rows >= kBlockMinRows) {
+    if (d.row_len <= kTinyCols) hipLaunchKernelGGL((softmax_rows_block_kernel<kTinyCols, 1>), grid, block, 0, s, x, out, d);
+    else if (d.row_len <= kElementCols) hipLaunchKernelGGL((softmax_rows_block_kernel<512, 1>), grid, block, 0, s, x, out, d);
+    else hipLaunchKernelGGL((softmax_rows_block_kernel<512, 4>), grid, block, 0, s, x, out, d);
+  } else if (d.row_len <= 1024 && d.n_rows >= kBlockMinLongRows) {
+    hipLaunchKernelGGL((softmax_rows_block_kernel<1024, 4>), grid, block, 0, s, x, out, d);
+  } else if (d.row_len <= 512) {
+    launch_chunks<1, 2>(x, out, d, s);
+  } else if (d.row_len <= 1024) {
+    launch_chunks<4, 1>(x, out, d, s);
+  } else if (d.row_len <= 2048) {
+    launch_chunks<2, 4>(x, out, d, s);
+  } else if (d.row_len <= 4096) {
+    launch_chunks<4, 4>(x, out, d, s);
+  } else if (d.row_len <= 8192) {
+    launch_chunks<8, 4>(x, out, d, s);
+  } else if (d.row_len <= kChunkCols) {
+    launch_chunks<16, 4>(x, out, d, s);
+  } else {
+    hipLaunchKernelGGL(softmax_rows_stream_kernel, grid, block, 0, s, x, out, d);
+  }
 }
 
 __global__ void exp_f32_kernel(const float *x, float *y, int64_t n) {
@@ -628,35 +664,14 @@ extern "C" int tabby_softmax_rows_device(const float *x_dev, float *out_dev, int
   const size_t bytes = (size_t)n_rows * row_len * sizeof(float);
   if (xb != ob && xb < ob + bytes && ob < xb + bytes)
     return record_failure(TABBY_EINVAL, "out must be x itself or not overlap it");
-  const RowDims d{n_rows, row_len, causal_period, causal_offset};
   const hipStream_t s = (hipStream_t)stream;
-  const dim3 grid((unsigned)((n_rows + kSmWaves - 1) / kSmWaves)), block(kSmWaves * kWaveSize);
-  // Rows of up to kChunkCols entries are held in registers from the load to the store; longer
-  // ones take three passes. Enough rows to fill the chip share the instructions of their sums
-  // (softmax_rows_block_kernel, four rows per wave's adds; an entry per lane at a time up to
-  // kElementCols, four beyond), up to 1,024 entries: 14 x 1,024
-  // causal rows of 1,024 took 27.4 us against 33.0 by chunks, but 280 rows of 920 took 9.6 us
-  // against 7.1, and 14 x 512 rows of 2,048 took 44.2 us (with room for 2,048) against 41.7.
-  if (row_len <= 512 && n_rows >= kBlockMinRows) {
-    if (row_len <= kTinyCols) hipLaunchKernelGGL((softmax_rows_block_kernel<kTinyCols, 1>), grid, block, 0, s, x_dev, out_dev, d);
-    else if (row_len <= kElementCols) hipLaunchKernelGGL((softmax_rows_block_kernel<512, 1>), grid, block, 0, s, x_dev, out_dev, d);
-    else hipLaunchKernelGGL((softmax_rows_block_kernel<512, 4>), grid, block, 0, s, x_dev, out_dev, d);
-  } else if (row_len <= 1024 && n_rows >= kBlockMinLongRows) {
-    hipLaunchKernelGGL((softmax_rows_block_kernel<1024, 4>), grid, block, 0, s, x_dev, out_dev, d);
-  } else if (row_len <= 512) {
-    launch_chunks<1, 2>(x_dev, out_dev, d, s);
-  } else if (row_len <= 1024) {
-    launch_chunks<4, 1>(x_dev, out_dev, d, s);
-  } else if (row_len <= 2048) {
-    launch_chunks<2, 4>(x_dev, out_dev, d, s);
-  } else if (row_len <= 4096) {
-    launch_chunks<4, 4>(x_dev, out_dev, d, s);
-  } else if (row_len <= 8192) {
-    launch_chunks<8, 4>(x_dev, out_dev, d, s);
-  } else if (row_len <= kChunkCols) {
-    launch_chunks<16, 4>(x_dev, out_dev, d, s);
-  } else {
-    hipLaunchKernelGGL(softmax_rows_stream_kernel, grid, block, 0, s, x_dev, out_dev, d);
+  // A launch takes fewer than 2^32 threads (past that its grid wraps, with no error), and a row at most
+  // kMaxRowThreads: larger batches go in several, each of whole causal periods, so that every row keeps
+  // its place in its own. (causal_period <= row_len, which is below 2^18 for that many rows.)
+  const int step = causal_period > 0 && n_rows > kLaunchRows ? kLaunchRows / causal_period * causal_period : kLaunchRows;
+  for (int64_t row = 0; row < n_rows; row += step) {
+    const RowDims d{(int)std::min<int64_t>(step, n_rows - row), row_len, causal_period, causal_offset};
+    launch_rows(x_dev + row * row_len, out_dev + row * row_len, d, s);
   }
   TABBY_HIP_CHECK(hipGetLastError());
   return TABBY_OK;

@@ -272,6 +272,33 @@ def test_softmax_short_row_edges(oracle, row_len):
     test_softmax_chunk_edges(oracle, 259, row_len)
 
 
+@pytest.mark.parametrize("threads,row_len,period", [(64, 4, 3), (1024, 8193, 7)])
+def test_softmax_more_rows_than_a_launch_takes(oracle, threads, row_len, period):
+    # A launch takes fewer than 2^32 threads, `threads` to a row of this length: in place, rows of zeros
+    # but for a few on both sides of the line, causal rows whose places go on across it. (1 and 137 GB.)
+    torch = _torch()
+    line = (1 << 32) // threads
+    n_rows = line + 3
+    if torch.cuda.mem_get_info()[0] < n_rows * row_len * 4 + (8 << 30):
+        pytest.skip("not enough free device memory")
+    x = torch.zeros(n_rows * row_len, device="cuda")
+    rng = np.random.default_rng(4)
+    at = [0, 1, (1 << 22) - 2, (1 << 22) - 1, line - 3, line - 2, line - 1, line, n_rows - 1]
+    rows = {r: rng.normal(0, 3, row_len).astype(np.float32) for r in at}
+    for r, v in rows.items():
+        x[r * row_len:(r + 1) * row_len] = torch.from_numpy(v).cuda()
+    print(f"softmax of {n_rows} rows of {row_len}, in place", flush=True)
+    S.softmax_rows(x, n_rows, row_len, period, row_len - period, out=x)
+    for r, v in rows.items():
+        valid = row_len - period + r % period + 1
+        want = np.zeros(row_len, np.float32)
+        want[:valid] = oracle.softmax_rows(v[:valid], 1, valid)
+        got = x[r * row_len:(r + 1) * row_len].cpu().numpy()
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), f"row {r}"
+    del x
+    torch.cuda.empty_cache()
+
+
 def test_softmax_special_rows(oracle):
     row_len = 300
     x = np.random.default_rng(9).normal(0, 1, (6, row_len)).astype(np.float32)
