@@ -3279,8 +3279,11 @@ __global__ __launch_bounds__(kSortThreads) void head_sort_kernel(Launch L, Works
     sort_segment(sort, L, W, row, g, slots, plan);
     __syncthreads();  // `sort` is reused by the next segment
   }
-  // The workgroup's sorted entries, weights and sums are released with its arrival; the last to
-  // arrive has acquired every other's.
+  // Every wave's sorted entries, weights and sums are released at agent scope before the workgroup
+  // arrives (the barrier alone makes a wave wait for its LDS operations, not for its stores, and the
+  // release of wave 0's arrival only for its own; the reader is on another XCD); the last to arrive has
+  // acquired every other's.
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
   __syncthreads();
   if (threadIdx.x == 0)
     last = __hip_atomic_fetch_add(W.head_arrived + row, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
