@@ -2684,7 +2684,7 @@ __device__ __forceinline__ double exp_sum_term(double y, const double *table) {
 // 8-byte stores scattered over each slice's 16 KB, took 26 us here). One 64-bit LDS add per
 // entry counts it (the low 12 bits) and adds its weight (the upper 52) in fixed point: bin b's
 // weights, below 2^-k, k = floor(b * width), are scaled by 2^(40 + k), so 2,048 of them stay
-// below 2^52 and each is rounded by at most 2^-41 of 2^-k, 2^-39 of its value (a bin is at most
+// below 2^52 and each is rounded by at most 2^-41 of 2^-k, 2^-39.5 of its value (a bin is at most
 // 0.43 binary orders wide: the range stored is within 37.5 T of the max).
 constexpr int kHeadSparse = 8 * kWaveSize;
 constexpr int kTableMin = 32;
@@ -3309,14 +3309,16 @@ __global__ __launch_bounds__(kSortThreads) void head_sort_kernel(Launch L, Works
 // V8's, so their comparisons decide as the reference's only when they clear their threshold by
 // the errors of both, each rounding 2^-53 relative. The reference's running sum at place j,
 // c_j, carries n roundings of its scaled total (n the vocabulary) and j + 2 of its own. Here
-// the total carries fewer than 64 additions and the 2^-43 of exp_sum_term's terms, a partial
-// sum one addition for each entry of a bin, the 8 ulp of exp_nonpos's and the 2^-39 of a
-// table's, all of them an argument within 37.5 * 1.5 ulp (a product by 1/T). So the cut needs (n + 2 j + the place's bin +
-// kPickAdds) * 2^-53 on both sides: 2^-35.6 at 151,936 and a shallow cut, against gaps of about
-// 1e-6 between neighbouring sums. In the draw the scaled total cancels: the cut's place takes
-// the place of n. A row that does not clear them has its head sorted and summed bit for bit
-// (head_sort_kernel). poolMass is 1 (the pool is the whole row) within the n * 2^-53 of a
-// sequential sum.
+// the total carries fewer than 64 additions and the 2^-43 of exp_sum_term's terms; a partial
+// sum one addition for each entry of a bin, the 8 ulp of exp_nonpos's and the 2^-39.5 of a
+// table's (kTableError), all of them an argument within 37.5 * 1.5 ulp (a product by 1/T). So the
+// cut, a partial sum against the total, needs (n + 2 j + the place's bin + kPickAdds) * 2^-53 on
+// both sides: 2^-35.5 at 151,936 and a shallow cut, against gaps of about 1e-6 between neighbouring
+// sums. In the draw the scaled total cancels: the cut's place takes the place of n, and both
+// sides of the comparison are partial sums, of which each may carry a table's error (tied entries
+// all round the same way): kPickAdds holds it twice. A row that does not clear them has its head
+// sorted and summed bit for bit (head_sort_kernel). poolMass is 1 (the pool is the whole row)
+// within the n * 2^-53 of a sequential sum.
 //
 // What bounds it: latency -- dependent rounds of loads, LDS atomics and barriers over a few
 // thousand entries of one row. Sorting the head took 983 us for 16 rows of 151,936 at T = 1,
@@ -3326,7 +3328,10 @@ __global__ __launch_bounds__(kSortThreads) void head_sort_kernel(Launch L, Works
 constexpr int kPickList = 4 * kWaveSize;  // entries one wave sorts
 constexpr int kPickKept = 4;              // stored entries per thread kept in registers
 constexpr int kPickFew = kPickKept * kPlanThreads;
-constexpr int kPickAdds = 4096 + (1 << 14);  // 2^-39: head_kernel's fixed-point weights
+// An entry of a table, rounded by at most half of 2^-kWeightBits of 2^-k (head_kernel), weighs at
+// least 2^-(1.43) of 2^-k: 2^-39.57 of its value, in roundings of 2^-53.
+constexpr int kTableError = 11100;
+constexpr int kPickAdds = 4096 + 2 * kTableError;
 constexpr int kPlanWaves = kPlanThreads / kWaveSize;
 static_assert(kPickBins == kPlanThreads, "one bin per thread");
 
