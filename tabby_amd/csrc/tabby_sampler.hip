@@ -3798,6 +3798,7 @@ __global__ void exp_kernel(const double *x, double *y, int64_t n) {
 constexpr int kPoolWaves = 16;
 constexpr int kPoolThreads = kPoolWaves * kWaveSize;
 constexpr int kPoolListCap = 8192;
+constexpr int kPoolMaxParts = 8;
 constexpr int kPoolBoundKeys = 4 * kPoolThreads;
 // Rows of at least this many chunks (the sample then at most a quarter of the row) stream at a
 // guessed first bound (pool_row_kernel).
@@ -4090,24 +4091,133 @@ __device__ __forceinline__ uint64_t pool_select(PoolSmem &sm, Batches &batches, 
   return pool_select_from(sm, batches, need, lo2, hi2, 1, index_bits);
 }
 
+// The end of a row, by its whole workgroup, from the C candidates -- sm.u.list[i] for i <
+// kPoolListCap, else region[i]; all with a key of at least theta_key; the histogram zeroed -- and the
+// statistics rs: its exact top kk, unsorted, to `sorted` in LDS for a row this workgroup samples
+// itself (valid parameters, a pool of at most kcap, finite statistics: every finite pool), else to
+// region[0 .. kept) for pool_handoff_kernel (whole-vocabulary rows). PART: of a part of a row, to
+// region[0 .. kept) for pool_merge_kernel.
+template <bool PART, typename In>
+__device__ __forceinline__ void pool_finish(PoolSmem &sm, const Launch &L, const Workspace &W, int row, int part,
+                                            const tabby_row_params &P, bool valid_params, int keff, int kk,
+                                            const In *src, uint64_t *region, uint32_t C, uint32_t theta_key,
+                                            const RowStats &rs) {
+  const int w = __builtin_amdgcn_readfirstlane(wave_id()), lane = wave_lane();
+  // The row's outcome: a status (parameters outside the contract,
+  // statistics outside the domain, a whole-vocabulary row with no head pass), a pool this
+  // workgroup samples (`here`), or a whole-vocabulary row for pool_handoff_kernel and the head
+  // kernels. (C >= kk >= 1 for a pool in the domain: theta has kk elements at or above it --
+  // the floor always, a guessed bound once the count above has shown it.)
+  const bool in_domain = rs.max > -INFINITY && rs.max < INFINITY && rs.sum_exp > 0.0 && rs.sum_exp < INFINITY;
+  const bool pool = keff <= L.kcap;
+  int32_t status = TABBY_OK;
+  if (PART) {
+    // A part that is all -inf keeps its candidates: the row may need them. One that holds what puts
+    // the row out of the domain keeps none.
+    if (!(rs.max < INFINITY)) status = TABBY_EDOMAIN;
+  } else if (!valid_params || !in_domain) status = !valid_params ? TABBY_EINVAL : TABBY_EDOMAIN;
+  else if (!pool && !L.head_pass) status = TABBY_EINVAL;
+  else if (pool && C == 0u) status = TABBY_EDOMAIN;
+  const bool here = !PART && status == TABBY_OK && pool;
+  auto put = [&](uint32_t at, uint64_t v) {
+    if (here) sm.sorted[at] = v; else region[at] = v;
+  };
+  uint32_t kept = 0u;
+  const bool selects = status == TABBY_OK && kk > 0;
+  if (selects && C > (uint32_t)kk) {
+    uint32_t sel_begin = 0u, sel_end = C;  // the entries `batches` visits (pool_select narrows them)
+    auto batches = [&](auto &&g) {
+      for (uint32_t base = sel_begin; base < sel_end; base += kPoolBatch * kPoolThreads) {
+        uint64_t v[kPoolBatch];
+        bool ok[kPoolBatch];
+#pragma unroll
+        for (int u = 0; u < kPoolBatch; ++u) {
+          const uint32_t i = base + u * kPoolThreads + threadIdx.x;
+          ok[u] = i < sel_end;
+          v[u] = !ok[u] ? 0ull : i < (uint32_t)kPoolListCap ? sm.u.list[i] : region[i];
+        }
+        g(v, ok);
+      }
+    };
+    // Every candidate's key lies between theta's and the row max's.
+    // The compaction's and the gather's slot counters, published by the passes' barriers.
+    if (threadIdx.x == 0) {
+      sm.bs.slot = 0u;
+      sm.bs.slot2 = 0u;
+      sm.bs.u[0] = ~0u;
+      sm.bs.u[1] = 0u;
+    }
+    const uint64_t thr = pool_select(sm, batches, (uint32_t)kk, theta_key, key_of(rs.max), C, sel_begin, sel_end,
+                                     L.vocab > 1 ? 32 - __builtin_clz((unsigned)(L.vocab - 1)) : 1);
+    sel_begin = 0u;  // the gather below visits every candidate
+    sel_end = C;
+    // (No barrier: the last pass's search, which read the histogram that `sorted` overlays,
+    // ended with one.)
+    // region[0 .. kk) lies below the overflow entries (kk <= 1,024 < kPoolListCap).
+    if (w == 0) TABBY_STAMP(18);
+    batches([&](const uint64_t (&v)[kPoolBatch], const bool (&ok)[kPoolBatch]) {
+      bool take[kPoolBatch];
+      uint32_t at[kPoolBatch];
+#pragma unroll
+      for (int u = 0; u < kPoolBatch; ++u) take[u] = ok[u] && v[u] >= thr;
+      wave_slots(take, &sm.bs.slot, at);
+#pragma unroll
+      for (int u = 0; u < kPoolBatch; ++u)
+        if (take[u] && at[u] < (uint32_t)kk) put(at[u], v[u]);
+    });
+    kept = (uint32_t)kk;
+  } else if (selects) {
+    for (uint32_t i = threadIdx.x; i < C; i += kPoolThreads) put(i, sm.u.list[i]);  // C <= kk: in LDS
+    kept = C;
+  }
+  if constexpr (!PART) if (here) {
+    // sampleFromTopK over the pool, sorted descending.
+    const int count = (int)kept;
+    const int npow = next_pow2(count);
+    for (int i = count + (int)threadIdx.x; i < npow; i += kPoolThreads) sm.sorted[i] = 0ull;
+    __syncthreads();  // the gather's reads of the list are done: finish_row reuses it
+    if (w == 0) TABBY_STAMP(19);
+    block_merge_sort_desc<kPoolWaves>(sm.sorted, sm.u.merge, npow);
+    if (w == 0) TABBY_STAMP(20);
+    finish_row<kKcapLarge, In, PoolSmem, kPoolWaves>(sm, L, row, src, count, rs.max, rs.sum_exp, P);
+  }
+  if (w == 0) {
+    if (lane == 0) {
+      SliceStat st;
+      st.max = rs.max;
+      st.count = PART ? kept : here || status != TABBY_OK ? kPoolRowDone : kept;
+      st.sum = rs.sum_exp;
+      W.stats[(size_t)row * kMaxSplits + part] = st;
+      if (!PART && status != TABBY_OK) {
+        write_status(L, row, status, rs.max, rs.sum_exp);
+        W.row_state[row].status = status;
+      }
+    }
+    TABBY_STAMP(21);
+    TABBY_STAMP_REAL(25);
+  }
+}
+
 // Two workgroups per CU (74 KB of LDS and at most 64 VGPRs each): 512 rows run in one round,
 // and one row's bound and tail overlap the other's streaming (the SIMDs issue the older
 // workgroup's waves first, so the first-dispatched row ends its stream well before the
 // other, whose tail alone then runs with nothing streaming beside it).
-template <typename In, int VEC>
+template <typename In, int VEC, bool PART>
 __global__ __launch_bounds__(kPoolThreads, 8) void pool_row_kernel(Launch L, Workspace W) {
   __shared__ PoolSmem sm;
-  const int row = (int)blockIdx.x;
+  int row = (int)blockIdx.x, part = 0;
+  if constexpr (PART) row_slice_of((int)blockIdx.x, L.rows, L.parts, row, part);
   const int w = __builtin_amdgcn_readfirstlane(wave_id()), lane = wave_lane();  // w: scalar
   const tabby_row_params P = L.params[row];
-  const int n = L.vocab;
+  const int begin = PART ? part * L.slice_len : 0;
+  const int n = PART ? min(L.slice_len, L.vocab - begin) : L.vocab;
   const int nchunks = (n + kWChunk - 1) / kWChunk;
   const int full_chunks = n / kWChunk;
   const bool valid_params = params_valid(P, L.k_max);
-  const int keff = effective_k(P, n);
+  const int keff = effective_k(P, L.vocab);
   const int kk = slice_keep(valid_params, keff, n, L.kcap, L.head_pass, L.topk_cap);
-  const In *src = reinterpret_cast<const In *>(L.logits) + (size_t)row * n;
-  uint64_t *region = W.cands + (size_t)row * W.row_cand_stride;
+  const In *src = reinterpret_cast<const In *>(L.logits) + (size_t)row * L.vocab + begin;
+  uint64_t *region = W.cands + (size_t)row * W.row_cand_stride + begin;  // room for every element
   if (w == 0) {
     TABBY_STAMP(16);
     TABBY_STAMP_REAL(24);
@@ -4178,7 +4288,10 @@ __global__ __launch_bounds__(kPoolThreads, 8) void pool_row_kernel(Launch L, Wor
   // candidates again at the certain bound if the guess leaves fewer than kk. Rows of at most
   // kPoolAllRow elements take every element as a candidate: the list holds them, and a sample of
   // theirs is the row or nearly so, and its select costs more than the candidates that it keeps out.
-  const bool guess = kk > 1 && kk < n && nchunks >= kPoolGuessChunks;
+  // (Not a small pool in parts: half of its bound is a few entries of the sample, whose share of the
+  // part varies by a quarter, and one part of many that falls short holds its row up: 32 rows of
+  // 300,000 in two parts, lists of 32, the call 152 us with a guess, 133 without.)
+  const bool guess = kk > (PART ? kWaveSize : 1) && kk < n && nchunks >= kPoolGuessChunks;
   float theta = -INFINITY;
   if (kk > 0 && kk < n && n > kPoolAllRow) {
     theta = sample_bound(guess ? (uint32_t)kk / 2u : (uint32_t)kk);
@@ -4220,13 +4333,13 @@ __global__ __launch_bounds__(kPoolThreads, 8) void pool_row_kernel(Launch L, Wor
       uint64_t *dst = sm.u.list + pos;
 #pragma unroll
       for (int e = 0; e < kWChunkPerLane; ++e) {
-        if (cur[e] >= theta) *dst++ = composite(key_of(cur[e]), (uint32_t)wave_local<VEC>(c, e));
+        if (cur[e] >= theta) *dst++ = composite(key_of(cur[e]), (uint32_t)(begin + wave_local<VEC>(c, e)));
       }
     } else {
 #pragma unroll
       for (int e = 0; e < kWChunkPerLane; ++e) {
         if (cur[e] >= theta) {
-          const uint64_t v = composite(key_of(cur[e]), (uint32_t)wave_local<VEC>(c, e));
+          const uint64_t v = composite(key_of(cur[e]), (uint32_t)(begin + wave_local<VEC>(c, e)));
           if (pos < (uint32_t)kPoolListCap) sm.u.list[pos] = v; else region[pos] = v;
           ++pos;
         }
@@ -4310,7 +4423,7 @@ __global__ __launch_bounds__(kPoolThreads, 8) void pool_row_kernel(Launch L, Wor
           at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
           if (take) {
             const uint32_t pos = at + (uint32_t)lanes_below(m);
-            const uint64_t e = composite(key_of(v[u]), (uint32_t)(base + u * kPoolThreads + (int)threadIdx.x));
+            const uint64_t e = composite(key_of(v[u]), (uint32_t)(begin + base + u * kPoolThreads + (int)threadIdx.x));
             if (pos < (uint32_t)kPoolListCap) sm.u.list[pos] = e; else region[pos] = e;
           }
         }
@@ -4319,104 +4432,47 @@ __global__ __launch_bounds__(kPoolThreads, 8) void pool_row_kernel(Launch L, Wor
     __syncthreads();
     C = sm.count;
   }
-  // The row's exact top kk of the candidates, unsorted: to `sorted` in LDS for a row this
-  // workgroup samples itself (valid parameters, a pool of at most kcap, finite statistics:
-  // every finite pool), else to region[0 .. kept) for pool_handoff_kernel (whole-vocabulary rows).
   if (w == 0) {
     TABBY_STAMP(17);
     TABBY_RECORD(31, C);
     TABBY_RECORD(29, rescan ? 1 : 0);
   }
-  const RowStats rs = row_stats(sm.stats, kPoolWaves);
-  // The row's outcome: a status (parameters outside the contract,
-  // statistics outside the domain, a whole-vocabulary row with no head pass), a pool this
-  // workgroup samples (`here`), or a whole-vocabulary row for pool_handoff_kernel and the head
-  // kernels. (C >= kk >= 1 for a pool in the domain: theta has kk elements at or above it --
-  // the floor always, a guessed bound once the count above has shown it.)
-  const bool in_domain = rs.max > -INFINITY && rs.max < INFINITY && rs.sum_exp > 0.0 && rs.sum_exp < INFINITY;
-  const bool pool = keff <= L.kcap;
-  int32_t status = TABBY_OK;
-  if (!valid_params || !in_domain) status = !valid_params ? TABBY_EINVAL : TABBY_EDOMAIN;
-  else if (!pool && !L.head_pass) status = TABBY_EINVAL;
-  else if (pool && C == 0u) status = TABBY_EDOMAIN;
-  const bool here = status == TABBY_OK && pool;
-  auto put = [&](uint32_t at, uint64_t v) {
-    if (here) sm.sorted[at] = v; else region[at] = v;
-  };
-  uint32_t kept = 0u;
-  const bool selects = status == TABBY_OK && kk > 0;
-  if (selects && C > (uint32_t)kk) {
-    uint32_t sel_begin = 0u, sel_end = C;  // the entries `batches` visits (pool_select narrows them)
-    auto batches = [&](auto &&g) {
-      for (uint32_t base = sel_begin; base < sel_end; base += kPoolBatch * kPoolThreads) {
-        uint64_t v[kPoolBatch];
-        bool ok[kPoolBatch];
-#pragma unroll
-        for (int u = 0; u < kPoolBatch; ++u) {
-          const uint32_t i = base + u * kPoolThreads + threadIdx.x;
-          ok[u] = i < sel_end;
-          v[u] = !ok[u] ? 0ull : i < (uint32_t)kPoolListCap ? sm.u.list[i] : region[i];
-        }
-        g(v, ok);
-      }
-    };
-    // Every candidate's key lies between theta's and the row max's.
-    // The compaction's and the gather's slot counters, published by the passes' barriers.
-    if (threadIdx.x == 0) {
-      sm.bs.slot = 0u;
-      sm.bs.slot2 = 0u;
-      sm.bs.u[0] = ~0u;
-      sm.bs.u[1] = 0u;
+  pool_finish<PART>(sm, L, W, row, part, P, valid_params, keff, kk, src, region, C, key_of(theta),
+                    row_stats(sm.stats, kPoolWaves));
+}
+
+// A row of parts from their lists (each the part's exact top kk): the row's candidates, at most
+// kPoolMaxParts * kcap, all in LDS. Ends as pool_row_kernel does.
+template <typename In>
+__global__ __launch_bounds__(kPoolThreads, 8) void pool_merge_kernel(Launch L, Workspace W) {
+  static_assert(kPoolMaxParts * kKcapLarge <= kPoolListCap && kPoolMaxParts <= kPoolWaves, "the parts' lists fit");
+  __shared__ PoolSmem sm;
+  const int row = (int)blockIdx.x, lane = wave_lane();
+  const tabby_row_params P = L.params[row];
+  const bool valid_params = params_valid(P, L.k_max);
+  const int keff = effective_k(P, L.vocab);
+  const int kk = slice_keep(valid_params, keff, L.vocab, L.kcap, L.head_pass, L.topk_cap);
+  const In *src = reinterpret_cast<const In *>(L.logits) + (size_t)row * L.vocab;
+  uint64_t *region = W.cands + (size_t)row * W.row_cand_stride;
+  const SliceStat *stats = W.stats + (size_t)row * kMaxSplits;
+  const RowStats rs = row_stats(stats, L.parts);  // every wave alike
+  pool_hist_clear(sm);
+  if (threadIdx.x == 0) sm.count = ~0u;
+  __syncthreads();
+  uint32_t C = 0u, low = ~0u;
+  for (int p = 0; p < L.parts; ++p) {
+    const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)rs.cnt[0], p);
+    for (uint32_t i = threadIdx.x; i < n; i += kPoolThreads) {
+      const uint64_t v = region[(size_t)p * L.slice_len + i];
+      sm.u.list[C + i] = v;
+      low = min(low, composite_key(v));
     }
-    const uint64_t thr = pool_select(sm, batches, (uint32_t)kk, key_of(theta), key_of(rs.max), C, sel_begin, sel_end,
-                                     n > 1 ? 32 - __builtin_clz((unsigned)(n - 1)) : 1);
-    sel_begin = 0u;  // the gather below visits every candidate
-    sel_end = C;
-    // (No barrier: the last pass's search, which read the histogram that `sorted` overlays,
-    // ended with one.)
-    // region[0 .. kk) lies below the overflow entries (kk <= 1,024 < kPoolListCap).
-    if (w == 0) TABBY_STAMP(18);
-    batches([&](const uint64_t (&v)[kPoolBatch], const bool (&ok)[kPoolBatch]) {
-      bool take[kPoolBatch];
-      uint32_t at[kPoolBatch];
-#pragma unroll
-      for (int u = 0; u < kPoolBatch; ++u) take[u] = ok[u] && v[u] >= thr;
-      wave_slots(take, &sm.bs.slot, at);
-#pragma unroll
-      for (int u = 0; u < kPoolBatch; ++u)
-        if (take[u] && at[u] < (uint32_t)kk) put(at[u], v[u]);
-    });
-    kept = (uint32_t)kk;
-  } else if (selects) {
-    for (uint32_t i = threadIdx.x; i < C; i += kPoolThreads) put(i, sm.u.list[i]);  // C <= kk: in LDS
-    kept = C;
+    C += n;
   }
-  if (here) {
-    // sampleFromTopK over the pool, sorted descending.
-    const int count = (int)kept;
-    const int npow = next_pow2(count);
-    for (int i = count + (int)threadIdx.x; i < npow; i += kPoolThreads) sm.sorted[i] = 0ull;
-    __syncthreads();  // the gather's reads of the list are done: finish_row reuses it
-    if (w == 0) TABBY_STAMP(19);
-    block_merge_sort_desc<kPoolWaves>(sm.sorted, sm.u.merge, npow);
-    if (w == 0) TABBY_STAMP(20);
-    finish_row<kKcapLarge, In, PoolSmem, kPoolWaves>(sm, L, row, src, count, rs.max, rs.sum_exp, P);
-  }
-  if (w == 0) {
-    if (lane == 0) {
-      SliceStat st;
-      st.max = rs.max;
-      st.count = here || status != TABBY_OK ? kPoolRowDone : kept;
-      st.sum = rs.sum_exp;
-      W.stats[(size_t)row * kMaxSplits] = st;
-      if (status != TABBY_OK) {
-        write_status(L, row, status, rs.max, rs.sum_exp);
-        W.row_state[row].status = status;
-      }
-    }
-    TABBY_STAMP(21);
-    TABBY_STAMP_REAL(25);
-  }
+  low = ~wave_max_u32(~low);
+  if (lane == 0) atomicMin(&sm.count, low);
+  __syncthreads();
+  pool_finish<false>(sm, L, W, row, 0, P, valid_params, keff, kk, src, region, C, sm.count, rs);
 }
 
 }  // namespace tabby
@@ -4553,6 +4609,20 @@ int row_parts(int rows, int vocab, int cus, int &part_len) {
   return (vocab + part_len - 1) / part_len;
 }
 
+// Few long rows of a large-pool batch: parts of at least kPoolMinPart elements, a pool_row_kernel
+// workgroup each, as many as there are CUs at most (1: none; sets part_len). One CU streams 1,048,576
+// elements alone in 75 us (k = 50; 135 at k = 1,024); in seven parts the call takes 29 and 43; 16 rows
+// 82 -> 35 (48.6 in the slices that served few rows before), 16 of 500,000 44.5 -> 32.3. Parts of
+// 131,072 gained nothing over a whole row (8 rows of 262,144: 29.6 and 30.4), nor do two parts a row
+// on every CU (128 of them 37.4 and 43.3).
+constexpr int kPoolMinPart = 9 << 14;
+int pool_parts(int rows, int vocab, int cus, int &part_len) {
+  const int parts = std::min(std::min(cus / rows, vocab / kPoolMinPart), kPoolMaxParts);
+  if (parts < 2 || 3 * rows > cus) return 1;
+  part_len = ((vocab + parts - 1) / parts + kWChunk - 1) / kWChunk * kWChunk;
+  return (vocab + part_len - 1) / part_len;
+}
+
 template <typename In, int VEC, bool HEAD>
 void launch_first(const Launch &L, const Workspace &W, hipStream_t stream) {
   const dim3 slices((unsigned)(L.rows * L.splits)), rows((unsigned)L.rows);
@@ -4574,8 +4644,14 @@ hipError_t launch_pair(const Launch &L, const Workspace &W, hipStream_t stream) 
     if (L.head_pass) launch_first<In, VEC, true>(L, W, stream);
     else launch_first<In, VEC, false>(L, W, stream);
   } else {
-    // pool_row_kernel ends every row but a head pass's whole-vocabulary ones.
-    hipLaunchKernelGGL((pool_row_kernel<In, VEC>), rows, dim3(kPoolThreads), 0, stream, L, W);
+    // pool_row_kernel (or, for rows in parts, pool_merge_kernel) ends every row but a head pass's
+    // whole-vocabulary ones.
+    if (L.parts > 1) {
+      hipLaunchKernelGGL((pool_row_kernel<In, VEC, true>), dim3((unsigned)(L.rows * L.parts)), dim3(kPoolThreads), 0, stream, L, W);
+      hipLaunchKernelGGL((pool_merge_kernel<In>), rows, dim3(kPoolThreads), 0, stream, L, W);
+    } else {
+      hipLaunchKernelGGL((pool_row_kernel<In, VEC, false>), rows, dim3(kPoolThreads), 0, stream, L, W);
+    }
     if (L.head_pass) hipLaunchKernelGGL(pool_handoff_kernel, rows, dim3(kBlock), 0, stream, L, W);
   }
   return hipGetLastError();
@@ -4632,6 +4708,7 @@ Plan plan_launch(int rows, int vocab, int dtype, const void *logits, int k_max, 
     // One row of 32,000 at k = 512: 35 -> 19.5.
     L.splits = 1;
     L.slice_len = vocab;
+    L.parts = pool_parts(rows, vocab, cus, L.slice_len);
   } else if (L.kcap <= kWaveKcap && rows * 2 > cus && rows < cus) {
     // Between half the CUs and all of them: one 16-wave workgroup per row all the same (the
     // idle CUs leave the others more of the HBM bandwidth). Against the one-wave slices and

@@ -590,6 +590,52 @@ def test_large_pools_few_rows(oracle, rows, vocab, dtype):
     compare(w, res, ids, vals, run_oracle(oracle, w, cap), cap)
 
 
+@pytest.mark.parametrize("rows,vocab,dtype", [(3, 294912, np.float32), (9, 300001, np.float32), (5, 500000, np.float16),
+                                              (2, 1048576, np.float32)])
+def test_large_pools_long_rows_in_parts(oracle, rows, vocab, dtype):
+    # Two to seven parts a row, merged by pool_merge_kernel: a part all -inf, a row with fewer finite
+    # entries than its pool, ties across parts (the lower index wins), a short last part that holds the
+    # row's top, whole-vocabulary rows and lists.
+    w = synth.random_workload(rows=rows, vocab=vocab, seed=rows + vocab, k_choices=(1, 50, 300, 1024, 0),
+                              ties=rows % 2 == 1, top_ps=(0.9, 0.98, 1.0))
+    w.logits[0, : vocab // 2 + 1] = -np.inf
+    w.top_k[0] = 1024
+    keep = np.random.default_rng(vocab).choice(vocab, 20, replace=False)
+    kept = w.logits[1, keep].copy()
+    w.logits[1] = -np.inf
+    w.logits[1, keep] = kept
+    w.top_k[1] = 300
+    if rows > 2:
+        w.logits[2] = 1.25
+        w.top_k[2] = 1000
+    if rows > 4:
+        w.logits[3, -700:] += 9.0
+        w.top_k[3:5] = 600, 0
+    w.logits = w.logits.astype(dtype)
+    print(f"long rows in parts: {rows} x {vocab} {dtype.__name__}", flush=True)
+    res, ids, vals = run_gpu(w, k_max=1024, topk_cap=300)
+    compare(w, res, ids, vals, run_oracle(oracle, w, 300), 300)
+
+
+def test_large_pools_long_rows_outside_contract(oracle):
+    import torch
+    rows, vocab = 6, 300001
+    x = torch.randn(rows, vocab, device="cuda")
+    x[0] = float("-inf")
+    x[1, 7] = float("nan")
+    x[2, vocab - 1] = float("inf")
+    p = S.make_params(S.SamplingParams(0.7, 500, 0.9), rows, 0.25)
+    p["top_k"][[3, 4]] = 2000, 0
+    with S.GpuSampler(vocab_max=vocab, rows_max=rows, k_max=1024) as g:
+        pd = torch.from_numpy(p.view(np.uint8).copy()).cuda()
+        rd = torch.zeros(rows * S.RESULT_DTYPE.itemsize, dtype=torch.uint8, device="cuda")
+        g.sample_device(x, pd, rd)
+        res = rd.cpu().numpy().view(S.RESULT_DTYPE)
+    assert list(res["status"]) == [S.TABBY_EDOMAIN] * 3 + [S.TABBY_EINVAL] * 2 + [0]
+    o = oracle.sample_row(x[5].cpu().numpy(), 500, 0.7, 0.9, 0.25)
+    assert (int(res["id"][5]), int(res["considered"][5])) == (o["id"], o["considered"])
+
+
 @pytest.mark.parametrize("vocab", [32769, 50257, 65537, 151937])
 def test_parts_with_idle_waves(oracle, vocab):
     # Rows cut into parts of 16,384 elements or fewer: the last part has fewer chunks than its
