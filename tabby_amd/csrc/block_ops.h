@@ -31,18 +31,6 @@ struct BlockScratchT {
 };
 using BlockScratch = BlockScratchT<kWaves>;
 
-template <int NW>
-__device__ __forceinline__ float block_max(float v, BlockScratchT<NW> &s) {
-  v = wave_max(v);
-  __syncthreads();
-  if (lane_id() == 0) s.f[wave_id()] = v;
-  __syncthreads();
-  float r = s.f[0];
-#pragma unroll
-  for (int i = 1; i < NW; ++i) r = fmaxf(r, s.f[i]);
-  return r;
-}
-
 // Fixed reduction tree, so the result is bit-identical from run to run.
 template <int NW>
 __device__ __forceinline__ double block_sum(double v, BlockScratchT<NW> &s) {

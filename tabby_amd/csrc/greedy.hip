@@ -132,9 +132,10 @@ __global__ __launch_bounds__(BLOCK) void argmax_kernel(const In *logits, int voc
 }
 
 // One wave per row, a lane per split. What bounds it is its chain of loads: the partials and the
-// row's first entry come in one round trip. 32 rows of 151,936 f32, a call that is waited for: 27.7
-// us, against 31.2 with a lane per row that read its partials, then the first entry, then the
-// answer's own; back to back 10.8 against 11.3, where two runs of one build differ by more.
+// row's first entry come in one round trip. 32 rows of 151,936 f32: 2.8 us traced, against 4.0 with a
+// lane per row that read its partials, then the first entry, then the answer's own; a call that is
+// waited for 21.4 us against 23.5. Back to back the two launches' host time bounds the call either
+// way (10.2-11.0 us).
 // (A row finished by the last of its workgroups to arrive, with no second launch, took 13.9 us:
 // the store, the count and the partials then wait on memory one after another.)
 template <typename In>

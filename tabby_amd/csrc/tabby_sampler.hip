@@ -22,11 +22,13 @@
 //   * wave_merge_kernel: grid = rows; each 256-lane workgroup combines its row's slices: max,
 //     sum-exp, the exact top-k over the 64-bit (value key, ~index) composites -- the lower index
 //     wins ties, as in sampler.ts:28 -- and sampleFromTopK's f64 tail.
-// Pools above 256 take pool_row_kernel, one workgroup per row from the first element to the draw.
+// Pools above 256 take pool_row_kernel, one workgroup per row from the first element to the draw
+// (or, for few very long rows, one per part of a row, and pool_merge_kernel).
 // The kernel boundary orders the first kernel's writes before the second's reads; no
 // workgroup waits on another. Rows whose pool is the whole vocabulary (top_k = 0 beyond the
-// pool capacity) end in the merge when their largest entries decide them, else in two more
-// kernels that weigh the row's head and select in it (see head_kernel, head_pick_kernel).
+// pool capacity) end in the merge when their largest entries decide them; three more launches
+// follow where there may be such rows: head_kernel and head_pick_kernel weigh the others' heads and
+// select in them, and head_sort_kernel sorts the few heads that the selection cannot decide.
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -235,14 +237,6 @@ __device__ __forceinline__ int slice_keep(bool valid, int keff, int n, int kcap,
   if (!valid) return 0;
   if (keff <= kcap) return min(keff, n);
   return head_pass ? min(max(topk_cap, kHeadList), n) : 0;
-}
-
-// The first active lane's f64, bit for bit (the readfirstlane builtin takes 32-bit ints).
-__device__ __forceinline__ double readfirstlane_f64(double v) {
-  const uint64_t b = (uint64_t)__double_as_longlong(v);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)b);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(b >> 32));
-  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
 __device__ __forceinline__ double readlane_f64(double v, int lane) {
@@ -510,8 +504,6 @@ __device__ __forceinline__ uint32_t wave_slot(bool take, uint32_t *slot) {
   return base + lanes_below(mask);
 }
 
-// Raw loads of chunk `chunk` (no masking, so nothing consumes them until the next
-// iteration and they stay in flight). Lanes past the end reread the slice's last vector.
 // ---------------------------------------------------------------------------------------
 // Kernel 1 for pools of at most 256 (wave_kernel): grid = rows x splits, one wave per
 // workgroup, so nothing in it waits at a barrier. Each wave streams its slice of a row from
@@ -532,53 +524,6 @@ constexpr int kWChunk = kWaveSize * kWChunkPerLane;
 constexpr int kWListCap = 512;
 constexpr int kWaveKcap = 256;
 constexpr int kPruneBins = 256;
-
-template <typename In, int VEC>
-__device__ __forceinline__ void wave_load(const In *src, int n, int chunk, float (&x)[kWChunkPerLane]) {
-  constexpr int ITEMS = kWChunkPerLane / VEC;
-#pragma unroll
-  for (int j = 0; j < ITEMS; ++j) {
-    const int le = chunk * kWChunk + (j * kWaveSize + wave_lane()) * VEC;
-    float v[VEC];
-    Loader<In, VEC>::load(src + min(le, n - VEC), v);  // past the end: reread, masked later
-#pragma unroll
-    for (int c = 0; c < VEC; ++c) x[j * VEC + c] = v[c];
-  }
-}
-
-// Chunk `chunk` lies entirely inside the slice: no clamping.
-template <typename In, int VEC>
-__device__ __forceinline__ void wave_load_full(const In *src, int chunk, float (&x)[kWChunkPerLane]) {
-  constexpr int ITEMS = kWChunkPerLane / VEC;
-  const In *base = src + chunk * kWChunk + wave_lane() * VEC;
-#pragma unroll
-  for (int j = 0; j < ITEMS; ++j) {
-    float v[VEC];
-    Loader<In, VEC>::load(base + j * kWaveSize * VEC, v);
-#pragma unroll
-    for (int c = 0; c < VEC; ++c) x[j * VEC + c] = v[c];
-  }
-}
-
-// Chunk `chunk` by one code path whatever the chunk: lanes past the slice's end reread its
-// last vector, and a chunk past the last (chunk >= nchunks) loads the slice's first vector
-// into every lane (one line, never used). Branching between wave_load_full and wave_load
-// made the compiler land the loads in temporaries and copy them at once -- waiting for the
-// prefetched chunk right after issuing it.
-template <typename In, int VEC>
-__device__ __forceinline__ void wave_load_any(const In *src, int n, int chunk, int nchunks,
-                                              float (&x)[kWChunkPerLane]) {
-  constexpr int ITEMS = kWChunkPerLane / VEC;
-  const bool live = chunk < nchunks;
-#pragma unroll
-  for (int j = 0; j < ITEMS; ++j) {
-    const int le = chunk * kWChunk + (j * kWaveSize + wave_lane()) * VEC;
-    float v[VEC];
-    Loader<In, VEC>::load(src + (live ? min(le, n - VEC) : 0), v);
-#pragma unroll
-    for (int c = 0; c < VEC; ++c) x[j * VEC + c] = v[c];
-  }
-}
 
 template <int VEC>
 __device__ __forceinline__ int wave_local(int chunk, int e) {
@@ -2868,7 +2813,7 @@ __global__ __launch_bounds__(kWaveSize) void head_kernel(Launch L, Workspace W) 
 // batches in descending order. The concatenation of the sorted segments is the sorted head.
 // kSegCap leaves room below 1,024 for the bucket that crosses a segment's end, so that a
 // segment is normally sorted as 1,024 entries: at 1,024 segments of 1,025-1,032 entries were
-// padded to 2,048 and took twice as long (17.9 vs 8.2 us on config 4's largest head).
+// padded to 2,048 and took twice as long (17.9 vs 8.2 us on a head of 13,000 entries).
 constexpr int kHeadBuckets = 4096;
 constexpr int kSegCap = 896;
 constexpr int kSegLds = 8192;
@@ -3631,7 +3576,7 @@ __device__ __forceinline__ bool head_pick(PickSmem &sm, const Launch &L, const W
   const PickBin pb(rs, kTableBins);
   const size_t tables = (size_t)row * W.acc_stride * kTableBins;
   const bool tabled = slice_n > (uint32_t)kTableMin;
-  if (tid < kPlanThreads) sm.off[tid] = slice_n;
+  sm.off[tid] = slice_n;
   __syncthreads();
   {
     const int b = tid % kTableBins;
@@ -3777,8 +3722,8 @@ __global__ void exp_kernel(const double *x, double *y, int64_t n) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Pools of 257..1024 (k_max > 256) in batches of at least as many rows as CUs: one 16-wave
-// workgroup per row streams it as row_kernel does (each wave's first two chunks, then chunks
+// Pools of 257..1024 (k_max > 256), however many the rows: one 16-wave
+// workgroup per row (or part of one: pool_parts) streams it as row_kernel does (each wave's first two chunks, then chunks
 // claimed from an LDS counter) with the lane max and sum-exp, and appends every element at
 // or above the row's first bound to one LDS list shared by its waves: a wave reserves room
 // for a chunk's candidates with one LDS atomic, with no barrier, and past kPoolListCap
@@ -3787,9 +3732,7 @@ __global__ void exp_kernel(const double *x, double *y, int64_t n) {
 // distinct elements; the kk-th largest of their keys (its top 22 bits: a lower bound) has kk
 // elements at or above it, so it never exceeds the row's kk-th largest -- and long rows
 // stream at the (kk/2)-th instead, checked at the end (the rows whose count falls short take
-// their candidates again at the certain bound). (The 4-wave slice kernel started from
-// the first chunk's kk-th largest -- a quarter of that chunk at kk = 1,024 -- and pruned its
-// list with two workgroup barriers per chunk: config 5 took 135 us there.) At the end the
+// their candidates again at the certain bound); short rows have none (kPoolAllRow). At the end the
 // workgroup selects the row's exact top kk from the list (pool_select), gathers it into LDS,
 // sorts it and samples it (finish_row over its 16 waves); a row
 // outside the contract gets its status here too. Only a head pass's whole-vocabulary rows
@@ -4027,7 +3970,7 @@ __device__ __forceinline__ uint64_t pool_select_from(PoolSmem &sm, Batches &batc
 // until one key remains -- a quantized row resolves in one), then over the tied key's index
 // digits. After the first pass only the chosen bin's entries matter: they are copied behind
 // the candidates (B entries at list[C ..), when C + B fits the LDS list) and `batches` is moved
-// onto them, so the later passes visit those B alone instead of all C (config 5: ~2,800
+// onto them, so the later passes visit those B alone instead of all C (512 rows of 151,936 tied logits at k = 1,024: ~2,800
 // candidates, a tied bin of a few hundred; the later passes had re-read every candidate).
 // Indices are below 2^index_bits.
 // The caller has set sm.bs.slot2 = 0, sm.bs.u[0] = ~0 and sm.bs.u[1] = 0 (the compaction's

@@ -76,7 +76,7 @@ def _spiked_row(seed: int, vocab: int, sigma: float, spikes: int) -> np.ndarray:
 
 
 def config(n: int, rows: int | None = None, vocab: int | None = None, seed: int = 2024) -> Workload:
-    """BASELINE.json configs[n-1]; rows / vocab may be reduced for quick parity tests."""
+    """The n-th of the benchmark's five workloads; rows / vocab may be reduced for quick parity tests."""
     if n == 1:
         V = vocab or 49152
         row = normals(stream_seed(seed, 0, 1), V, 2.5).astype(np.float32)

@@ -8,7 +8,7 @@ import numpy as np
 from tabby_amd import sampler as S
 from tabby_amd.synth import Workload
 
-REL_TOL = 1e-5  # normalised probabilities within 1e-5 relative
+REL_TOL = 1e-5  # normalised probabilities
 
 
 def params_of(w: Workload) -> np.ndarray:

@@ -73,8 +73,8 @@ def _check(oracle, logits, params, res, ctx):
 # form -- the per-row kernel's small-pool tail and its sorted merge (256, 200 rows), parts of
 # rows merged by the wave-merge kernel (5 rows of 100,000), one workgroup per row among few
 # rows (5 rows of 33,000), one-wave slices and their merge (61 short rows), the large-pool
-# streaming kernel and merge_kernel<1024> (256 rows), the 256-lane slice kernel with pools
-# above 256 (8 rows), and whole-vocabulary rows (the head kernels, beside finite rows).
+# streaming kernel, as many rows as CUs (256) and few (8, "slice kernel" for what served them
+# before), and whole-vocabulary rows (the head kernels, beside finite rows).
 SHAPES = [
     ("row kernel", 256, 12000, (1, 50, 100, 200, 256), 256, False),
     ("row kernel 200 rows", 200, 12000, (1, 50, 256), 256, True),

@@ -1,6 +1,6 @@
 """GPU parity: libtabby_sampler.so (through its C ABI) against the CPU oracle on identical
 seeded logits and uniforms. Ids, candidate sets and counts must be bit-exact; the f64
-probabilities within 1e-5 relative (the tolerance of BASELINE.json's north_star)."""
+probabilities within 1e-5 relative."""
 import numpy as np
 import pytest
 
@@ -51,8 +51,8 @@ def test_config5_sorted_slice_lists(oracle):
 
 
 def test_large_pool_capacity_mixed_k(oracle):
-    # k_max 1024 sends every row through the 256-lane slices; small and large k mix, with
-    # ties and -inf, on few enough slices per row for the sorted-list merge.
+    # k_max 1024 sends every row through pool_row_kernel; small and large k mix, with ties and
+    # -inf, on fewer rows than CUs.
     w = synth.random_workload(rows=192, vocab=20000, seed=17, ties=True, neg_inf_frac=0.3,
                               k_choices=(1, 64, 300, 1024))
     res, ids, vals = run_gpu(w, k_max=1024, topk_cap=1024)
@@ -114,7 +114,7 @@ def test_pool_row_kernel_rows_outside_contract(oracle):
 def test_pool_row_kernel_batch_with_head_pass(oracle):
     # 256 rows with k_max 1024 and TABBY_FLAG_FULL_VOCAB: pool_row_kernel samples the pools
     # (k 50, 300, 1000) and writes the statuses itself, and hands the whole-vocabulary rows
-    # (k 0) to merge_kernel and the head kernels, which skip the rows it ended.
+    # (k 0) to pool_handoff_kernel and the head kernels, which skip the rows it ended.
     import torch
     w = synth.random_workload(rows=256, vocab=4000, seed=31, k_choices=(0, 50, 300, 1000), ties=True,
                               neg_inf_frac=0.05)
@@ -338,11 +338,11 @@ def test_ties_and_neg_inf(oracle):
 
 @pytest.mark.parametrize("k", [20, 50, 64])
 def test_first_chunk_unrepresentative(oracle, k):
-    # Vocab 147,456 on 4 rows is cut into 36 slices of 4,096, and each slice's first chunk
-    # sets its starting theta. Rows 0-1 put one large value per lane in the first 256
-    # elements of every 4,096-block and keep the rest small (the first chunk holds the whole
-    # top of the slice); row 2 is sorted ascending (every first chunk is its slice's
-    # smallest: a low theta, many candidates, many prunes); row 3 descending.
+    # Vocab 147,456 on 4 rows is cut into nine parts of 16,384, of one chunk per wave, whose
+    # maxima set a part's first bound. Rows 0-1 put one large value per lane in the first 256
+    # elements of every 4,096-block and keep the rest small (every fourth wave holds the top of
+    # its part); row 2 is sorted ascending (the earlier parts' tops all lie below the later
+    # parts' bounds); row 3 descending.
     V = 147456
     w = synth.random_workload(rows=4, vocab=V, seed=41, k_choices=(k,), temperatures=(0.7,),
                               top_ps=(0.9,), sigma=1.0)
@@ -520,11 +520,11 @@ def test_full_vocab_mixed_with_finite_rows(oracle):
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
 @pytest.mark.parametrize("topk_cap,k_max", [(0, 64), (16, 64), (16, 1024), (300, 1024)])
 def test_full_vocab_fast_finish_edges(oracle, dtype, topk_cap, k_max):
-    # Whole-vocabulary rows that the merge's sorted top list may finish (head_fast_kernel) or
-    # must hand to the sorted head: fewer finite entries than the list (the rest -inf), a spike
-    # over a band of ~150 distinct small terms under top-p 0.5 (their ulp counts tie now and
-    # then: the sorted head decides those rows), a plateau whose mass pushes the total past its
-    # binade, and greedy rows.
+    # Whole-vocabulary rows that end from their sorted top list (in the merge or in
+    # head_pick_kernel) or by selection: fewer finite entries than the list (the rest -inf; without
+    # a cut the list is the whole head, summed bit for bit), a spike over a band of ~150 distinct
+    # small terms whose cut is the spike, a plateau of 3,000 whose cut lies hundreds deep, and
+    # greedy and cold rows.
     rows, vocab = 32, 30000
     w = synth.random_workload(rows=rows, vocab=vocab, seed=5150 + topk_cap, k_choices=(0,),
                               temperatures=(0.7,), top_ps=(0.95,), sigma=2.0)
@@ -537,14 +537,14 @@ def test_full_vocab_fast_finish_edges(oracle, dtype, topk_cap, k_max):
             row[keep] = rng.normal(0, 2, 10).astype(np.float32)
             w.logits[r] = row
             w.temperature[r], w.top_p[r] = (0.7, 1.0) if r % 8 == 0 else (0.0, 0.9)
-        elif kind == 1:  # spike + band of distinct terms in [2^-8, 2^-7): P_N < 2 with the band
+        elif kind == 1:  # spike + band of distinct terms in [2^-8, 2^-7)
             row = rng.normal(-20, 1, vocab).astype(np.float32)
             row[rng.integers(vocab)] = 10.0
             band = rng.choice(vocab, 150, replace=False)
             row[band] = (10.0 + rng.uniform(np.log(2.0 ** -8), np.log(2.0 ** -7), 150)).astype(np.float32)
             w.logits[r] = row
             w.temperature[r], w.top_p[r] = 1.0, 0.5
-        elif kind == 2:  # a plateau of 3,000 near the max: its mass leaves P_N's binade
+        elif kind == 2:  # a plateau of 3,000 near the max
             row = rng.normal(0, 2, vocab).astype(np.float32)
             row[rng.choice(vocab, 3000, replace=False)] = (12.0 - rng.uniform(0, 0.5, 3000)).astype(np.float32)
             row[rng.integers(vocab)] = 12.0
@@ -555,8 +555,8 @@ def test_full_vocab_fast_finish_edges(oracle, dtype, topk_cap, k_max):
     w.logits[:] = w.logits.astype(dtype).astype(np.float32)
     if dtype == np.float16:
         w.logits = w.logits.astype(np.float16)
-    # k_max 1024: the list comes from merge_kernel (pools above 256); a 300-entry list is too
-    # long to hand over, and those rows take the sorted head.
+    # k_max 1024: the list, of 300 entries too, comes from pool_handoff_kernel, and no merge decides
+    # a row before the head kernels.
     res, ids, vals = run_gpu(w, k_max=k_max, topk_cap=topk_cap)
     _log(f"full vocab fast finish {dtype.__name__} cap={topk_cap} k_max={k_max}",
          compare(w, res, ids, vals, run_oracle(oracle, w, topk_cap), topk_cap))
@@ -938,7 +938,7 @@ def test_sum_exp_shift_invariant(oracle, offset):
 
 
 def test_config5_full_512_rows(oracle):
-    # BASELINE config 5 at its stated size: one slice per row of the 256-lane slice kernel.
+    # 512 rows of 151,936, k = 1,024, ties and -inf: pool_row_kernel, two workgroups to a CU.
     w = synth.config(5)
     assert w.rows == 512
     res, ids, vals = run_gpu(w, k_max=1024, topk_cap=1024)

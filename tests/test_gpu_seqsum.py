@@ -57,8 +57,8 @@ def test_dense_ties_long(wide):
 
 @pytest.mark.parametrize("stop", [np.inf, 0.98])
 def test_quantised_logit_terms(stop, wide):
-    # Weights of logits on a 0.25 grid (few distinct values, many repeats), sorted, as in
-    # BASELINE config 5; the top-p stop variant cuts inside the run.
+    # Weights of logits on a 0.25 grid (few distinct values, many repeats), sorted; the top-p
+    # stop variant cuts inside the run.
     rng = np.random.default_rng(5)
     levels = np.sort(np.round(rng.normal(0, 2, 1024) * 4) / 4)[::-1]
     s = np.exp(levels - levels[0])
