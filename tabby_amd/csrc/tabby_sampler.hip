@@ -2625,7 +2625,7 @@ __device__ __forceinline__ double exp_sum_term(double y, const double *table) {
 // A warm row stores several percent of its entries (store_threshold), more than head_pick_kernel
 // could search in one workgroup without order (64 rows at T = 1: 78 us there), so a slice that
 // stores more than kTableMin orders its entries by bin and writes each bin's weight and where
-// its entries start (18 us there and 17 us here, traced; storing the whole head in bin order, its
+// its entries start (18.6 us there and 20 here, traced; storing the whole head in bin order, its
 // 8-byte stores scattered over each slice's 16 KB, took 26 us here). One 64-bit LDS add per
 // entry counts it (the low 12 bits) and adds its weight (the upper 52) in fixed point: bin b's
 // weights, below 2^-k, k = floor(b * width), are scaled by 2^(40 + k), so 2,048 of them stay
